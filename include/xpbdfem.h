@@ -231,11 +231,14 @@ typedef struct xf_scene_opts {
                                    with their O (68 B a node), no body has volume passes or
                                    damping and the energy constrains tets (not in the last
                                    substep of a step call, which stores the velocities) */
-    uint32_t tet_lanes;         /* sweep-block launches: lanes per tet, 1 (0 = 1) or 4 (four lanes of a
-                                   quad share one tet, each owning one node: the per-node work is
-                                   split four ways, for launches whose phases are latency-bound; the
+    uint32_t tet_lanes;         /* sweep-block launches: lanes per tet, 1 or 4 (four lanes of a quad
+                                   share one tet, three holding its x, y and z components and one the
+                                   inverse masses, for launches whose phases are latency-bound; the
                                    simultaneous MixedSel / YeohSkinFast projection without damping,
-                                   else step calls fail with XF_E_UNSUPPORTED). Same results. */
+                                   else step calls fail with XF_E_UNSUPPORTED), or 0: 4, on 256-thread
+                                   workgroups whatever block_size is, where that projection runs, every
+                                   launch has at most one workgroup per compute unit and no phase more
+                                   than 64 tets; else 1. Same results. */
     uint32_t contract;          /* sweep-block launches: 1 runs kernels compiled with multiply-add
                                    contraction (fused multiply-adds in the element chain and the
                                    node phase: about a quarter fewer instructions per tet). Results
@@ -264,8 +267,9 @@ typedef struct xf_scene_info {
     uint32_t fused_finish;   /* 1: under the current settings, step calls in XF_LAUNCH_BLOCKS end
                                 their substeps inside the last block launch (see separate_finish;
                                 the energy is not checked here) */
-    uint32_t tet_lanes;      /* lanes per tet of sweep-block launches in use (xf_scene_opts.tet_lanes,
-                                or the autotuner's choice) */
+    uint32_t tet_lanes;      /* lanes per tet of sweep-block launches in use: xf_scene_opts.tet_lanes,
+                                the autotuner's choice or, where those leave it automatic, that of the
+                                last block launch run (1 before the first step) */
     uint32_t block_lds_limit; /* LDS bytes one sweep-block workgroup may use: the device's
                                  per-workgroup limit (160 KiB on gfx950); it caps a slot at
                                  block_lds_limit / 32 nodes and decides whether the node phase
@@ -275,8 +279,8 @@ typedef struct xf_scene_info {
     uint32_t block_node_stride; /* LDS bytes per slot node in the last block launch run: 48 where
                                    every block launch has at most two workgroups per compute unit,
                                    the projection is simultaneous MixedSel / YeohSkinFast without
-                                   damping, one lane per tet, and the nodes fit (fewer LDS bank
-                                   conflicts); else 32 (also before the first step) */
+                                   damping, no phase has more tets than a workgroup takes at once,
+                                   and the nodes fit (fewer LDS bank conflicts); else 32 (also before the first step) */
 } xf_scene_info;
 
 /* ------------------------------------------------------------ context */

@@ -1,0 +1,82 @@
+"""Sweep-block launches with the lanes per tet left to the library
+(xf_scene_opts.tet_lanes = 0): four lanes where every launch has at most one
+workgroup per compute unit and every phase fits 64 quads, else one. Bar:
+bit-exact with one lane per tet and with the oracle's serial sweep in the
+reported order, at the edges of the rule and of the block layout that goes
+with it."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+import workloads
+import xpbdfem as xf
+
+pytestmark = pytest.mark.gpu
+
+
+def run(ctx, wl, **opts):
+    sc = workloads.make_scene(ctx, wl, sweep_blocks=True, launch_mode=xf.LAUNCH_BLOCKS, **opts)
+    for _ in range(2):
+        sc.step(wl["substeps"], float(wl["dt"]))
+    x, v = sc.get_state(0)
+    order, info = sc.order(0)[0], sc.info()
+    sc.close()
+    return x, v, order, info
+
+
+# cells, block_lanes, settings, lanes per tet expected
+CASES = [
+    ((1, 1, 1), 0, {}, 4),                       # two launch colours, phases of one tet
+    ((3, 2, 5), 0, {}, 4),
+    ((12, 4, 4), 0, {}, 4),                      # one slot a launch, 60 tets a phase
+    ((12, 4, 4), 0, dict(energy=5), 1),          # no quad form of the energy
+    ((12, 4, 4), 0, dict(simultaneous=0), 1),
+    ((12, 4, 4), 0, dict(damping=0.01), 1),
+    ((40, 9, 11), 64, {}, 4),                    # ragged slots
+    (64, 256, {}, 4),                            # one phase of 64 separate tets: every quad busy
+    (65, 256, {}, 1),                            # one more than the quads
+]
+
+
+def mesh(cells):
+    if not isinstance(cells, int):
+        return xf.tet_block(*cells, (0.1, 0.1, 0.1), (0.0, -0.2, -0.2))
+    one, t4 = xf.tet_block(1, 1, 1, (0.1, 0.1, 0.1), (0.0, 0.0, 0.0))
+    p = one.reshape(-1, 3)[t4[:4]]
+    xyz = np.concatenate([p + np.float32([0.3 * j, 0.0, 0.0]) for j in range(cells)])
+    return xyz.astype(np.float32).ravel(), np.arange(4 * cells, dtype=np.uint32)
+
+
+@pytest.mark.parametrize("cells,lanes,settings,want", CASES)
+@pytest.mark.parametrize("energy", [4, 7])
+def test_automatic_lanes(ctx, cells, lanes, settings, want, energy):
+    wl = workloads.beam_neo_12x4x4(energy=energy)
+    xyz, tets = mesh(cells)
+    wl = dict(wl, xyz=xyz, tets=tets, pinned=(xyz[0::3] == 0.0).astype(np.uint8),
+              settings=dict(wl["settings"], **settings))
+    x, v, order, info = run(ctx, wl, block_lanes=lanes)
+    assert info["tet_lanes"] == want
+    ob = po.body_from_workload(wl, "ref64")
+    ob.substep(po.params_from_settings(wl["dt"], wl["settings"]), order, count=2 * wl["substeps"])
+    assert np.array_equal(x, ob.X) and np.array_equal(v, ob.V)
+
+
+def test_automatic_lanes_packed_layout(ctx):
+    """A beam whose runs of consecutive blocks would be more slots than
+    compute units: the blocks are laid out so that they are not, and the
+    reported order and the results are those of one lane per tet and of
+    per-colour launches over the same layout."""
+    wl = workloads.beam_yeoh(96, 24, 24)
+    wl = dict(wl, substeps=5)
+    a = run(ctx, wl)
+    b = run(ctx, wl, tet_lanes=1)
+    assert a[3]["tet_lanes"] == 4 and b[3]["tet_lanes"] == 1
+    assert a[3]["n_block_slots"] <= 4 * 256
+    assert np.array_equal(a[2], b[2])
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    sc = workloads.make_scene(ctx, wl, sweep_blocks=True)
+    for _ in range(2):
+        sc.step(wl["substeps"], float(wl["dt"]))
+    x, v = sc.get_state(0)
+    sc.close()
+    assert np.array_equal(x, a[0]) and np.array_equal(v, a[1])

@@ -770,6 +770,10 @@ struct NodeLds {
         p[0] = make_double2(v.x, v.y);
         p[1] = make_double2(v.z, v.w);
     }
+    // component c of node k (x, y, z, w)
+    __device__ __forceinline__ double* comp(uint32_t k, uint32_t c) const {
+        return reinterpret_cast<double*>(at(k)) + c;
+    }
     // position only (w, the inverse mass, is not changed by a projection)
     __device__ __forceinline__ void put_xyz(uint32_t k, double x, double y, double z) const {
         double2* p = at(k);
@@ -797,34 +801,46 @@ __device__ __forceinline__ void block_tet(const BlockTet& t, uint32_t i, NodeLds
     xs.put_xyz(id, x[3][0], x[3][1], x[3][2]);
 }
 
-// Value of v in lane L of this lane's quad (lanes 4k .. 4k + 3), by DPP
-// quad_perm broadcast.
+// v of another lane of this lane's quad (lanes 4k .. 4k + 3), by DPP
+// quad_perm: lane i reads lane Pi. Bounds control on with full masks lets the
+// compiler fold the move into the instruction that uses it.
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ float quad_perm(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), P0 | (P1 << 2) | (P2 << 4) | (P3 << 6), 0xF,
+                                                      0xF, true));
+}
 template <int L>
 __device__ __forceinline__ float quad_lane(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), L * 0x55, 0xF, 0xF, false));
+    return quad_perm<L, L, L, L>(v);
 }
 
-// One tet of a block phase on the four lanes of a quad: lane q owns node q.
-// SolveElementMixed with the simultaneous solve (MixedSel / YeohSkinFast;
-// E = 0 picks per body), damping off, in exactly the operations and order of
-// solve_tet: the per-tet scalars (I1, F, adjugate, J, the Cramer solve) are
-// computed by all four lanes alike, each node's gradients, its terms of the
-// sums of the 2x2 system and its position update by its own lane; the root
-// node's gradient -(g0 + g1 + g2) and the sums over nodes are assembled in
-// node order from the other lanes by DPP. Results equal block_tet bit for
-// bit.
-template <int E, bool AUX>
-__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<32> xs,
+// One tet of a block phase on the four lanes of a quad, split by component:
+// lanes 0, 1, 2 hold x, y, z of every vector of the tet (positions,
+// gradients, rows of F), lane 3 the four inverse masses, which are the fourth
+// component of the node records. SolveElementMixed with the simultaneous
+// solve (MixedSel / YeohSkinFast; E = 0 picks per body), damping off, in
+// exactly the operations and order of solve_tet:
+//  - P, the gradients, F, the updates: each lane its own component;
+//  - column a of the adjugate is the cross product of rows a + 1 and a + 2 of
+//    F, which the lane reads from its neighbours (cofactors that solve_tet
+//    negates come out as the reversed difference, the same value);
+//  - a dot product is each lane's product, then (x + y) + z by DPP, valid in
+//    lanes 0 and 1 (x + y and y + x round alike);
+//  - the 2x2 system: lane 0 holds the I1 row, lane 1 the volume row, so one
+//    reciprocal serves both and the Cramer solve is one expression.
+// Results equal block_tet's bit for bit. The chain is about half as long as
+// one lane's (293 against 560 VALU instructions for YeohSkinFast), which
+// counts where a phase has fewer waves than the chip has SIMDs.
+template <int E, bool AUX, uint32_t NS>
+__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<NS> xs,
                                                const XfBodyParams* __restrict__ bodies, float comp1_u, float a_u,
                                                float dt) {
     static_assert(E == 0 || E == 4 || E == 7, "quad lanes take MixedSel / YeohSkinFast");
-    const uint32_t ia = t.loc.x & 0xFFFFu, ib = t.loc.x >> 16, ic = t.loc.y & 0xFFFFu, id = t.loc.y >> 16;
-    const double4 na = xs.get(ia), nb = xs.get(ib), nc = xs.get(ic), nd = xs.get(id);
-    const double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
-    const bool q0 = q == 0u, q1 = q == 1u, q2 = q == 2u, q3 = q == 3u;
-    const uint32_t own = q0 ? ia : (q1 ? ib : (q2 ? ic : id));
-    const double4 xo = q0 ? na : (q1 ? nb : (q2 ? nc : nd));
-    const float w = (float)xo.w;
+    double* const n0 = xs.comp(t.loc.x & 0xFFFFu, q);
+    double* const n1 = xs.comp(t.loc.x >> 16, q);
+    double* const n2 = xs.comp(t.loc.y & 0xFFFFu, q);
+    double* const n3 = xs.comp(t.loc.y >> 16, q);
+    const double x[4] = {*n0, *n1, *n2, *n3};
 
     float comp1 = comp1_u, a = a_u;
     uint32_t body = 0;
@@ -841,111 +857,98 @@ __device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, No
     const float QR[3] = {t.q3.x, t.q3.y, t.q3.z};
     const float comp0 = t.q3.w;
 
-    float P[3][3];
-    gather_p(x, P);
-
-    // Prefactored I1 (neo_prefactored): the energy on every lane, the
-    // gradient of node q on lane q, g[i] = (2 QQ_i) P_i + QR_a P_a + QR_b P_b
-    // in the pair order (0,1), (0,2), (1,2).
-    float u = 0.0f;
+    float P[3], w[4];
 #pragma unroll
-    for (int i = 0; i < 3; i++) u = u + QQ[i] * dot3(P[i], P[i]);
+    for (int i = 0; i < 3; i++) P[i] = (float)(x[i] - x[3]);
+#pragma unroll
+    for (int n = 0; n < 4; n++) w[n] = quad_lane<3>((float)x[n]);
+    // a . b in lanes 0 and 1
+    auto dot = [](float a, float b) {
+        const float m = a * b;
+        return (m + quad_perm<1, 0, 2, 3>(m)) + quad_lane<2>(m);
+    };
+
+    // prefactored I1 (neo_prefactored)
+    float u = 0.0f, g0[4], g1[4];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        u = u + QQ[i] * dot(P[i], P[i]);
+        g0[i] = (2.0f * QQ[i]) * P[i];
+    }
     {
         int k = 0;
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = i + 1; j < 3; j++) {
-                u = u + QR[k] * dot3(P[i], P[j]);
+                u = u + QR[k] * dot(P[i], P[j]);
+                g0[i] = g0[i] + QR[k] * P[j];
+                g0[j] = g0[j] + QR[k] * P[i];
                 ++k;
             }
     }
-    const float cq = 2.0f * (q0 ? QQ[0] : (q1 ? QQ[1] : QQ[2]));
-    const float qa = q2 ? QR[1] : QR[0];
-    const float qb = q0 ? QR[1] : QR[2];
-    float g0[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const float pn = q0 ? P[0][r] : (q1 ? P[1][r] : P[2][r]);
-        const float pa = q0 ? P[1][r] : P[0][r];
-        const float pb = q2 ? P[1][r] : P[2][r];
-        float g = cq * pn;
-        g = g + qa * pa;
-        g = g + qb * pb;
-        g0[r] = g;
-    }
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const float root = ((0.0f - quad_lane<0>(g0[r])) - quad_lane<1>(g0[r])) - quad_lane<2>(g0[r]);
-        g0[r] = q3 ? root : g0[r];
-    }
+    g0[3] = ((0.0f - g0[0]) - g0[1]) - g0[2];
     float U0 = u;
     if (yf) {
         const float IM = U0 - 3.0f;
         U0 = fmaxf(0.0001f, C[0] * IM + C[1] * IM * IM + C[2] * IM * IM * IM);
-        const float gScale = C[0] + 2.0f * C[1] * IM + 3.0f * C[2] * IM * IM;
+        const float gScale = quad_lane<0>(C[0] + 2.0f * C[1] * IM + 3.0f * C[2] * IM * IM);
 #pragma unroll
-        for (int r = 0; r < 3; r++) g0[r] = g0[r] * gScale;
+        for (int n = 0; n < 4; n++) g0[n] = g0[n] * gScale;
     }
 
-    // (J - a)^2 volume term (volume_term): F, adjugate and J on every lane,
-    // node q's row of G Qi^T on lane q.
-    float F[3][3], adj[3][3], GJ[3][3];
-    defgrad(Qi, P, F);
-    const float J = adjdet(F, adj);
-    const float U1 = 0.0f + 1.0f * ((J - a) * (J - a));
+    // (J - a)^2 volume term (volume_term)
+    float F[3], A[3], B[3], adj[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) F[r] = Qi[0][r] * P[0] + Qi[1][r] * P[1] + Qi[2][r] * P[2];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        A[r] = quad_perm<1, 2, 0, 3>(F[r]);
+        B[r] = quad_perm<2, 0, 1, 3>(F[r]);
+    }
+    adj[0] = A[1] * B[2] - A[2] * B[1];
+    adj[1] = A[2] * B[0] - A[0] * B[2];
+    adj[2] = A[0] * B[1] - A[1] * B[0];
+    const float J = quad_lane<0>(F[0] * adj[0] + F[1] * adj[1] + F[2] * adj[2]);
+    const float U1 = (J - a) * (J - a);
     const float sJ = 2.0f * (J - a);
 #pragma unroll
-    for (int c = 0; c < 3; c++)
+    for (int c = 0; c < 3; c++) adj[c] = adj[c] * sJ;
 #pragma unroll
-        for (int r = 0; r < 3; r++) GJ[c][r] = adj[c][r] * sJ;
-    float Qn[3];
-#pragma unroll
-    for (int c = 0; c < 3; c++) Qn[c] = q0 ? Qi[0][c] : (q1 ? Qi[1][c] : Qi[2][c]);
-    float g1[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++) g1[r] = 0.0f + (GJ[0][r] * Qn[0] + GJ[1][r] * Qn[1] + GJ[2][r] * Qn[2]);
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const float root = ((0.0f - quad_lane<0>(g1[r])) - quad_lane<1>(g1[r])) - quad_lane<2>(g1[r]);
-        g1[r] = q3 ? root : g1[r];
-    }
+    for (int j = 0; j < 3; j++) g1[j] = 0.0f + (adj[0] * Qi[j][0] + adj[1] * Qi[j][1] + adj[2] * Qi[j][2]);
+    g1[3] = ((0.0f - g1[0]) - g1[1]) - g1[2];
 
-    // EnergyXpbdConstrainSimultaneous<2>, Cramer branch (constrain2): the
-    // node sums in node order, then the solve on every lane.
-    const float alpha0 = comp0 / (dt * dt);
-    const float alpha1 = comp1 / (dt * dt);
-    const float t00 = w * dot3(g0, g0), t10 = w * dot3(g1, g0), t11 = w * dot3(g1, g1);
+    // EnergyXpbdConstrainSimultaneous<2>, Cramer branch (constrain2)
     float A0 = 1.0e-22f, A1 = 1.0e-22f, A2 = 1.0e-22f;
-    A0 = A0 + quad_lane<0>(t00);
-    A0 = A0 + quad_lane<1>(t00);
-    A0 = A0 + quad_lane<2>(t00);
-    A0 = A0 + quad_lane<3>(t00);
-    A0 = A0 + 2.0f * U0 * alpha0;
-    const float b0 = -2.0f * U0;
-    A1 = A1 + quad_lane<0>(t10);
-    A1 = A1 + quad_lane<1>(t10);
-    A1 = A1 + quad_lane<2>(t10);
-    A1 = A1 + quad_lane<3>(t10);
-    A2 = A2 + quad_lane<0>(t11);
-    A2 = A2 + quad_lane<1>(t11);
-    A2 = A2 + quad_lane<2>(t11);
-    A2 = A2 + quad_lane<3>(t11);
-    A2 = A2 + 2.0f * U1 * alpha1;
-    const float b1 = -2.0f * U1;
-    const float invA00 = 1.0f / A0;
-    const float invA11 = 1.0f / A2;
-    const float invDet = 1.0f / fmaxf(0.00000001f, 1.0f - (A1 * invA00) * (A1 * invA11));
-    const float l0 = invDet * ((b0 * invA00) - (A1 * invA00) * (b1 * invA11));
-    const float l1 = invDet * ((b1 * invA11) - (b0 * invA00) * (A1 * invA11));
-    double xn[3] = {xo.x, xo.y, xo.z};
 #pragma unroll
-    for (int r = 0; r < 3; r++) {
-        float acc = 0.0f + l0 * g0[r];
-        acc = acc + l1 * g1[r];
-        xn[r] = xn[r] + (double)(w * acc);
+    for (int n = 0; n < 4; n++) {
+        A0 = A0 + w[n] * dot(g0[n], g0[n]);
+        A1 = A1 + w[n] * dot(g1[n], g0[n]);
+        A2 = A2 + w[n] * dot(g1[n], g1[n]);
     }
-    xs.put_xyz(own, xn[0], xn[1], xn[2]);
+    const bool row1 = (q & 1u) != 0u;
+    const float U = row1 ? U1 : U0;
+    const float alpha = row1 ? comp1 / (dt * dt) : comp0 / (dt * dt);
+    const float Ad = (row1 ? A2 : A0) + 2.0f * U * alpha;
+    const float invA = 1.0f / Ad;
+    const float be = (-2.0f * U) * invA;  // b0 invA00 | b1 invA11
+    const float pq = A1 * invA;           // A1 invA00 | A1 invA11
+    const float invDet = 1.0f / fmaxf(0.00000001f, 1.0f - pq * quad_perm<1, 0, 2, 3>(pq));
+    const float l = invDet * (be - pq * quad_perm<1, 0, 2, 3>(be));
+    const float l0 = quad_lane<0>(l), l1 = quad_lane<1>(l);
+    double xn[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+        float acc = 0.0f + l0 * g0[n];
+        acc = acc + l1 * g1[n];
+        xn[n] = x[n] + (double)(w[n] * acc);
+    }
+    if (q != 3u) {
+        *n0 = xn[0];
+        *n1 = xn[1];
+        *n2 = xn[2];
+        *n3 = xn[3];
+    }
 }
 
 // A slot's nodes into LDS (stage_nodes) and back (write_nodes), kStage list
@@ -1003,6 +1006,10 @@ __device__ __forceinline__ void write_nodes(uint32_t tid, uint32_t bs, uint32_t 
 // those nodes, and O is not read by the projection (FIN excludes DAMP).
 // tend: the clock, read for the end time of the substep (advanced by an
 // earlier launch). fsingle: the scene has one body.
+// PF: register sets of element data, loaded PF - 1 phases ahead. One lane per
+// tet: 2 (a phase lasts 1.2 us, longer than a load, and the chain needs the
+// registers). Quads: 3 (a phase lasts 0.7 us, less than a load from beyond L2:
+// 1.43 against 1.44 ms per frame of the 96x24x24 beam with 2, 1.49 with 4).
 template <int E, bool SIM, bool AUX, bool DAMP, bool OVER, bool FIN, bool QUAD = false, uint32_t NS = 32>
 __global__ __launch_bounds__(256) void xf_project_blocks(
     uint32_t nph, uint32_t nmax, uint32_t ntet, const uint32_t* __restrict__ rec, const uint32_t* __restrict__ bnode,
@@ -1014,7 +1021,6 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
     static_assert(!(FIN && (DAMP || E == 30)), "the fused node phase needs a projection that leaves O unread");
     static_assert(!QUAD || (SIM && !DAMP && (E == 0 || E == 4 || E == 7)),
                   "quad lanes take the simultaneous MixedSel / YeohSkinFast projection without damping");
-    static_assert(NS == 32u || !QUAD, "quad lanes take 32-byte nodes");
     if (clock != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
         clock[0] = clock[0] + dt;
         uint32_t* tick = reinterpret_cast<uint32_t*>(clock) + 1;
@@ -1032,14 +1038,15 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
     const uint32_t ftot = FIN ? nmax + fmax : 0u;
     double4* os = FIN ? reinterpret_cast<double4*>(xs.base + (NS / 16u) * ftot) : nullptr;
     uint32_t* fs = FIN ? reinterpret_cast<uint32_t*>(os + ftot) : nullptr;
-    // QUAD: four lanes per tet (lane tid & 3 owns node tid & 3), bs / 4 tets
+    // QUAD: four lanes per tet (block_tet_quad), bs / 4 tets
     // at a time; else one lane per tet
     const uint32_t lt = QUAD ? tid >> 2 : tid, per = QUAD ? bs >> 2 : bs;
+    constexpr uint32_t PF = QUAD ? 3 : 2;
     auto load = [&](uint32_t j) {
         return load_block_tet<AUX>(min(r[2 * j] + lt, last), tloc, tg0, tg1, tg2, tg3, taux);
     };
     auto solve = [&](const BlockTet& t, uint32_t i) {
-        if constexpr (QUAD) block_tet_quad<E, AUX>(t, tid & 3u, xs, bodies, comp1_u, a_u, dt);
+        if constexpr (QUAD) block_tet_quad<E, AUX, NS>(t, tid & 3u, xs, bodies, comp1_u, a_u, dt);
         else block_tet<E, SIM, AUX, DAMP, NS>(t, i, xs, tidx, O, bodies, comp1_u, a_u, dt);
     };
     // each lane's first tet of the phase is t; with OVER, lanes go on to the
@@ -1052,7 +1059,8 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
                 solve(load_block_tet<AUX>(b + k, tloc, tg0, tg1, tg2, tg3, taux), b + k);
         __syncthreads();
     };
-    BlockTet ta = load(0), tb;
+    BlockTet t[PF];
+    t[0] = load(0);
     if constexpr (FIN) {
         // nodes, their O and their ids staged for the end of the substep
         const uint32_t* fl = fextra + (size_t)blockIdx.x * ftot;
@@ -1068,13 +1076,16 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
         stage_nodes(tid, bs, nmax, bn, X, xs);
     }
     __syncthreads();
-    // phases in pairs, element data of the next phase loaded before solving
-    // the current one (ta: even phases, tb: odd phases)
-    for (uint32_t j = 0; j < nph; j += 2) {
-        tb = load(min(j + 1u, jl));
-        phase(j, ta);
-        ta = load(min(j + 2u, jl));
-        if (j + 1u < nph) phase(j + 1u, tb);
+    // element data of phase j + PF - 1 loaded before solving phase j (set
+    // j mod PF), so that the wait before a phase covers only that phase's loads
+#pragma unroll
+    for (uint32_t k = 1; k + 1 < PF; k++) t[k] = load(min(k, jl));
+    for (uint32_t j = 0; j < nph; j += PF) {
+#pragma unroll
+        for (uint32_t k = 0; k < PF; k++) {
+            t[(k + PF - 1) % PF] = load(min(j + k + PF - 1, jl));
+            if (k == 0 || j + k < nph) phase(j + k, t[k]);
+        }
     }
     if constexpr (FIN) {
         // (single-body scenes read the body's parameters once)
@@ -1617,17 +1628,21 @@ XfBlocksFn pick_blocks_ad(bool aux, bool damp, bool fin) {
     return damp ? xf_project_blocks<E, SIM, false, true, OVER, false> : xf_project_blocks<E, SIM, false, false, OVER, false>;
 }
 // 48-byte nodes: the simultaneous MixedSel / YeohSkinFast projection without
-// damping, one lane per tet, no phase beyond the workgroup's lanes; else
-// nullptr (the launch keeps 32-byte nodes)
+// damping, no phase beyond the workgroup's lanes; else nullptr (the launch
+// keeps 32-byte nodes)
+template <int E, bool QUAD>
+XfBlocksFn pick_blocks_wide_aux(bool aux, bool fin) {
+    if (fin)
+        return aux ? xf_project_blocks<E, true, true, false, false, true, QUAD, 48>
+                   : xf_project_blocks<E, true, false, false, false, true, QUAD, 48>;
+    return aux ? xf_project_blocks<E, true, true, false, false, false, QUAD, 48>
+               : xf_project_blocks<E, true, false, false, false, false, QUAD, 48>;
+}
 template <int E>
 XfBlocksFn pick_blocks_wide(bool sim, bool aux, bool damp, bool over, bool fin, bool quad) {
     if constexpr (E == 0 || E == 4 || E == 7) {
-        if (!sim || damp || over || quad) return nullptr;
-        if (fin)
-            return aux ? xf_project_blocks<E, true, true, false, false, true, false, 48>
-                       : xf_project_blocks<E, true, false, false, false, true, false, 48>;
-        return aux ? xf_project_blocks<E, true, true, false, false, false, false, 48>
-                   : xf_project_blocks<E, true, false, false, false, false, false, 48>;
+        if (!sim || damp || over) return nullptr;
+        return quad ? pick_blocks_wide_aux<E, true>(aux, fin) : pick_blocks_wide_aux<E, false>(aux, fin);
     }
     return nullptr;
 }

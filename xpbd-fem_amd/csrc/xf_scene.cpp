@@ -334,6 +334,10 @@ struct xf_scene {
     // what limits them; blk_nstride: the bytes per node of the last launch
     bool blk_wide = false;
     uint32_t blk_nstride = 32;
+    uint32_t blk_tet_lanes = 1;  // lanes per tet of the last block launch
+    // layout index of every block inside its launch colour, per body: the
+    // order of the blocks' tets in each colour and of the slots (LayoutBlocks)
+    std::vector<std::vector<uint32_t>> blk_lay;
     uint32_t* blk_fin = nullptr;
     uint2* tloc = nullptr;
     uint32_t* tout = nullptr;  // per schedule position: the tet's slot in body-concatenated, body-local order
@@ -699,6 +703,22 @@ int HeldNodes(xf_scene* s, float dt) {
     return XF_OK;
 }
 
+// Lanes per tet of the sweep-block launches: opts.tet_lanes, or where that is
+// 0 (automatic) four when every launch has at most one workgroup per compute
+// unit and every phase fits the 64 quads of a 256-thread workgroup. A launch
+// is then bound by the chain of one tet, which a quad halves (launches of the
+// 96x24x24 beam: 8.5 us with quads, 11.8 us without); with a second workgroup
+// on a compute unit, two waves share each SIMD and the quads' larger total of
+// instructions takes back what the shorter chain gave (11.5 us at 264
+// workgroups on 256 compute units).
+uint32_t TetLanes(const xf_scene* s, int energy, bool sim) {
+    if (s->opts.tet_lanes) return s->opts.tet_lanes;
+    if (!(energy == 0 || energy == 4 || energy == 7) || !sim || s->dproj || s->blk_pmax > 64) return 1;
+    for (const xf_scene::BlockLaunch& L : s->blk)
+        if (L.nslot > (uint32_t)s->n_cu) return 1;
+    return 4;
+}
+
 int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, LaunchTimer* timer) {
     xf_ctx* ctx = s->ctx;
     hipStream_t st = ctx->stream;
@@ -809,6 +829,10 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     int rc = node(0, false);
     if (rc) return rc;
     const bool blocks = s->opts.launch_mode == XF_LAUNCH_BLOCKS;
+    const bool quad = blocks && TetLanes(s, energy, sim) == 4;
+    // automatic quads: 64 tets a phase on 256 threads (block_size is the workgroup of one-lane launches)
+    const uint32_t blk_threads = quad && s->opts.tet_lanes == 0 ? 256u : block;
+    s->blk_tet_lanes = quad ? 4u : 1u;
     // the node phase rides on the substep's last block launch when nothing
     // runs between the sweep and the velocity update (no volume passes), the
     // velocities need not be stored (no damping passes, not the call's last
@@ -830,11 +854,11 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
                 XF_HIP(ctx, hipEventRecord(e0, st));
             }
             auto launch = s->opts.contract ? xf_launch_blocks_contract : xf_launch_blocks;
-            XF_HIP(ctx, launch(st, energy, sim, s->aux, s->dproj, block, L.nslot, L.nph, s->blk_nmax, s->T,
+            XF_HIP(ctx, launch(st, energy, sim, s->aux, s->dproj, blk_threads, L.nslot, L.nph, s->blk_nmax, s->T,
                                s->blk_pmax, s->blk_rec + L.rec_off, s->blk_node + L.node_off, s->tloc, s->tidx,
                                s->tg[0], s->tg[1], s->tg[2], s->tg[3], s->taux, s->X, s->O, s->bp, s->comp1_u,
                                s->a_u, dt, first ? s->clock : nullptr, fin && q == s->blk_last, s->blk_fin,
-                               s->blk_fmax, s->clock, s->bodies.size() == 1, s->opts.tet_lanes == 4,
+                               s->blk_fmax, s->clock, s->bodies.size() == 1, quad,
                                s->lds_limit, s->blk_wide, &s->blk_nstride));
             first = false;
             if (timer) {
@@ -946,8 +970,119 @@ struct BlockTables {
     std::vector<uint32_t> rec, node, fin;
 };
 
+// A workgroup of the quad launches sweeps at most this many tets a phase.
+constexpr uint32_t kQuadTets = 64;
+
+// Layout order of the blocks of every launch colour (blk_lay): body, then
+// block number, or, where slots of kQuadTets tets merged from consecutive
+// blocks would be more than the compute units although the tets would fill
+// no more than all of them, an order in which they are not. Then blocks go,
+// in that order, into the fullest of a few open bins that still holds them
+// (a bin: at most kQuadTets tets in each phase, its nodes within LDS), and the
+// layout is the bins one after another; the few open bins keep a slot's
+// blocks near each other. On the 96x24x24 beam (blocks of 1 to 24 tets a
+// phase) 264 slots a launch become 226 on 256 compute units; the eight
+// compute units that swept two slots took 11 us where the others took 8.
+// Blocks of one launch colour share no node, so their order in memory does
+// not enter the results; the reported sweep order stays body, block, visit.
+void LayoutBlocks(xf_scene* s) {
+    const uint32_t slot_nodes = (uint32_t)std::min<size_t>(s->lds_limit / 32, 65535);
+    s->blk_lay.assign(s->bodies.size(), std::vector<uint32_t>());
+    struct Block {
+        uint32_t body, k, nodes;
+    };
+    std::vector<Block> blocks[4];
+    for (size_t bi = 0; bi < s->bodies.size(); bi++) {
+        const xf::SweepBlocks& sb = s->sweep[bi];
+        s->blk_lay[bi].resize(sb.n_blocks);
+        for (uint32_t k = 0; k < sb.n_blocks; k++) {
+            s->blk_lay[bi][k] = (uint32_t)blocks[sb.launch[k]].size();
+            blocks[sb.launch[k]].push_back({(uint32_t)bi, k, 0});
+        }
+    }
+    // tets per phase of each block, row-major by layout index
+    std::vector<uint32_t> count[4];
+    for (int q = 0; q < 4; q++) count[q].assign(blocks[q].size() * (size_t)s->blk[q].nph, 0);
+    for (size_t bi = 0; bi < s->bodies.size(); bi++) {
+        const xf::SweepBlocks& sb = s->sweep[bi];
+        for (uint32_t t = 0; t < s->bodies[bi].t; t++) {
+            const uint32_t k = sb.block[t], q = sb.launch[k];
+            count[q][s->blk_lay[bi][k] * (size_t)s->blk[q].nph + sb.phase[t]]++;
+        }
+    }
+    for (int q = 0; q < 4; q++) {
+        const uint32_t nph = s->blk[q].nph;
+        const size_t nb = blocks[q].size();
+        if (nb <= (size_t)s->n_cu) continue;
+        // slots of consecutive blocks, and the least number of slots any order can reach
+        std::vector<uint64_t> total(nph, 0);
+        std::vector<uint32_t> fill(nph, 0);
+        size_t runs = 1;
+        bool small = true;
+        for (size_t m = 0; m < nb; m++) {
+            const uint32_t* c = &count[q][m * nph];
+            bool fits = true;
+            for (uint32_t j = 0; j < nph; j++) {
+                total[j] += c[j];
+                small = small && c[j] <= kQuadTets;
+                fits = fits && fill[j] + c[j] <= kQuadTets;
+            }
+            if (!fits) {
+                runs++;
+                std::fill(fill.begin(), fill.end(), 0u);
+            }
+            for (uint32_t j = 0; j < nph; j++) fill[j] += c[j];
+        }
+        const uint64_t most = *std::max_element(total.begin(), total.end());
+        if (!small || runs <= (size_t)s->n_cu || most > (uint64_t)kQuadTets * (uint64_t)s->n_cu) continue;
+        // nodes per block: four per tet is enough of a bound here
+        for (size_t m = 0; m < nb; m++)
+            for (uint32_t j = 0; j < nph; j++) blocks[q][m].nodes += 4 * count[q][m * nph + j];
+        struct Bin {
+            std::vector<uint32_t> fill, members;
+            uint32_t nodes = 0, level = 0;
+        };
+        constexpr size_t kOpen = 16;
+        std::vector<Bin> bins;
+        std::vector<size_t> open;
+        for (size_t m = 0; m < nb; m++) {
+            const uint32_t* c = &count[q][m * nph];
+            size_t best = open.size();
+            for (size_t o = 0; o < open.size(); o++) {
+                const Bin& b = bins[open[o]];
+                bool fits = b.nodes + blocks[q][m].nodes <= slot_nodes;
+                for (uint32_t j = 0; j < nph && fits; j++) fits = b.fill[j] + c[j] <= kQuadTets;
+                if (fits && (best == open.size() || b.level > bins[open[best]].level)) best = o;
+            }
+            if (best == open.size()) {
+                if (open.size() == kOpen) {  // close the fullest
+                    size_t full = 0;
+                    for (size_t o = 1; o < open.size(); o++)
+                        if (bins[open[o]].level > bins[open[full]].level) full = o;
+                    open.erase(open.begin() + full);
+                }
+                best = open.size();
+                open.push_back(bins.size());
+                bins.emplace_back();
+                bins.back().fill.assign(nph, 0);
+            }
+            Bin& b = bins[open[best]];
+            for (uint32_t j = 0; j < nph; j++) {
+                b.fill[j] += c[j];
+                b.level = std::max(b.level, b.fill[j]);
+            }
+            b.nodes += blocks[q][m].nodes;
+            b.members.push_back((uint32_t)m);
+        }
+        if (bins.size() > (size_t)s->n_cu) continue;
+        uint32_t next = 0;
+        for (const Bin& b : bins)
+            for (uint32_t m : b.members) s->blk_lay[blocks[q][m].body][blocks[q][m].k] = next++;
+    }
+}
+
 // Sweep-block tables for the slot cap lanes_opt (0: automatic). Blocks of
-// launch colour q in layout order (body, then block number: the order of
+// launch colour q in layout order (LayoutBlocks: the order of
 // their tets inside each colour q, j) are merged, consecutive ones, into
 // workgroup slots while every phase of the slot holds at most lanes_opt
 // tets and its nodes fit LDS; a slot's
@@ -961,12 +1096,9 @@ int PackBlocks(xf_scene* s, uint32_t lanes_opt, BlockTables* bt) {
     // a slot's nodes (32 B each in LDS) within the device's per-workgroup LDS
     const uint32_t kSlotNodes = (uint32_t)std::min<size_t>(s->lds_limit / 32, 65535);
     uint32_t nblk[4] = {0, 0, 0, 0};
-    std::vector<std::vector<uint32_t>> lay(s->bodies.size());
-    for (size_t bi = 0; bi < s->bodies.size(); bi++) {
-        const xf::SweepBlocks& sb = s->sweep[bi];
-        lay[bi].resize(sb.n_blocks);
-        for (uint32_t k = 0; k < sb.n_blocks; k++) lay[bi][k] = nblk[sb.launch[k]]++;
-    }
+    const std::vector<std::vector<uint32_t>>& lay = s->blk_lay;
+    for (const xf::SweepBlocks& sb : s->sweep)
+        for (uint32_t k = 0; k < sb.n_blocks; k++) nblk[sb.launch[k]]++;
     s->n_blocks = nblk[0] + nblk[1] + nblk[2] + nblk[3];
     // per block: sorted node list; per schedule position: the block's layout index
     std::vector<std::vector<uint32_t>> bnodes[4];
@@ -1029,8 +1161,7 @@ int PackBlocks(xf_scene* s, uint32_t lanes_opt, BlockTables* bt) {
             gfirst[q].push_back(nblk[q]);
         }
     };
-    int n_cu = 256;
-    XF_HIP(ctx, hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    const int n_cu = s->n_cu;
     uint32_t lanes_cap = lanes_opt;
     if (lanes_cap == 0) {
         // the largest cap that leaves >= 4 slots per compute unit in every launch colour
@@ -1105,8 +1236,7 @@ int PackBlocks(xf_scene* s, uint32_t lanes_opt, BlockTables* bt) {
     s->blk_fmax = 0;
     bt->fin.clear();
     std::vector<uint32_t> extra;
-    int cus = 256;
-    XF_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    const int cus = s->n_cu;
     // fused only where the last launch is latency-bound (at most two
     // workgroups per compute unit): with more, the longer write-back and
     // the LDS of O cost more than the node launch they save
@@ -1402,8 +1532,8 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
         return Fail(ctx, XF_E_INVALID, "ring_lanes must be 0, 16 or 32");
     if (s->opts.sweep_blocks > 1) return Fail(ctx, XF_E_INVALID, "sweep_blocks must be 0 or 1");
     if (s->opts.separate_finish > 1) return Fail(ctx, XF_E_INVALID, "separate_finish must be 0 or 1");
-    if (s->opts.tet_lanes == 0) s->opts.tet_lanes = 1;
-    if (s->opts.tet_lanes != 1 && s->opts.tet_lanes != 4) return Fail(ctx, XF_E_INVALID, "tet_lanes must be 0, 1 or 4");
+    if (s->opts.tet_lanes != 0 && s->opts.tet_lanes != 1 && s->opts.tet_lanes != 4)
+        return Fail(ctx, XF_E_INVALID, "tet_lanes must be 0, 1 or 4");
     if (s->opts.block_lanes > 256) return Fail(ctx, XF_E_INVALID, "block_lanes must be at most 256");
     if (s->opts.contract > 1) return Fail(ctx, XF_E_INVALID, "contract must be 0 or 1");
     if (s->opts.sweep_blocks && s->opts.xcd_slabs)
@@ -1415,6 +1545,12 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
             if (!b.user_colour.empty())
                 return Fail(ctx, XF_E_INVALID, "sweep_blocks colours the tets itself; a body has tet_colour");
     XF_HIP(ctx, hipSetDevice(ctx->device));
+    XF_HIP(ctx, hipDeviceGetAttribute(&s->n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    {
+        int lds = 65536;
+        XF_HIP(ctx, hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
+        s->lds_limit = (size_t)lds;
+    }
 
     // Sweep blocks: colour (q, j) = phase j of the blocks of launch colour q,
     // numbered over the launch colours that hold blocks.
@@ -1506,36 +1642,59 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
     s->h_tg3.assign(s->T, make_float4(0, 0, 0, 0));
     s->h_taux.assign(s->T, make_float4(0, 0, 0, 0));
     std::vector<float2> h_tdmp(s->T);
-    std::vector<uint32_t> cursor(s->bodies.size(), 0);
     uint32_t pos = 0;
-    for (uint32_t c = 0; c < s->ncol; c++) {
-        s->colour_begin[c] = pos;
-        for (size_t bi = 0; bi < s->bodies.size(); bi++) {
-            Body& b = s->bodies[bi];
-            if (b.sched_pos.empty()) b.sched_pos.assign(b.t, 0);
-            uint32_t& k = cursor[bi];
-            while (k < b.t && b.colour[b.order[k]] == c) {
-                uint32_t t = b.order[k++];
-                const uint32_t* is = &b.tets[4 * (size_t)t];
-                const float* q = &b.ec.qi[9 * (size_t)t];
-                const float* qq = &b.ec.qq[3 * (size_t)t];
-                const float* qr = &b.ec.qr[3 * (size_t)t];
-                h_tidx[pos] = make_uint4(b.node_base + is[0], b.node_base + is[1], b.node_base + is[2],
-                                         b.node_base + is[3]);
-                h_tg0[pos] = make_float4(q[0], q[1], q[2], q[3]);
-                h_tg1[pos] = make_float4(q[4], q[5], q[6], q[7]);
-                h_tg2[pos] = make_float4(q[8], qq[0], qq[1], qq[2]);
-                s->h_tg3[pos] = make_float4(qr[0], qr[1], qr[2], 0.0f);
-                uint32_t bid = (uint32_t)bi;
-                float bidf;
-                memcpy(&bidf, &bid, 4);
-                s->h_taux[pos] = make_float4(0.0f, 1.0f, bidf, 0.0f);
-                uint32_t local = k - 1;  // position in the body's sweep order
-                float localf;
-                memcpy(&localf, &local, 4);
-                h_tdmp[pos] = make_float2(b.ec.area[t], localf);
-                b.sched_pos[t] = pos;
-                ++pos;
+    // the k-th tet of body bi's sweep order at the next schedule position
+    auto emit = [&](uint32_t bi, uint32_t k) {
+        Body& b = s->bodies[bi];
+        const uint32_t t = b.order[k];
+        const uint32_t* is = &b.tets[4 * (size_t)t];
+        const float* q = &b.ec.qi[9 * (size_t)t];
+        const float* qq = &b.ec.qq[3 * (size_t)t];
+        const float* qr = &b.ec.qr[3 * (size_t)t];
+        h_tidx[pos] = make_uint4(b.node_base + is[0], b.node_base + is[1], b.node_base + is[2], b.node_base + is[3]);
+        h_tg0[pos] = make_float4(q[0], q[1], q[2], q[3]);
+        h_tg1[pos] = make_float4(q[4], q[5], q[6], q[7]);
+        h_tg2[pos] = make_float4(q[8], qq[0], qq[1], qq[2]);
+        s->h_tg3[pos] = make_float4(qr[0], qr[1], qr[2], 0.0f);
+        float bidf;
+        memcpy(&bidf, &bi, 4);
+        s->h_taux[pos] = make_float4(0.0f, 1.0f, bidf, 0.0f);
+        float localf;
+        memcpy(&localf, &k, 4);  // position in the body's sweep order
+        h_tdmp[pos] = make_float2(b.ec.area[t], localf);
+        b.sched_pos[t] = pos;
+        ++pos;
+    };
+    for (Body& b : s->bodies) b.sched_pos.assign(b.t, 0);
+    if (s->opts.sweep_blocks) {
+        // each colour: its blocks in layout order, a block's tets in the body's sweep order
+        LayoutBlocks(s);
+        struct Run {
+            uint32_t lay, body, first, count;
+        };
+        std::vector<std::vector<Run>> runs(s->ncol);
+        for (uint32_t bi = 0; bi < (uint32_t)s->bodies.size(); bi++) {
+            const Body& b = s->bodies[bi];
+            for (uint32_t k = 0; k < b.t;) {
+                const uint32_t t = b.order[k], blk = sweep[bi].block[t], first = k;
+                while (k < b.t && b.colour[b.order[k]] == b.colour[t] && sweep[bi].block[b.order[k]] == blk) k++;
+                runs[b.colour[t]].push_back({s->blk_lay[bi][blk], bi, first, k - first});
+            }
+        }
+        for (uint32_t c = 0; c < s->ncol; c++) {
+            s->colour_begin[c] = pos;
+            std::sort(runs[c].begin(), runs[c].end(), [](const Run& a, const Run& b) { return a.lay < b.lay; });
+            for (const Run& r : runs[c])
+                for (uint32_t k = 0; k < r.count; k++) emit(r.body, r.first + k);
+        }
+    } else {
+        std::vector<uint32_t> cursor(s->bodies.size(), 0);
+        for (uint32_t c = 0; c < s->ncol; c++) {
+            s->colour_begin[c] = pos;
+            for (uint32_t bi = 0; bi < (uint32_t)s->bodies.size(); bi++) {
+                const Body& b = s->bodies[bi];
+                uint32_t& k = cursor[bi];
+                while (k < b.t && b.colour[b.order[k]] == c) emit(bi, k++);
             }
         }
     }
@@ -1543,11 +1702,6 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
     if (pos != s->T) return Fail(ctx, XF_E_INVALID, "internal: schedule covers %u of %u tets", pos, s->T);
 
     BlockTables bt;
-    {
-        int lds = 65536;
-        XF_HIP(ctx, hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
-        s->lds_limit = (size_t)lds;
-    }
     if (s->opts.sweep_blocks) {
         int prc = PackBlocks(s, s->opts.block_lanes, &bt);
         if (prc) return prc;
@@ -1596,7 +1750,6 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
         (rc = DevAlloc(ctx, &s->barrier_err, 1, &s->device_bytes)) ||
         (rc = DevAlloc(ctx, &s->tout, s->T, &s->device_bytes)))
         return rc;
-    XF_HIP(ctx, hipDeviceGetAttribute(&s->n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
     hipStream_t st = ctx->stream;
     XF_HIP(ctx, hipMemcpyAsync(s->X, hX.data(), sizeof(double4) * s->N, hipMemcpyHostToDevice, st));
     XF_HIP(ctx, hipMemcpyAsync(s->O, hO.data(), sizeof(double4) * s->N, hipMemcpyHostToDevice, st));
@@ -1654,7 +1807,7 @@ XF_API int xf_scene_info_get(const xf_scene* s, xf_scene_info* info) {
         if (b.settings.volume_passes != 0 || b.settings.damping > 0.0f || b.settings.pbd_damping > 0.0f) fused = false;
     if (s->nkin || s->manip_on) fused = false;
     info->fused_finish = fused ? 1u : 0u;
-    info->tet_lanes = s->opts.tet_lanes;
+    info->tet_lanes = s->opts.tet_lanes ? s->opts.tet_lanes : s->blk_tet_lanes;
     info->block_lds_limit = (uint32_t)s->lds_limit;
     info->block_node_stride = s->blk_nstride;
     info->contract = s->opts.contract && s->opts.launch_mode == XF_LAUNCH_BLOCKS ? 1u : 0u;
