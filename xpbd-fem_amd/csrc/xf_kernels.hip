@@ -224,8 +224,12 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
         return load_block_tet<AUX>(min(r[2 * j] + lt, last), tloc, tg0, tg1, tg2, tg3, taux);
     };
     auto solve = [&](const BlockTet& t, uint32_t i) {
-        if constexpr (QUAD) block_tet_quad<E, AUX, NS>(t, tid & 3u, xs, bodies, comp1_u, a_u, dt);
-        else block_tet<E, SIM, AUX, DAMP, NS>(t, i, xs, tidx, O, bodies, comp1_u, a_u, dt);
+        if constexpr (QUAD) {
+            const TetMaterial m = tet_material<AUX>(t.ax, comp1_u, a_u);
+            const XfBodyParams& bp = bodies[m.body];
+            const float C[3] = {bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]};
+            block_tet_quad<NS>(t, tid & 3u, xs, E == 7 || (E == 0 && bp.energy == 7), C, m.comp1, m.a, dt);
+        } else block_tet<E, SIM, AUX, DAMP, NS>(t, i, xs, tidx, O, bodies, comp1_u, a_u, dt);
     };
     // each lane's first tet of the phase is t; with OVER, lanes go on to the
     // tets beyond the workgroup's lanes

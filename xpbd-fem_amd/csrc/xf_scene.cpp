@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/xpbdfem.h"
+#include "xf_body.h"
 #include "xf_device.h"
 #include "xf_host_util.h"
 #include "xf_sched.h"
@@ -126,6 +127,12 @@ extern "C" hipError_t xf_launch_frame(hipStream_t s, int energy, bool sim, bool 
                                       const float4* tg2, const float4* tg3, const float4* taux, double4* X,
                                       double4* O, double4* V, const XfBodyParams* bodies, float comp1_u, float a_u,
                                       float dt, float* clock, uint32_t* arrive, uint32_t* err);
+
+extern "C" size_t xf_body_lds_bytes(uint32_t n);
+extern "C" bool xf_body_needs_slots(int energy, bool sim, bool damp, bool passes);
+extern "C" hipError_t xf_launch_body(hipStream_t s, int energy, bool sim, bool aux, bool damp, uint32_t threads,
+                                     uint32_t nbodies, size_t lds_limit, const XfBodyArgs* args,
+                                     const XfBodyData* d);
 
 struct xf_ctx {
     int device = 0;
@@ -340,6 +347,11 @@ struct xf_scene {
     std::vector<std::vector<uint32_t>> blk_lay;
     uint32_t* blk_fin = nullptr;
     uint2* tloc = nullptr;
+    // whole-call launches of small bodies (xf_body.hip; BuildBodyTables):
+    // usable for per-colour step calls when body_threads != 0
+    uint32_t body_threads = 0, body_ncol = 0, body_nmax = 0;
+    uint32_t* body_rec = nullptr;
+    uint2* body_loc = nullptr;
     uint32_t* tout = nullptr;  // per schedule position: the tet's slot in body-concatenated, body-local order
     // kinematic targets of all bodies (global node ids, FP64 positions) and
     // the manipulator (target xyz, node id bits in w; kNoNode: none)
@@ -492,12 +504,32 @@ void ComputeMaterial(xf_scene* s) {
     }
 }
 
+// Whether per-colour step calls run as one launch per call, a workgroup per
+// body (xf_launch_body): the scene has the tables (BuildBodyTables), the
+// energy constrains tets with the terms of energies 3..7, and nothing outside
+// a body moves its nodes.
+bool WholeCalls(const xf_scene* s, int energy) {
+    return s->body_threads != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR &&
+           (energy == 0 || (energy >= 3 && energy <= 7)) && s->nkin == 0 && !s->manip_on;
+}
+
+// Whether the launches of the current settings read the per-tet material
+// slots (taux): per-tet or per-body material, volume passes, or a whole-call
+// launch with passes or damping.
+bool NeedSlots(xf_scene* s) {
+    if (s->aux || s->vpasses > 0) return true;
+    const xf_settings& st = s->bodies[0].settings;  // one body: aux covers several
+    const int energy = (int)KernelEnergy(st.energy);
+    return s->body_threads != 0 && (energy >= 3 && energy <= 7) &&
+           xf_body_needs_slots(energy, st.simultaneous != 0, s->dproj, s->vpasses != 0 || s->post != 0);
+}
+
 int UploadMaterial(xf_scene* s) {
     xf_ctx* ctx = s->ctx;
     bool had_aux = s->aux;
     ComputeMaterial(s);
     if (s->aux != had_aux) DropGraph(s);
-    bool need_taux = s->aux || s->vpasses > 0;
+    bool need_taux = NeedSlots(s);
     if (need_taux && !s->taux) {
         int rc = DevAlloc(ctx, &s->taux, s->T, &s->device_bytes);
         if (rc) return rc;
@@ -819,6 +851,26 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
                                     s->tdmp, s->colour_begin_d, s->N, s->tidx, s->tg[0], s->tg[1], s->tg[2],
                                     s->tg[3], s->taux, s->X, s->O, s->V, s->bp, s->comp1_u, s->a_u, dt, s->clock,
                                     s->arrive, s->barrier_err));
+        if (timer) {
+            XF_HIP(ctx, hipEventRecord(e1, st));
+            timer->ev_proj.push_back(e0);
+            timer->ev_proj.push_back(e1);
+        }
+        return XF_OK;
+    }
+    if (WholeCalls(s, energy)) {
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        if (timer) {
+            XF_HIP(ctx, hipEventCreate(&e0));
+            XF_HIP(ctx, hipEventCreate(&e1));
+            XF_HIP(ctx, hipEventRecord(e0, st));
+        }
+        const XfBodyArgs args = {substeps,     s->body_ncol, s->T, s->body_nmax, s->vpasses, s->post, s->tick_host,
+                                 s->time_host, dt,           s->comp1_u, s->a_u};
+        const XfBodyData data = {s->body_rec, s->body_loc, s->tg[0], s->tg[1], s->tg[2], s->tg[3], s->taux,
+                                 s->tdmp,     s->X,        s->O,     s->V,     s->bp,    s->clock};
+        XF_HIP(ctx, xf_launch_body(st, energy, sim, s->aux, s->dproj, s->body_threads, (uint32_t)s->bodies.size(),
+                                   s->lds_limit, &args, &data));
         if (timer) {
             XF_HIP(ctx, hipEventRecord(e1, st));
             timer->ev_proj.push_back(e0);
@@ -1324,6 +1376,70 @@ int UploadBlocks(xf_scene* s, const BlockTables& bt) {
     return XF_OK;
 }
 
+// Tables of the whole-call launches (xf_body.hip) and the rule for using
+// them: every body's nodes fit the LDS of a workgroup with their O, and one
+// sweep over the colours is estimated shorter in a workgroup per body than as
+// a launch per colour. In microseconds (measured): a phase of up to 64 tets
+// 0.85 (quads), a larger one 1.0 plus 0.5 per 256 tets (a wave on each SIMD);
+// a colour launch 2.7 plus 0.2 per thousand tets of its colour. Leaves
+// body_threads 0 and the tables empty where the launches per colour are the
+// better choice.
+struct BodyTables {
+    std::vector<uint32_t> rec;
+    std::vector<uint2> loc;
+};
+void BuildBodyTables(xf_scene* s, BodyTables* bt) {
+    const uint32_t B = (uint32_t)s->bodies.size();
+    uint32_t nmax = 0, ncol = 0, cmax = 0;
+    for (const Body& b : s->bodies) {
+        nmax = std::max(nmax, (b.n + 3) / 4 * 4);
+        ncol = std::max(ncol, b.ncol);
+    }
+    if (xf_body_lds_bytes(nmax) > s->lds_limit || nmax > 65535) return;
+    ncol += ncol % 2;
+    std::vector<uint32_t> rec(2 * (size_t)B * ncol, 0u);
+    double longest = 0.0, sum = 0.0;
+    for (uint32_t bi = 0; bi < B; bi++) {
+        const Body& b = s->bodies[bi];
+        double us = 0.0;
+        for (uint32_t k = 0; k < b.t;) {
+            const uint32_t c = b.colour[b.order[k]];
+            const uint32_t first = k;
+            while (k < b.t && b.colour[b.order[k]] == c) k++;
+            // a body's tets of a colour are one run of the schedule except
+            // where sweep blocks of several bodies share a slot layout
+            uint32_t lo = UINT32_MAX, hi = 0;
+            for (uint32_t j = first; j < k; j++) {
+                lo = std::min(lo, b.sched_pos[b.order[j]]);
+                hi = std::max(hi, b.sched_pos[b.order[j]]);
+            }
+            const uint32_t count = k - first;
+            if (hi - lo + 1 != count) return;
+            rec[2 * ((size_t)bi * ncol + c)] = lo;
+            rec[2 * ((size_t)bi * ncol + c) + 1] = count;
+            cmax = std::max(cmax, count);
+            us += count <= 64 ? 0.85 : 1.0 + 0.5 * ((count + 255) / 256);
+        }
+        longest = std::max(longest, us);
+        sum += us;
+    }
+    const double whole = std::max(longest, sum / s->n_cu);
+    const double launches = 2.7 * s->ncol + 0.2e-3 * s->T;
+    if (whole >= launches) return;
+    bt->rec = std::move(rec);
+    bt->loc.resize(s->T);
+    for (const Body& b : s->bodies)
+        for (uint32_t t = 0; t < b.t; t++) {
+            const uint32_t* is = &b.tets[4 * (size_t)t];
+            uint32_t l[4];
+            for (int i = 0; i < 4; i++) l[i] = xf_body_slot(is[i]);
+            bt->loc[b.sched_pos[t]] = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        }
+    s->body_ncol = ncol;
+    s->body_nmax = nmax;
+    s->body_threads = std::min(512u, std::max(256u, (cmax + 63) / 64 * 64));
+}
+
 int CheckSettings(xf_ctx* ctx, const xf_settings* st) {
     if (!EnergySupported(st->energy))
         return Fail(ctx, XF_E_INVALID, "energy %u out of range (the Settings field has 5 bits)", st->energy);
@@ -1420,7 +1536,7 @@ XF_API void xf_scene_destroy(xf_scene* s) {
     void* ptrs[] = {s->X,  s->O,     s->V,     s->tidx,  s->tg[0],         s->tg[1],  s->tg[2],
                     s->tg[3], s->taux, s->bp, s->clock, s->counter, s->colour_begin_d, s->arrive,
                     s->barrier_err, s->tdmp, s->rmeta, s->rinfo, s->rnodes, s->rincb, s->rinc, s->rtet,
-                    s->blk_rec, s->blk_node, s->tloc, s->blk_fin, s->tout, s->kin_idx, s->kin_pos, s->manip};
+                    s->blk_rec, s->blk_node, s->tloc, s->blk_fin, s->body_rec, s->body_loc, s->tout, s->kin_idx, s->kin_pos, s->manip};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (xf_scene::AdjBuf* b : {&s->adj_ck_x, &s->adj_ck_v, &s->adj_tape, &s->adj_xs, &s->adj_o, &s->adj_xb,
@@ -1770,6 +1886,17 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
     XF_HIP(ctx, hipMemcpyAsync(s->tg[2], h_tg2.data(), sizeof(float4) * s->T, hipMemcpyHostToDevice, st));
     XF_HIP(ctx, hipMemcpyAsync(s->tdmp, h_tdmp.data(), sizeof(float2) * s->T, hipMemcpyHostToDevice, st));
     if (s->opts.sweep_blocks && (rc = UploadBlocks(s, bt))) return rc;
+    BodyTables body;
+    BuildBodyTables(s, &body);
+    if (s->body_threads) {
+        if ((rc = DevAlloc(ctx, &s->body_rec, body.rec.size(), &s->device_bytes)) ||
+            (rc = DevAlloc(ctx, &s->body_loc, body.loc.size(), &s->device_bytes)))
+            return rc;
+        XF_HIP(ctx, hipMemcpyAsync(s->body_rec, body.rec.data(), sizeof(uint32_t) * body.rec.size(),
+                                   hipMemcpyHostToDevice, st));
+        XF_HIP(ctx, hipMemcpyAsync(s->body_loc, body.loc.data(), sizeof(uint2) * body.loc.size(),
+                                   hipMemcpyHostToDevice, st));
+    }
     uint32_t uzero = 0;
     static const uint32_t kClockZero[kClockWords] = {0u, 0u};  // time 0.0f, tick 0
     XF_HIP(ctx, hipMemcpyAsync(s->clock, kClockZero, sizeof(kClockZero), hipMemcpyHostToDevice, st));
@@ -1846,7 +1973,8 @@ XF_API int xf_scene_step(xf_scene* s, uint32_t substeps, float dt) {
     bool sim;
     int rc = Prepare(s, dt, &energy, &sim);
     if (rc) return rc;
-    if (!s->opts.use_graph || s->opts.launch_mode == XF_LAUNCH_PERSISTENT) {
+    // one launch per call needs no graph
+    if (!s->opts.use_graph || s->opts.launch_mode == XF_LAUNCH_PERSISTENT || WholeCalls(s, energy)) {
         rc = Enqueue(s, substeps, dt, energy, sim, nullptr);
     } else {
         if (!s->graph_exec || s->graph_substeps != substeps || s->graph_dt != dt || s->graph_energy != energy ||
@@ -2662,7 +2790,7 @@ XF_API int xf_scene_adjoint_noalloc(xf_scene* s, uint32_t substeps, float dt, ui
     if (s->material_dirty && !s->taux) {
         bool had = s->aux;
         ComputeMaterial(s);
-        bool need_taux = s->aux || s->vpasses > 0;
+        bool need_taux = NeedSlots(s);
         s->aux = had;
         if (need_taux)
             return Fail(ctx, XF_E_STATE,

@@ -287,23 +287,11 @@ __device__ __forceinline__ void solve_tet(bool yeohFast, const float C[3], doubl
     }
 }
 
-// SolveVolumeOnly for tet i of the sweep order (Fem.cpp:840-867): the
-// (J - 1)^2 term alone with compliance = settings.compliance * volume (taux.w)
-// and a scalar XPBD update. Bodies with fewer than pass + 1 volume passes
-// skip the tet.
-__device__ __forceinline__ void volume_one(uint32_t i, uint32_t pass, const uint4* __restrict__ tidx,
-                                           const float4* __restrict__ tg0, const float4* __restrict__ tg1,
-                                           const float4* __restrict__ tg2, const float4* __restrict__ taux,
-                                           double4* __restrict__ X, const XfBodyParams* __restrict__ bodies,
-                                           float dt) {
-    float4 ax = taux[i];
-    if (pass >= bodies[__float_as_uint(ax.z)].volume_passes) return;
-    uint4 id = tidx[i];
-    float4 q0 = tg0[i], q1 = tg1[i], q2 = tg2[i];
-    double4 na = X[id.x], nb = X[id.y], nc = X[id.z], nd = X[id.w];
+// SolveVolumeOnly of one tet (Fem.cpp:840-867): the (J - 1)^2 term alone with
+// compliance comp = settings.compliance * volume and a scalar XPBD update.
+__device__ __forceinline__ void volume_solve(const float4& q0, const float4& q1, const float4& q2, double x[4][3],
+                                             const float w[4], float comp, float dt) {
     float Qi[3][3] = {{q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, {q1.z, q1.w, q2.x}};
-    double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
-    float w[4] = {(float)na.w, (float)nb.w, (float)nc.w, (float)nd.w};
     float P[3][3];
     gather_p(x, P);
     float U = 0.0f;
@@ -314,7 +302,24 @@ __device__ __forceinline__ void volume_one(uint32_t i, uint32_t pass, const uint
         for (int r = 0; r < 3; r++) g[n][r] = 0.0f;
     volume_term(Qi, P, 1.0f, U, g);
     root_grad(g);
-    constrain1(x, w, U, g, dt, ax.w);
+    constrain1(x, w, U, g, dt, comp);
+}
+
+// volume_solve of tet i of the sweep order (compliance in taux.w). Bodies
+// with fewer than pass + 1 volume passes skip the tet.
+__device__ __forceinline__ void volume_one(uint32_t i, uint32_t pass, const uint4* __restrict__ tidx,
+                                           const float4* __restrict__ tg0, const float4* __restrict__ tg1,
+                                           const float4* __restrict__ tg2, const float4* __restrict__ taux,
+                                           double4* __restrict__ X, const XfBodyParams* __restrict__ bodies,
+                                           float dt) {
+    float4 ax = taux[i];
+    if (pass >= bodies[__float_as_uint(ax.z)].volume_passes) return;
+    uint4 id = tidx[i];
+    float4 q0 = tg0[i], q1 = tg1[i], q2 = tg2[i];
+    double4 na = X[id.x], nb = X[id.y], nc = X[id.z], nd = X[id.w];
+    double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
+    float w[4] = {(float)na.w, (float)nb.w, (float)nc.w, (float)nd.w};
+    volume_solve(q0, q1, q2, x, w, ax.w, dt);
     X[id.x] = make_double4(x[0][0], x[0][1], x[0][2], na.w);
     X[id.y] = make_double4(x[1][0], x[1][1], x[1][2], nb.w);
     X[id.z] = make_double4(x[2][0], x[2][1], x[2][2], nc.w);
@@ -501,7 +506,39 @@ __device__ __forceinline__ bool in_damp_range(const XfBodyParams& bp, float2 dm,
     return pos >= bp.n_tets * k / 8u && pos < bp.n_tets * (k + 1u) / 8u;
 }
 
-// Rayleigh post damping of tet i (DampElement, Fem.cpp:910-929).
+// Whether the Rayleigh post pass / the PBD pass of this substep covers a tet
+// (dm: its surface area and position in the body's sweep order).
+__device__ __forceinline__ bool damps_post(const XfBodyParams& bp, float2 dm, uint32_t tick) {
+    return bp.rtype >= 2u && bp.damping > 0.0f && in_damp_range(bp, dm, tick);
+}
+__device__ __forceinline__ bool damps_pbd(const XfBodyParams& bp, float2 dm, uint32_t tick) {
+    return bp.pbd > 0.0f && in_damp_range(bp, dm, tick);
+}
+
+// Rayleigh post damping of one tet (DampElement, Fem.cpp:910-929) on the
+// velocities v of its nodes.
+template <int E>
+__device__ __forceinline__ void damp_solve(const XfBodyParams& bp, const float4& q0, const float4& q1,
+                                           const float4& q2, const float4& q3, float comp1, float a,
+                                           const double x[4][3], double v[4][3], const float w[4], float dt) {
+    float damp = bp.rtype == 3u ? bp.damping * 8.0f : bp.damping;
+    float C[3] = {bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]};
+    float Qi[3][3] = {{q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, {q1.z, q1.w, q2.x}};
+    float QQ[3] = {q2.y, q2.z, q2.w};
+    float QR[3] = {q3.x, q3.y, q3.z};
+    float U[2], g0[4][3], g1[4][3];
+    element_ug<E>(bp.energy == 7u, C, x, Qi, QQ, QR, comp1, a, U, g0, g1);
+    if constexpr (E == 20 || E == 22) {
+        rayleigh1(v, w, U[0], g0, dt, q3.w, damp);  // SolveElementPixar in DampingMode::On
+    } else if (bp.simultaneous) {
+        rayleigh2(v, w, U, g0, g1, dt, q3.w, comp1, damp);
+    } else {
+        rayleigh1(v, w, U[0], g0, dt, q3.w, damp);
+        rayleigh1(v, w, U[1], g1, dt, comp1, damp);
+    }
+}
+
+// damp_solve of tet i of the sweep order.
 template <int E, bool AUX>
 __device__ __forceinline__ void damp_one(uint32_t i, const uint4* __restrict__ tidx, const float4* __restrict__ tg0,
                                          const float4* __restrict__ tg1, const float4* __restrict__ tg2,
@@ -518,36 +555,30 @@ __device__ __forceinline__ void damp_one(uint32_t i, const uint4* __restrict__ t
         body = __float_as_uint(ax.z);
     }
     const XfBodyParams& bp = bodies[body];
-    if (!(bp.rtype >= 2u && bp.damping > 0.0f) || !in_damp_range(bp, tdmp[i], tick)) return;
-    float damp = bp.rtype == 3u ? bp.damping * 8.0f : bp.damping;
+    if (!damps_post(bp, tdmp[i], tick)) return;
     uint4 id = tidx[i];
     float4 q0 = tg0[i], q1 = tg1[i], q2 = tg2[i], q3 = tg3[i];
     double4 na = X[id.x], nb = X[id.y], nc = X[id.z], nd = X[id.w];
     double4 va = V[id.x], vb = V[id.y], vc = V[id.z], vd = V[id.w];
-    float C[3] = {bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]};
-    float Qi[3][3] = {{q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, {q1.z, q1.w, q2.x}};
-    float QQ[3] = {q2.y, q2.z, q2.w};
-    float QR[3] = {q3.x, q3.y, q3.z};
     double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
     double v[4][3] = {{va.x, va.y, va.z}, {vb.x, vb.y, vb.z}, {vc.x, vc.y, vc.z}, {vd.x, vd.y, vd.z}};
     float w[4] = {(float)na.w, (float)nb.w, (float)nc.w, (float)nd.w};
-    float U[2], g0[4][3], g1[4][3];
-    element_ug<E>(bp.energy == 7u, C, x, Qi, QQ, QR, comp1, a, U, g0, g1);
-    if constexpr (E == 20 || E == 22) {
-        rayleigh1(v, w, U[0], g0, dt, q3.w, damp);  // SolveElementPixar in DampingMode::On
-    } else if (bp.simultaneous) {
-        rayleigh2(v, w, U, g0, g1, dt, q3.w, comp1, damp);
-    } else {
-        rayleigh1(v, w, U[0], g0, dt, q3.w, damp);
-        rayleigh1(v, w, U[1], g1, dt, comp1, damp);
-    }
+    damp_solve<E>(bp, q0, q1, q2, q3, comp1, a, x, v, w, dt);
     V[id.x] = make_double4(v[0][0], v[0][1], v[0][2], 0.0);
     V[id.y] = make_double4(v[1][0], v[1][1], v[1][2], 0.0);
     V[id.z] = make_double4(v[2][0], v[2][1], v[2][2], 0.0);
     V[id.w] = make_double4(v[3][0], v[3][1], v[3][2], 0.0);
 }
 
-// PBD damping of tet i (Geo.cpp:806-809), factor min(1, pbd / surfaceArea).
+// PBD damping of one tet (Geo.cpp:806-809), factor min(1, pbd / surfaceArea).
+__device__ __forceinline__ void pbd_solve(const XfBodyParams& bp, float area, const double x[4][3], double v[4][3],
+                                          const float w[4]) {
+    float f = (bp.rtype == 3u ? bp.pbd_amortized : bp.pbd) / area;
+    f = f < 1.0f ? f : 1.0f;
+    pbd_damp(x, v, w, f);
+}
+
+// pbd_solve of tet i of the sweep order.
 template <bool AUX>
 __device__ __forceinline__ void pbd_one(uint32_t i, const uint4* __restrict__ tidx, const float4* __restrict__ taux,
                                         const float2* __restrict__ tdmp, const double4* __restrict__ X,
@@ -557,16 +588,14 @@ __device__ __forceinline__ void pbd_one(uint32_t i, const uint4* __restrict__ ti
     if constexpr (AUX) body = __float_as_uint(taux[i].z);
     const XfBodyParams& bp = bodies[body];
     float2 dm = tdmp[i];
-    if (!(bp.pbd > 0.0f) || !in_damp_range(bp, dm, tick)) return;
-    float f = (bp.rtype == 3u ? bp.pbd_amortized : bp.pbd) / dm.x;
-    f = f < 1.0f ? f : 1.0f;
+    if (!damps_pbd(bp, dm, tick)) return;
     uint4 id = tidx[i];
     double4 na = X[id.x], nb = X[id.y], nc = X[id.z], nd = X[id.w];
     double4 va = V[id.x], vb = V[id.y], vc = V[id.z], vd = V[id.w];
     double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
     double v[4][3] = {{va.x, va.y, va.z}, {vb.x, vb.y, vb.z}, {vc.x, vc.y, vc.z}, {vd.x, vd.y, vd.z}};
     float w[4] = {(float)na.w, (float)nb.w, (float)nc.w, (float)nd.w};
-    pbd_damp(x, v, w, f);
+    pbd_solve(bp, dm.x, x, v, w);
     V[id.x] = make_double4(v[0][0], v[0][1], v[0][2], 0.0);
     V[id.y] = make_double4(v[1][0], v[1][1], v[1][2], 0.0);
     V[id.z] = make_double4(v[2][0], v[2][1], v[2][2], 0.0);
@@ -626,6 +655,17 @@ __device__ __forceinline__ BlockTet load_block_tet(uint32_t i, const uint2* __re
     if constexpr (AUX) t.ax = taux[i];
     t.loc = tloc[i];
     return t;
+}
+
+// Material and body of a tet: per tet (AUX), else uniform and body 0.
+struct TetMaterial {
+    float comp1, a;
+    uint32_t body;
+};
+template <bool AUX>
+__device__ __forceinline__ TetMaterial tet_material(const float4& ax, float comp1_u, float a_u) {
+    if constexpr (AUX) return {ax.x, ax.y, __float_as_uint(ax.z)};
+    return {comp1_u, a_u, 0u};
 }
 
 // A slot's nodes in LDS, node k at byte k * NS: (x, y) in its first 16
@@ -696,7 +736,7 @@ __device__ __forceinline__ float quad_lane(float v) {
 // lanes 0, 1, 2 hold x, y, z of every vector of the tet (positions,
 // gradients, rows of F), lane 3 the four inverse masses, which are the fourth
 // component of the node records. SolveElementMixed with the simultaneous
-// solve (MixedSel / YeohSkinFast; E = 0 picks per body), damping off, in
+// solve (MixedSel / YeohSkinFast), damping off, in
 // exactly the operations and order of solve_tet:
 //  - P, the gradients, F, the updates: each lane its own component;
 //  - column a of the adjugate is the cross product of rows a + 1 and a + 2 of
@@ -709,27 +749,15 @@ __device__ __forceinline__ float quad_lane(float v) {
 // Results equal block_tet's bit for bit. The chain is about half as long as
 // one lane's (293 against 560 VALU instructions for YeohSkinFast), which
 // counts where a phase has fewer waves than the chip has SIMDs.
-template <int E, bool AUX, uint32_t NS>
-__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<NS> xs,
-                                               const XfBodyParams* __restrict__ bodies, float comp1_u, float a_u,
-                                               float dt) {
-    static_assert(E == 0 || E == 4 || E == 7, "quad lanes take MixedSel / YeohSkinFast");
+// yf: the body's energy is YeohSkinFast, with coefficients C.
+template <uint32_t NS>
+__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<NS> xs, bool yf,
+                                               const float C[3], float comp1, float a, float dt) {
     double* const n0 = xs.comp(t.loc.x & 0xFFFFu, q);
     double* const n1 = xs.comp(t.loc.x >> 16, q);
     double* const n2 = xs.comp(t.loc.y & 0xFFFFu, q);
     double* const n3 = xs.comp(t.loc.y >> 16, q);
     const double x[4] = {*n0, *n1, *n2, *n3};
-
-    float comp1 = comp1_u, a = a_u;
-    uint32_t body = 0;
-    if constexpr (AUX) {
-        comp1 = t.ax.x;
-        a = t.ax.y;
-        body = __float_as_uint(t.ax.z);
-    }
-    const XfBodyParams& bp = bodies[body];
-    const float C[3] = {bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]};
-    const bool yf = (E == 7) || (E == 0 && bp.energy == 7);
     const float Qi[3][3] = {{t.q0.x, t.q0.y, t.q0.z}, {t.q0.w, t.q1.x, t.q1.y}, {t.q1.z, t.q1.w, t.q2.x}};
     const float QQ[3] = {t.q2.y, t.q2.z, t.q2.w};
     const float QR[3] = {t.q3.x, t.q3.y, t.q3.z};
