@@ -19,205 +19,11 @@
 // pins, ground contact. Sphere contact is not differentiated.
 #include <hip/hip_runtime.h>
 
+#include "xf_adj.h"
 #include "xf_device.h"
 #include "xf_element.h"
 
 namespace {
-
-using xf::adjdet;
-using xf::apply_grad;
-using xf::defgrad;
-using xf::dot3;
-using xf::neo_prefactored;
-using xf::root_grad;
-
-// Adjoint of one simultaneous projection (forward: xf::solve_mixed_sim, as
-// xf_kernels.hip solve_tet for E = 4 / 7) in element precision R. x:
-// positions before it; xbar: in, adjoint of the positions after it; out,
-// adjoint of the positions before it. Returns d(loss)/d(log comp0) of this
-// projection.
-template <class R>
-__device__ __forceinline__ R adjoint_tet(bool yeoh, const R C[3], const double x[4][3], const float w[4],
-                                         const R Qi[3][3], const R QQ[3], const R QR[3], R comp0, R comp1, R a, R dt,
-                                         double xbar[4][3]) {
-    R P[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) P[i][r] = (R)(x[i][r] - x[3][r]);
-    R g0n[4][3], U0n;
-    neo_prefactored(QQ, QR, P, U0n, g0n);
-    R U0 = U0n, IM = R(0.0), cpoly = R(0.0), s = R(1.0), g0[4][3];
-#pragma unroll
-    for (int n = 0; n < 4; n++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) g0[n][r] = g0n[n][r];
-    if (yeoh) {
-        IM = U0n - R(3.0);
-        cpoly = C[0] * IM + C[1] * IM * IM + C[2] * IM * IM * IM;
-        U0 = fmax(R(0.0001), cpoly);
-        s = C[0] + R(2.0) * C[1] * IM + R(3.0) * C[2] * IM * IM;
-#pragma unroll
-        for (int n = 0; n < 4; n++)
-#pragma unroll
-            for (int r = 0; r < 3; r++) g0[n][r] = g0n[n][r] * s;
-    }
-    R F[3][3], adj[3][3], G[3][3], g1[4][3];
-    defgrad(Qi, P, F);
-    R J = adjdet(F, adj);
-    R d = J - a;
-    R U1 = R(0.0) + R(1.0) * (d * d);
-    R sv = R(2.0) * d;
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) G[c][r] = adj[c][r] * sv;
-#pragma unroll
-    for (int n = 0; n < 4; n++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) g1[n][r] = R(0.0);
-    apply_grad(G, Qi, g1);
-    root_grad(g1);
-    R alpha0 = comp0 / (dt * dt), alpha1 = comp1 / (dt * dt);
-    R A0 = R(1.0e-22), A1 = R(1.0e-22), A2 = R(1.0e-22);
-#pragma unroll
-    for (int n = 0; n < 4; n++) A0 = A0 + w[n] * dot3(g0[n], g0[n]);
-    A0 = A0 + R(2.0) * U0 * alpha0;
-    R b0 = -R(2.0) * U0;
-#pragma unroll
-    for (int n = 0; n < 4; n++) A1 = A1 + w[n] * dot3(g1[n], g0[n]);
-#pragma unroll
-    for (int n = 0; n < 4; n++) A2 = A2 + w[n] * dot3(g1[n], g1[n]);
-    A2 = A2 + R(2.0) * U1 * alpha1;
-    R b1 = -R(2.0) * U1;
-    R u = R(1.0) / A0, v = R(1.0) / A2;
-    R p = A1 * u, q = A1 * v, be0 = b0 * u, be1 = b1 * v;
-    R Dr = R(1.0) - p * q;
-    R invDet = R(1.0) / fmax(R(0.00000001), Dr);
-    R r0 = be0 - p * be1, r1 = be1 - be0 * q;
-    R l0 = invDet * r0, l1 = invDet * r1;
-
-    R g0b[4][3], g1b[4][3];
-    R l0b = R(0.0), l1b = R(0.0);
-#pragma unroll
-    for (int n = 0; n < 4; n++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            R accb = w[n] * (R)xbar[n][r];
-            l0b = l0b + g0[n][r] * accb;
-            l1b = l1b + g1[n][r] * accb;
-            g0b[n][r] = l0 * accb;
-            g1b[n][r] = l1 * accb;
-        }
-    R invDetb = l0b * r0 + l1b * r1;
-    R r0b = l0b * invDet, r1b = l1b * invDet;
-    R be0b = r0b - r1b * q, be1b = r1b - r0b * p;
-    R pb = R(0.0) - r0b * be1, qb = R(0.0) - r1b * be0;
-    R Drb = Dr > R(0.00000001) ? (R(0.0) - invDetb * invDet * invDet) : R(0.0);
-    pb = pb - Drb * q;
-    qb = qb - Drb * p;
-    R A1b = pb * u + qb * v;
-    R ub = pb * A1 + be0b * b0, vb = qb * A1 + be1b * b1;
-    R b0b = be0b * u, b1b = be1b * v;
-    R A0b = R(0.0) - ub * u * u, A2b = R(0.0) - vb * v * v;
-    R U0b = -R(2.0) * b0b + R(2.0) * alpha0 * A0b;
-    R U1b = -R(2.0) * b1b + R(2.0) * alpha1 * A2b;
-    R alpha0b = R(2.0) * U0 * A0b;
-#pragma unroll
-    for (int n = 0; n < 4; n++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            g0b[n][r] = g0b[n][r] + R(2.0) * A0b * w[n] * g0[n][r] + A1b * w[n] * g1[n][r];
-            g1b[n][r] = g1b[n][r] + A1b * w[n] * g0[n][r] + R(2.0) * A2b * w[n] * g1[n][r];
-        }
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) g1b[i][r] = g1b[i][r] - g1b[3][r];
-    R adjb[3][3], Fb[3][3], Pb[3][3];
-    R svb = R(0.0);
-#pragma unroll
-    for (int m = 0; m < 3; m++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            R Gb = g1b[0][r] * Qi[0][m] + g1b[1][r] * Qi[1][m] + g1b[2][r] * Qi[2][m];
-            adjb[m][r] = Gb * sv;
-            svb = svb + Gb * adj[m][r];
-        }
-    R db = R(2.0) * svb + R(2.0) * d * U1b;
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) Fb[c][r] = db * adj[r][c];
-    {
-        R m00 = F[0][0], m01 = F[0][1], m02 = F[0][2];
-        R m10 = F[1][0], m11 = F[1][1], m12 = F[1][2];
-        R m20 = F[2][0], m21 = F[2][1], m22 = F[2][2];
-        R t;
-        t = adjb[0][0]; Fb[1][1] += t * m22; Fb[2][2] += t * m11; Fb[1][2] -= t * m21; Fb[2][1] -= t * m12;
-        t = adjb[0][1]; Fb[0][1] -= t * m22; Fb[2][2] -= t * m01; Fb[0][2] += t * m21; Fb[2][1] += t * m02;
-        t = adjb[0][2]; Fb[0][1] += t * m12; Fb[1][2] += t * m01; Fb[0][2] -= t * m11; Fb[1][1] -= t * m02;
-        t = adjb[1][0]; Fb[1][0] -= t * m22; Fb[2][2] -= t * m10; Fb[1][2] += t * m20; Fb[2][0] += t * m12;
-        t = adjb[1][1]; Fb[0][0] += t * m22; Fb[2][2] += t * m00; Fb[0][2] -= t * m20; Fb[2][0] -= t * m02;
-        t = adjb[1][2]; Fb[0][0] -= t * m12; Fb[1][2] -= t * m00; Fb[0][2] += t * m10; Fb[1][0] += t * m02;
-        t = adjb[2][0]; Fb[1][0] += t * m21; Fb[2][1] += t * m10; Fb[1][1] -= t * m20; Fb[2][0] -= t * m11;
-        t = adjb[2][1]; Fb[0][0] -= t * m21; Fb[2][1] -= t * m00; Fb[0][1] += t * m20; Fb[2][0] += t * m01;
-        t = adjb[2][2]; Fb[0][0] += t * m11; Fb[1][1] += t * m00; Fb[0][1] -= t * m10; Fb[1][0] -= t * m01;
-    }
-#pragma unroll
-    for (int m = 0; m < 3; m++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) Pb[m][j] = Qi[m][0] * Fb[j][0] + Qi[m][1] * Fb[j][1] + Qi[m][2] * Fb[j][2];
-    R g0nb[4][3], U0nb;
-    if (yeoh) {
-        R polyb = cpoly > R(0.0001) ? U0b : R(0.0);
-        R sb = R(0.0);
-#pragma unroll
-        for (int n = 0; n < 4; n++)
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                sb = sb + g0b[n][r] * g0n[n][r];
-                g0nb[n][r] = g0b[n][r] * s;
-            }
-        U0nb = polyb * s + sb * (R(2.0) * C[1] + R(6.0) * C[2] * IM);
-    } else {
-#pragma unroll
-        for (int n = 0; n < 4; n++)
-#pragma unroll
-            for (int r = 0; r < 3; r++) g0nb[n][r] = g0b[n][r];
-        U0nb = U0b;
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) g0nb[i][r] = g0nb[i][r] - g0nb[3][r];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) Pb[i][r] = Pb[i][r] + U0nb * g0n[i][r] + R(2.0) * QQ[i] * g0nb[i][r];
-    {
-        int k = 0;
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = i + 1; j < 3; j++) {
-#pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    Pb[j][r] = Pb[j][r] + QR[k] * g0nb[i][r];
-                    Pb[i][r] = Pb[i][r] + QR[k] * g0nb[j][r];
-                }
-                ++k;
-            }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            xbar[i][r] = xbar[i][r] + (double)Pb[i][r];
-            xbar[3][r] = xbar[3][r] - (double)Pb[i][r];
-        }
-    return alpha0b * alpha0;
-}
 
 struct TetData {
     float Qi[3][3], QQ[3], QR[3], comp0, comp1, a;
@@ -400,14 +206,10 @@ __global__ __launch_bounds__(256) void xf_predict64(uint32_t n, double4* __restr
     if (i >= n) return;
     double4 xi = X[i], oi = O[i], vi = V[i];
     const XfBodyParams& p = bodies[(uint32_t)oi.w >> 1];
-    const double d = (double)p.dt;
-    const double gdx = (double)p.gravity[0] * d, gdy = (double)p.gravity[1] * d;
-    const double dragf = 1.0 - (double)p.drag;
-    double v[3] = {vi.x + gdx, vi.y + gdy, vi.z + 0.0};
-#pragma unroll
-    for (int r = 0; r < 3; r++) v[r] = v[r] * dragf;
+    double x[3] = {xi.x, xi.y, xi.z}, v[3] = {vi.x, vi.y, vi.z};
+    predict64_one(p, x, v);
     O[i] = make_double4(xi.x, xi.y, xi.z, oi.w);
-    X[i] = make_double4(xi.x + v[0] * d, xi.y + v[1] * d, xi.z + v[2] * d, xi.w);
+    X[i] = make_double4(x[0], x[1], x[2], xi.w);
 }
 
 // One colour of the FP64 projection; REC: records each tet's four node
@@ -425,10 +227,7 @@ __global__ __launch_bounds__(64) void xf_project64(uint32_t begin, uint32_t coun
         project_one<AUX, double, REC>(begin + k, tidx, tg0, tg1, tg2, tg3, taux, X, tape, bodies, comp1_u, a_u, dt);
 }
 
-// End of an FP64 substep for one node: a pinned node returns to O; other
-// nodes take the ground contact in double (static friction when the
-// tangential displacement is within mu * depth, else it shrinks by mu *
-// depth); then V = (X - O) / dt with 1 / dt in double.
+// End of an FP64 substep (finish64_one).
 // xs_out / oo_out (nullable): X after the sweep and O are copied there first.
 __global__ __launch_bounds__(256) void xf_finish64(uint32_t n, double4* __restrict__ X, const double4* __restrict__ O,
                                                    double4* __restrict__ V, const XfBodyParams* __restrict__ bodies,
@@ -442,123 +241,11 @@ __global__ __launch_bounds__(256) void xf_finish64(uint32_t n, double4* __restri
     }
     const uint32_t flags = (uint32_t)oi.w;
     const XfBodyParams& p = bodies[flags >> 1];
-    double x[3] = {xi.x, xi.y, xi.z};
+    double x[3] = {xi.x, xi.y, xi.z}, v[3];
     const double o[3] = {oi.x, oi.y, oi.z};
-    if (flags & 1u) {
-        x[0] = o[0];
-        x[1] = o[1];
-        x[2] = o[2];
-    } else if (p.collide & 1u) {
-        const double gy = (double)p.ground_y;
-        if (x[1] < gy) {
-            const double mu = (double)p.friction;
-            const double depth = gy - x[1];
-            x[1] = gy;
-            const double dx = x[0] - o[0], dz = x[2] - o[2];
-            const double t2 = dx * dx + dz * dz;
-            const double lim = mu * depth;
-            if (t2 <= lim * lim) {
-                x[0] = o[0];
-                x[2] = o[2];
-            } else {
-                const double sc = lim / sqrt(t2);
-                x[0] = x[0] - dx * sc;
-                x[2] = x[2] - dz * sc;
-            }
-        }
-    }
-    const double invdt = 1.0 / (double)p.dt;
+    finish64_one(p, flags, o, x, v);
     X[i] = make_double4(x[0], x[1], x[2], xi.w);
-    V[i] = make_double4((x[0] - o[0]) * invdt, (x[1] - o[1]) * invdt, (x[2] - o[2]) * invdt, 0.0);
-}
-
-// Square root of the element precision.
-__device__ __forceinline__ float rsqrt_of(float x) { return sqrtf(x); }
-__device__ __forceinline__ double rsqrt_of(double x) { return sqrt(x); }
-
-// Reverse of the end of one substep (velocity, pin, ground contact) for one
-// node, with the loss injected first when this substep ends a loss frame:
-// Xb += lw_i * (x_loss - target). xs / o: the node's position before the
-// contact pass and at the substep start (recorded by the forward replay).
-// R: element precision of the forward (float: FP32 contact and 1.0f / dt;
-// double: the FP64 element model). xbv / vbv: the node's Xb, Vb in, Xb out;
-// ob receives Ob.
-template <class R>
-__device__ __forceinline__ void node_end_one(uint32_t i, uint32_t flags, const XfBodyParams& p,
-                                             const double4* __restrict__ xs, const double4* __restrict__ o,
-                                             const double4* __restrict__ xloss, const double4* __restrict__ target,
-                                             const double* __restrict__ lw, double xbv[3], const double vbv[3],
-                                             double ob[3]) {
-    if (xloss) {
-        double4 xl = xloss[i], tg = target[i];
-        double wl = lw[i];
-        xbv[0] = xbv[0] + wl * (xl.x - tg.x);
-        xbv[1] = xbv[1] + wl * (xl.y - tg.y);
-        xbv[2] = xbv[2] + wl * (xl.z - tg.z);
-    }
-    const double invdt = sizeof(R) == 4 ? (double)p.invdt : 1.0 / (double)p.dt;
-    double xcb[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        xcb[r] = xbv[r] + vbv[r] * invdt;
-        ob[r] = 0.0 - vbv[r] * invdt;
-    }
-    double out[3] = {xcb[0], xcb[1], xcb[2]};
-    if (flags & 1u) {
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-            ob[r] = ob[r] + xcb[r];
-            out[r] = 0.0;
-        }
-    } else if (p.collide & 1u) {
-        double4 s4 = xs[i], o4 = o[i];
-        R gy = (R)p.ground_y;
-        R xy = (R)s4.y;
-        if (xy < gy) {
-            R mu = (R)p.friction;
-            R depth = gy - xy;
-            R dx = (R)(s4.x - o4.x), dz = (R)(s4.z - o4.z);
-            R t2 = dx * dx + dz * dz;
-            R lim = mu * depth;
-            out[1] = 0.0;
-            if (t2 <= lim * lim) {
-                ob[0] = ob[0] + xcb[0];
-                ob[2] = ob[2] + xcb[2];
-                out[0] = 0.0;
-                out[2] = 0.0;
-            } else {
-                R L = rsqrt_of(t2);
-                R ux = dx / L, uz = dz / L;
-                R bx = (R)xcb[0], bz = (R)xcb[2];
-                R ubv = ux * bx + uz * bz;
-                R kk = lim / L;
-                R px = kk * (bx - ux * ubv), pz = kk * (bz - uz * ubv);
-                out[0] = xcb[0] - (double)px;
-                out[2] = xcb[2] - (double)pz;
-                ob[0] = ob[0] + (double)px;
-                ob[2] = ob[2] + (double)pz;
-                out[1] = (double)(mu * ubv);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < 3; r++) xbv[r] = out[r];
-}
-
-// Reverse of the prediction (Geo.cpp:307-312) for one node: Xb <- Xb + Ob,
-// Vb <- Xb_pred * dt * (1 - drag) (1 - drag: the FP32 value, or formed in
-// double for the FP64 element model).
-template <class R>
-__device__ __forceinline__ void node_start_one(const XfBodyParams& p, double xb[3], const double ob[3],
-                                               double vb[3]) {
-    const double dt = (double)p.dt;
-    const double dragf = sizeof(R) == 4 ? (double)p.dragf : 1.0 - (double)p.drag;
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const double x0b = xb[r];
-        xb[r] = x0b + ob[r];
-        vb[r] = (x0b * dt) * dragf;
-    }
+    V[i] = make_double4(v[0], v[1], v[2], 0.0);
 }
 
 // Reverse of the node steps around one substep boundary, per node:
@@ -635,29 +322,43 @@ __global__ __launch_bounds__(256) void xf_loss_weights(uint32_t n, const double4
     lw[i] = 2.0 / (double)bodies[body].n_nodes;
 }
 
-// Squared-error sum of one body at one loss substep: thread (j, b) adds
+// Squared-error sum of one body at one loss substep: wave (j, b) adds
 // |x - target|^2 over the body's nodes in node order, component by
-// component, into e[j * nb + b] (one thread per term keeps the summation
-// order of a serial loop).
+// component, into e[j * nb + b]. The lanes form the squares of 64 nodes at a
+// time and one lane adds them, in the order of a serial loop, while the
+// others load the next (one thread that also loaded took 0.2 us a node, its
+// two dependent loads; 425 nodes 91 us).
 __global__ __launch_bounds__(64) void xf_body_sq_err(uint32_t n_loss, uint32_t nb, uint32_t n,
                                                      const double4* __restrict__ xloss,
                                                      const double4* __restrict__ tgt,
                                                      const XfBodyParams* __restrict__ bodies,
                                                      double* __restrict__ e) {
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double sq[2][3 * 64];
+    const uint32_t k = blockIdx.x, lane = threadIdx.x;
     if (k >= n_loss * nb) return;
-    uint32_t j = k / nb, b = k % nb;
+    const uint32_t j = k / nb, b = k % nb;
     const XfBodyParams& bp = bodies[b];
+    const uint32_t cnt = bp.n_nodes;
     const double4* x = xloss + (size_t)n * j + bp.node_base;
     const double4* t = tgt + (size_t)n * j + bp.node_base;
     double acc = 0.0;
-    for (uint32_t i = 0; i < bp.n_nodes; i++) {
-        double d0 = x[i].x - t[i].x, d1 = x[i].y - t[i].y, d2 = x[i].z - t[i].z;
-        acc += d0 * d0;
-        acc += d1 * d1;
-        acc += d2 * d2;
+    for (uint32_t i0 = 0, half = 0; i0 < cnt; i0 += 64, half ^= 1u) {
+        const uint32_t i = i0 + lane;
+        if (i < cnt) {
+            const double4 xi = x[i], ti = t[i];
+            const double d0 = xi.x - ti.x, d1 = xi.y - ti.y, d2 = xi.z - ti.z;
+            sq[half][3 * lane] = d0 * d0;
+            sq[half][3 * lane + 1] = d1 * d1;
+            sq[half][3 * lane + 2] = d2 * d2;
+        }
+        __syncthreads();
+        if (lane == 0) {
+            const uint32_t m = 3u * min(64u, cnt - i0);
+#pragma unroll 8
+            for (uint32_t q = 0; q < m; q++) acc += sq[half][q];
+        }
     }
-    e[k] = acc;
+    if (lane == 0) e[k] = acc;
 }
 
 // L = sum over loss substeps, then bodies, of e / n_b, and each body's share,
@@ -856,7 +557,7 @@ extern "C" hipError_t xf_launch_loss(hipStream_t s, uint32_t n_loss, uint32_t nb
                                      const double4* tgt, const XfBodyParams* bodies, double* e, double* out) {
     uint32_t terms = n_loss * nb;
     if (terms == 0) return hipSuccess;
-    hipLaunchKernelGGL(xf_body_sq_err, dim3((terms + 63) / 64), dim3(64), 0, s, n_loss, nb, n, xloss, tgt, bodies, e);
+    hipLaunchKernelGGL(xf_body_sq_err, dim3(terms), dim3(64), 0, s, n_loss, nb, n, xloss, tgt, bodies, e);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(xf_loss_total, dim3(1), dim3(64), 0, s, n_loss, nb, e, bodies, out);

@@ -39,3 +39,40 @@ struct XfBodyData {
     const XfBodyParams* bodies;
     float* clock;            // left at the end of the call
 };
+
+// Checkpoint windows of the adjoint of small bodies (xf_body_adjoint.hip):
+// one launch replays one window (workgroups [0, replays)) and reverses
+// another (the rest), a workgroup per body. N: nodes of the scene.
+struct XfBodyWindowArgs {
+    uint32_t nbodies;
+    uint32_t replays;   // workgroups that roll a window forward: nbodies or 0
+    uint32_t reverses;  // workgroups that reverse one: nbodies or 0
+    uint32_t ncol, ntet, nmax, N;
+    uint32_t cmax;      // most tets of a body in one colour
+    uint32_t roll_len, rev_len;  // substeps of the two windows
+    uint32_t rev_end;   // substep count at the end of the reversed window
+    uint32_t n_loss;    // loss substeps up to rev_end
+    float dt, comp1, a;
+};
+
+struct XfBodyWindowData {
+    const uint32_t* rec;
+    const uint2* loc;
+    const float4 *tg0, *tg1, *tg2, *tg3, *taux;
+    const XfBodyParams* bodies;
+    const double4* O;    // flags (.w)
+    // roll: start state, and either its records (tape, xs, oo) or its end state (x1, v1)
+    const double4 *x0, *v0;
+    double* tape_rec;
+    double4 *xs_rec, *oo_rec;
+    double4 *x1, *v1;
+    // reverse: records of its window, inverse masses, adjoint state, gradients, loss frames
+    const double* tape_rev;
+    const double4 *xs_rev, *oo_rev, *W;
+    double4 *Xb, *Vb;
+    void* gacc;          // float, or double in the FP64 element model
+    double* glog;
+    const double4 *xloss, *target;
+    const double* lw;
+    const uint32_t* loss_at;
+};

@@ -727,59 +727,70 @@ __device__ __forceinline__ float quad_perm(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), P0 | (P1 << 2) | (P2 << 4) | (P3 << 6), 0xF,
                                                       0xF, true));
 }
-template <int L>
-__device__ __forceinline__ float quad_lane(float v) {
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ double quad_perm(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xFFFFFFFFll), P0 | (P1 << 2) | (P2 << 4) | (P3 << 6), 0xF,
+                                               0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), P0 | (P1 << 2) | (P2 << 4) | (P3 << 6), 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <int L, class R>
+__device__ __forceinline__ R quad_lane(R v) {
     return quad_perm<L, L, L, L>(v);
 }
+// a . b of two vectors held one component per lane, valid in lanes 0 and 1:
+// (x + y) + z, where x + y and y + x round alike.
+template <class R>
+__device__ __forceinline__ R quad_dot(R a, R b) {
+    const R m = a * b;
+    return (m + quad_perm<1, 0, 2, 3>(m)) + quad_lane<2>(m);
+}
 
-// One tet of a block phase on the four lanes of a quad, split by component:
+// Element constants of a tet in the element precision R.
+template <class R>
+struct QuadTet {
+    R Qi[3][3], QQ[3], QR[3], comp0;
+};
+template <class R>
+__device__ __forceinline__ QuadTet<R> quad_tet(const BlockTet& t) {
+    return {{{(R)t.q0.x, (R)t.q0.y, (R)t.q0.z}, {(R)t.q0.w, (R)t.q1.x, (R)t.q1.y}, {(R)t.q1.z, (R)t.q1.w, (R)t.q2.x}},
+            {(R)t.q2.y, (R)t.q2.z, (R)t.q2.w},
+            {(R)t.q3.x, (R)t.q3.y, (R)t.q3.z},
+            (R)t.q3.w};
+}
+
+// The projection of one tet on the four lanes of a quad, split by component:
 // lanes 0, 1, 2 hold x, y, z of every vector of the tet (positions,
-// gradients, rows of F), lane 3 the four inverse masses, which are the fourth
-// component of the node records. SolveElementMixed with the simultaneous
+// gradients, rows of F); x: this lane's component of the four positions (any
+// value in lane 3), w: the inverse masses, in every lane; xn: the component
+// after the projection. SolveElementMixed with the simultaneous
 // solve (MixedSel / YeohSkinFast), damping off, in
-// exactly the operations and order of solve_tet:
+// exactly the operations and order of solve_tet and solve_mixed_sim:
 //  - P, the gradients, F, the updates: each lane its own component;
 //  - column a of the adjugate is the cross product of rows a + 1 and a + 2 of
 //    F, which the lane reads from its neighbours (cofactors that solve_tet
 //    negates come out as the reversed difference, the same value);
-//  - a dot product is each lane's product, then (x + y) + z by DPP, valid in
-//    lanes 0 and 1 (x + y and y + x round alike);
+//  - dot products by quad_dot, so scalars are valid in lanes 0 and 1;
 //  - the 2x2 system: lane 0 holds the I1 row, lane 1 the volume row, so one
 //    reciprocal serves both and the Cramer solve is one expression.
-// Results equal block_tet's bit for bit. The chain is about half as long as
-// one lane's (293 against 560 VALU instructions for YeohSkinFast), which
+// Results equal those of one lane bit for bit. The chain is about half as long
+// as one lane's (293 against 520 VALU instructions for MixedSel), which
 // counts where a phase has fewer waves than the chip has SIMDs.
 // yf: the body's energy is YeohSkinFast, with coefficients C.
-template <uint32_t NS>
-__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<NS> xs, bool yf,
-                                               const float C[3], float comp1, float a, float dt) {
-    double* const n0 = xs.comp(t.loc.x & 0xFFFFu, q);
-    double* const n1 = xs.comp(t.loc.x >> 16, q);
-    double* const n2 = xs.comp(t.loc.y & 0xFFFFu, q);
-    double* const n3 = xs.comp(t.loc.y >> 16, q);
-    const double x[4] = {*n0, *n1, *n2, *n3};
-    const float Qi[3][3] = {{t.q0.x, t.q0.y, t.q0.z}, {t.q0.w, t.q1.x, t.q1.y}, {t.q1.z, t.q1.w, t.q2.x}};
-    const float QQ[3] = {t.q2.y, t.q2.z, t.q2.w};
-    const float QR[3] = {t.q3.x, t.q3.y, t.q3.z};
-    const float comp0 = t.q3.w;
-
-    float P[3], w[4];
+template <class R>
+__device__ __forceinline__ void quad_solve(const QuadTet<R>& t, uint32_t q, const double x[4], const float w[4],
+                                           bool yf, const R C[3], R comp1, R a, R dt, double xn[4]) {
+    R P[3];
 #pragma unroll
-    for (int i = 0; i < 3; i++) P[i] = (float)(x[i] - x[3]);
-#pragma unroll
-    for (int n = 0; n < 4; n++) w[n] = quad_lane<3>((float)x[n]);
-    // a . b in lanes 0 and 1
-    auto dot = [](float a, float b) {
-        const float m = a * b;
-        return (m + quad_perm<1, 0, 2, 3>(m)) + quad_lane<2>(m);
-    };
+    for (int i = 0; i < 3; i++) P[i] = (R)(x[i] - x[3]);
 
     // prefactored I1 (neo_prefactored)
-    float u = 0.0f, g0[4], g1[4];
+    R u = R(0.0), g0[4], g1[4];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        u = u + QQ[i] * dot(P[i], P[i]);
-        g0[i] = (2.0f * QQ[i]) * P[i];
+        u = u + t.QQ[i] * quad_dot(P[i], P[i]);
+        g0[i] = (R(2.0) * t.QQ[i]) * P[i];
     }
     {
         int k = 0;
@@ -787,26 +798,26 @@ __device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, No
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = i + 1; j < 3; j++) {
-                u = u + QR[k] * dot(P[i], P[j]);
-                g0[i] = g0[i] + QR[k] * P[j];
-                g0[j] = g0[j] + QR[k] * P[i];
+                u = u + t.QR[k] * quad_dot(P[i], P[j]);
+                g0[i] = g0[i] + t.QR[k] * P[j];
+                g0[j] = g0[j] + t.QR[k] * P[i];
                 ++k;
             }
     }
-    g0[3] = ((0.0f - g0[0]) - g0[1]) - g0[2];
-    float U0 = u;
+    g0[3] = ((R(0.0) - g0[0]) - g0[1]) - g0[2];
+    R U0 = u;
     if (yf) {
-        const float IM = U0 - 3.0f;
-        U0 = fmaxf(0.0001f, C[0] * IM + C[1] * IM * IM + C[2] * IM * IM * IM);
-        const float gScale = quad_lane<0>(C[0] + 2.0f * C[1] * IM + 3.0f * C[2] * IM * IM);
+        const R IM = U0 - R(3.0);
+        U0 = fmax(R(0.0001), C[0] * IM + C[1] * IM * IM + C[2] * IM * IM * IM);
+        const R gScale = quad_lane<0>(C[0] + R(2.0) * C[1] * IM + R(3.0) * C[2] * IM * IM);
 #pragma unroll
         for (int n = 0; n < 4; n++) g0[n] = g0[n] * gScale;
     }
 
     // (J - a)^2 volume term (volume_term)
-    float F[3], A[3], B[3], adj[3];
+    R F[3], A[3], B[3], adj[3];
 #pragma unroll
-    for (int r = 0; r < 3; r++) F[r] = Qi[0][r] * P[0] + Qi[1][r] * P[1] + Qi[2][r] * P[2];
+    for (int r = 0; r < 3; r++) F[r] = t.Qi[0][r] * P[0] + t.Qi[1][r] * P[1] + t.Qi[2][r] * P[2];
 #pragma unroll
     for (int r = 0; r < 3; r++) {
         A[r] = quad_perm<1, 2, 0, 3>(F[r]);
@@ -815,46 +826,72 @@ __device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, No
     adj[0] = A[1] * B[2] - A[2] * B[1];
     adj[1] = A[2] * B[0] - A[0] * B[2];
     adj[2] = A[0] * B[1] - A[1] * B[0];
-    const float J = quad_lane<0>(F[0] * adj[0] + F[1] * adj[1] + F[2] * adj[2]);
-    const float U1 = (J - a) * (J - a);
-    const float sJ = 2.0f * (J - a);
+    const R J = quad_lane<0>(F[0] * adj[0] + F[1] * adj[1] + F[2] * adj[2]);
+    const R U1 = (J - a) * (J - a);
+    const R sJ = R(2.0) * (J - a);
 #pragma unroll
     for (int c = 0; c < 3; c++) adj[c] = adj[c] * sJ;
 #pragma unroll
-    for (int j = 0; j < 3; j++) g1[j] = 0.0f + (adj[0] * Qi[j][0] + adj[1] * Qi[j][1] + adj[2] * Qi[j][2]);
-    g1[3] = ((0.0f - g1[0]) - g1[1]) - g1[2];
+    for (int j = 0; j < 3; j++) g1[j] = R(0.0) + (adj[0] * t.Qi[j][0] + adj[1] * t.Qi[j][1] + adj[2] * t.Qi[j][2]);
+    g1[3] = ((R(0.0) - g1[0]) - g1[1]) - g1[2];
 
     // EnergyXpbdConstrainSimultaneous<2>, Cramer branch (constrain2)
-    float A0 = 1.0e-22f, A1 = 1.0e-22f, A2 = 1.0e-22f;
+    R A0 = R(1.0e-22), A1 = R(1.0e-22), A2 = R(1.0e-22);
 #pragma unroll
     for (int n = 0; n < 4; n++) {
-        A0 = A0 + w[n] * dot(g0[n], g0[n]);
-        A1 = A1 + w[n] * dot(g1[n], g0[n]);
-        A2 = A2 + w[n] * dot(g1[n], g1[n]);
+        A0 = A0 + w[n] * quad_dot(g0[n], g0[n]);
+        A1 = A1 + w[n] * quad_dot(g1[n], g0[n]);
+        A2 = A2 + w[n] * quad_dot(g1[n], g1[n]);
     }
     const bool row1 = (q & 1u) != 0u;
-    const float U = row1 ? U1 : U0;
-    const float alpha = row1 ? comp1 / (dt * dt) : comp0 / (dt * dt);
-    const float Ad = (row1 ? A2 : A0) + 2.0f * U * alpha;
-    const float invA = 1.0f / Ad;
-    const float be = (-2.0f * U) * invA;  // b0 invA00 | b1 invA11
-    const float pq = A1 * invA;           // A1 invA00 | A1 invA11
-    const float invDet = 1.0f / fmaxf(0.00000001f, 1.0f - pq * quad_perm<1, 0, 2, 3>(pq));
-    const float l = invDet * (be - pq * quad_perm<1, 0, 2, 3>(be));
-    const float l0 = quad_lane<0>(l), l1 = quad_lane<1>(l);
-    double xn[4];
+    const R U = row1 ? U1 : U0;
+    const R alpha = row1 ? comp1 / (dt * dt) : t.comp0 / (dt * dt);
+    const R Ad = (row1 ? A2 : A0) + R(2.0) * U * alpha;
+    const R invA = R(1.0) / Ad;
+    const R be = (R(-2.0) * U) * invA;  // b0 invA00 | b1 invA11
+    const R pq = A1 * invA;             // A1 invA00 | A1 invA11
+    const R invDet = R(1.0) / fmax(R(0.00000001), R(1.0) - pq * quad_perm<1, 0, 2, 3>(pq));
+    const R l = invDet * (be - pq * quad_perm<1, 0, 2, 3>(be));
+    const R l0 = quad_lane<0>(l), l1 = quad_lane<1>(l);
 #pragma unroll
     for (int n = 0; n < 4; n++) {
-        float acc = 0.0f + l0 * g0[n];
+        R acc = R(0.0) + l0 * g0[n];
         acc = acc + l1 * g1[n];
         xn[n] = x[n] + (double)(w[n] * acc);
     }
-    if (q != 3u) {
-        *n0 = xn[0];
-        *n1 = xn[1];
-        *n2 = xn[2];
-        *n3 = xn[3];
+}
+
+// The components of a tet's four nodes in LDS that lane q of its quad holds.
+template <uint32_t NS>
+struct QuadNodes {
+    double* n[4];
+    __device__ __forceinline__ QuadNodes(NodeLds<NS> s, const uint2& loc, uint32_t q)
+        : n{s.comp(loc.x & 0xFFFFu, q), s.comp(loc.x >> 16, q), s.comp(loc.y & 0xFFFFu, q), s.comp(loc.y >> 16, q)} {}
+    // the components, and the inverse masses (the fourth component) in every lane
+    __device__ __forceinline__ void get(double x[4], float w[4]) const {
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = *n[k];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = quad_lane<3>((float)x[k]);
     }
+    // positions only
+    __device__ __forceinline__ void put(uint32_t q, const double x[4]) const {
+        if (q != 3u)
+#pragma unroll
+            for (int k = 0; k < 4; k++) *n[k] = x[k];
+    }
+};
+
+// One tet of a block phase on the four lanes of a quad (quad_solve).
+template <uint32_t NS>
+__device__ __forceinline__ void block_tet_quad(const BlockTet& t, uint32_t q, NodeLds<NS> xs, bool yf,
+                                               const float C[3], float comp1, float a, float dt) {
+    const QuadNodes<NS> nodes(xs, t.loc, q);
+    double x[4], xn[4];
+    float w[4];
+    nodes.get(x, w);
+    quad_solve<float>(quad_tet<float>(t), q, x, w, yf, C, comp1, a, dt, xn);
+    nodes.put(q, xn);
 }
 
 // Collision projection of one unpinned node (no reference counterpart).
