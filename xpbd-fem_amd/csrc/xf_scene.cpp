@@ -128,6 +128,10 @@ extern "C" hipError_t xf_launch_frame(hipStream_t s, int energy, bool sim, bool 
                                       double4* O, double4* V, const XfBodyParams* bodies, float comp1_u, float a_u,
                                       float dt, float* clock, uint32_t* arrive, uint32_t* err);
 
+extern "C" hipError_t xf_launch_pack_state(hipStream_t s, uint32_t n, const double4* X, const double4* V, double* x,
+                                           double* v);
+extern "C" hipError_t xf_launch_unpack_state(hipStream_t s, uint32_t n, const double* x, const double* v, double4* X,
+                                             double4* O, double4* V);
 extern "C" size_t xf_body_lds_bytes(uint32_t n);
 extern "C" bool xf_body_needs_slots(int energy, bool sim, bool damp, bool passes);
 extern "C" hipError_t xf_launch_body_windows(hipStream_t s, bool aux, bool fp64, size_t lds_limit,
@@ -143,6 +147,12 @@ struct xf_ctx {
     hipStream_t stream = nullptr;
     unsigned char* scratch = nullptr;  // this device's copy of xf_adjoint_scratch (device address)
     std::string err;
+    // pinned host memory that node states pass through, in two halves: one is
+    // copied by the host while the device fills (or reads) the other. Allocated
+    // by the first transfer, freed with the context; a context is used by one
+    // thread at a time, and no transfer outlives its call.
+    unsigned char* stage = nullptr;
+    hipEvent_t stage_done[2] = {nullptr, nullptr};
     std::vector<xf_scene*> scenes;  // open scenes, destroyed with the context
 };
 
@@ -155,6 +165,11 @@ constexpr size_t kAdjointScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) unsigned char xf_adjoint_scratch[kAdjointScratchBytes];
 
 namespace {
+
+// Nodes of one half of a context's pinned staging memory (x and v, 3 doubles
+// each): 2 MiB, a few times what PCIe needs to run at its rate.
+constexpr uint32_t kStageNodes = (2u << 20) / 48;
+constexpr size_t kStageHalf = (size_t)48 * kStageNodes;
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -304,6 +319,7 @@ struct xf_scene {
     uint32_t* colour_begin_d = nullptr;  // ncol + 1 offsets (persistent launch)
     uint32_t* arrive = nullptr;          // grid-barrier arrivals (persistent launch)
     uint32_t* barrier_err = nullptr;     // set when a grid barrier timed out
+    bool ran_persistent = false;         // a persistent launch was enqueued (barrier_err may be set)
     // vertex rings in sweep order (colour-major, body-major inside a colour)
     bool rings_host = false, rings_dev = false;
     uint32_t R = 0, rcol = 0, rnmax = 0, rtmax = 0;
@@ -368,8 +384,6 @@ struct xf_scene {
     int n_cu = 256;
     // host mirrors
     std::vector<float4> h_tg3, h_taux;
-    std::vector<double> h_w;       // per node inverse mass
-    std::vector<double> h_oflags;  // per node O.w: (body << 1) | pinned
     std::vector<XfBodyParams> h_bp;  // body table staging (sized at finalize)
     bool material_dirty = true, params_dirty = true;
     bool aux = false;
@@ -849,6 +863,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
             XF_HIP(ctx, hipEventCreate(&e0));
             XF_HIP(ctx, hipEventCreate(&e1));
         }
+        s->ran_persistent = true;
         XF_HIP(ctx, hipMemsetAsync(s->arrive, 0, sizeof(uint32_t), st));
         if (timer) XF_HIP(ctx, hipEventRecord(e0, st));
         XF_HIP(ctx, xf_launch_frame(st, energy, sim, s->aux, s->dproj, blocks, substeps, s->ncol, s->vpasses, s->post,
@@ -1510,6 +1525,9 @@ XF_API int xf_ctx_create(int device, xf_ctx** out) {
 XF_API void xf_ctx_destroy(xf_ctx* ctx) {
     if (!ctx) return;
     while (!ctx->scenes.empty()) xf_scene_destroy(ctx->scenes.back());
+    for (hipEvent_t e : ctx->stage_done)
+        if (e) (void)hipEventDestroy(e);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -1830,15 +1848,11 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
 
     // Nodes.
     std::vector<double4> hX(s->N), hO(s->N), hV(s->N);
-    s->h_w.assign(s->N, 0.0);
-    s->h_oflags.assign(s->N, 0.0);
     for (size_t bi = 0; bi < s->bodies.size(); bi++) {
         const Body& b = s->bodies[bi];
         for (uint32_t i = 0; i < b.n; i++) {
             uint32_t g = b.node_base + i;
             double flags = (double)(((uint32_t)bi << 1) | (b.pinned[i] ? 1u : 0u));
-            s->h_w[g] = (double)b.ec.w[i];
-            s->h_oflags[g] = flags;
             // Node data enters as float and is held in double (Geo.cpp:713),
             // or as the caller's FP64 positions.
             double px, py, pz;
@@ -1851,7 +1865,7 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
                 py = b.xyz64[3 * i + 1];
                 pz = b.xyz64[3 * i + 2];
             }
-            hX[g] = make_double4(px, py, pz, s->h_w[g]);
+            hX[g] = make_double4(px, py, pz, (double)b.ec.w[i]);
             hO[g] = make_double4(px, py, pz, flags);
             hV[g] = make_double4(b.vel[3 * i], b.vel[3 * i + 1], b.vel[3 * i + 2], 0.0);
         }
@@ -1951,8 +1965,14 @@ XF_API int xf_scene_set_settings(xf_scene* s, uint32_t body, const xf_settings* 
     if (body >= s->bodies.size()) return Fail(s->ctx, XF_E_INVALID, "body %u out of range", body);
     int rc = CheckSettings(s->ctx, st);
     if (rc) return rc;
-    s->bodies[body].settings = *st;
-    s->material_dirty = true;
+    xf_settings& now = s->bodies[body].settings;
+    if (memcmp(&now, st, sizeof(now)) == 0) return XF_OK;  // what is uploaded (or waits to be) stays as it is
+    // the per-tet material, and which passes and kernels run (ComputeMaterial, NeedSlots)
+    if (now.energy != st->energy || now.simultaneous != st->simultaneous || now.compliance != st->compliance ||
+        now.poissons_ratio != st->poissons_ratio || now.volume_passes != st->volume_passes ||
+        now.damping != st->damping || now.rayleigh_type != st->rayleigh_type || now.pbd_damping != st->pbd_damping)
+        s->material_dirty = true;
+    now = *st;
     s->params_dirty = true;
     return XF_OK;
 }
@@ -2021,7 +2041,7 @@ namespace {
 // Reports a grid-barrier timeout of an earlier persistent launch (the flag
 // stays set, so the scene keeps failing loudly).
 int CheckBarrier(xf_scene* s) {
-    if (!s->barrier_err) return XF_OK;
+    if (!s->ran_persistent) return XF_OK;
     uint32_t e = 0;
     XF_HIP(s->ctx, hipMemcpyAsync(&e, s->barrier_err, sizeof(uint32_t), hipMemcpyDeviceToHost, s->ctx->stream));
     XF_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
@@ -2036,35 +2056,51 @@ XF_API int xf_scene_sync(xf_scene* s) {
     return s->finalized ? CheckBarrier(s) : XF_OK;
 }
 
+namespace {
+int EnsureStage(xf_ctx* ctx) {
+    if (ctx->stage) return XF_OK;
+    for (hipEvent_t& e : ctx->stage_done)
+        if (!e) XF_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    hipError_t e = hipHostMalloc((void**)&ctx->stage, 2 * kStageHalf, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        ctx->stage = nullptr;
+        return Fail(ctx, XF_E_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", 2 * kStageHalf, hipGetErrorString(e));
+    }
+    return XF_OK;
+}
+}  // namespace
+
 XF_API int xf_scene_get_state(xf_scene* s, uint32_t body, double* x, double* v) {
     if (!s) return XF_E_INVALID;
     if (!s->finalized) return Fail(s->ctx, XF_E_STATE, "scene is not finalized");
     if (body >= s->bodies.size()) return Fail(s->ctx, XF_E_INVALID, "body %u out of range", body);
     const Body& b = s->bodies[body];
-    std::vector<double4> tmp(b.n);
     xf_ctx* ctx = s->ctx;
     XF_HIP(ctx, hipSetDevice(ctx->device));
-    int brc = CheckBarrier(s);
-    if (brc) return brc;
-    if (x) {
-        XF_HIP(ctx, hipMemcpyAsync(tmp.data(), s->X + b.node_base, sizeof(double4) * b.n, hipMemcpyDeviceToHost,
-                                   ctx->stream));
+    int rc = CheckBarrier(s);
+    if (rc) return rc;
+    if (!x && !v) {
         XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        for (uint32_t i = 0; i < b.n; i++) {
-            x[3 * i] = tmp[i].x;
-            x[3 * i + 1] = tmp[i].y;
-            x[3 * i + 2] = tmp[i].z;
-        }
+        return XF_OK;
     }
-    if (v) {
-        XF_HIP(ctx, hipMemcpyAsync(tmp.data(), s->V + b.node_base, sizeof(double4) * b.n, hipMemcpyDeviceToHost,
-                                   ctx->stream));
-        XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        for (uint32_t i = 0; i < b.n; i++) {
-            v[3 * i] = tmp[i].x;
-            v[3 * i + 1] = tmp[i].y;
-            v[3 * i + 2] = tmp[i].z;
-        }
+    if ((rc = EnsureStage(ctx))) return rc;
+    // half h of the staging memory holds nodes [k, k + kStageNodes): x, then v
+    auto count = [&](uint32_t k) { return std::min(kStageNodes, b.n - k); };
+    auto half = [&](uint32_t k) { return reinterpret_cast<double*>(ctx->stage + (k / kStageNodes % 2) * kStageHalf); };
+    auto fill = [&](uint32_t k) -> int {
+        double* h = half(k);
+        XF_HIP(ctx, xf_launch_pack_state(ctx->stream, count(k), s->X + b.node_base + k, s->V + b.node_base + k,
+                                         x ? h : nullptr, v ? h + 3 * (size_t)kStageNodes : nullptr));
+        XF_HIP(ctx, hipEventRecord(ctx->stage_done[k / kStageNodes % 2], ctx->stream));
+        return XF_OK;
+    };
+    if ((rc = fill(0))) return rc;
+    for (uint32_t k = 0; k < b.n; k += kStageNodes) {
+        if (kStageNodes < b.n - k && (rc = fill(k + kStageNodes))) return rc;
+        XF_HIP(ctx, hipEventSynchronize(ctx->stage_done[k / kStageNodes % 2]));
+        const size_t bytes = sizeof(double) * 3 * (size_t)count(k);
+        if (x) memcpy(x + 3 * (size_t)k, half(k), bytes);
+        if (v) memcpy(v + 3 * (size_t)k, half(k) + 3 * (size_t)kStageNodes, bytes);
     }
     return XF_OK;
 }
@@ -2076,28 +2112,23 @@ XF_API int xf_scene_set_state(xf_scene* s, uint32_t body, const double* x, const
     const Body& b = s->bodies[body];
     xf_ctx* ctx = s->ctx;
     XF_HIP(ctx, hipSetDevice(ctx->device));
-    std::vector<double4> tmp(b.n);
-    if (x) {
+    if (!x && !v) return XF_OK;
+    int rc = EnsureStage(ctx);
+    if (rc) return rc;
+    for (uint32_t k = 0; k < b.n; k += kStageNodes) {
+        const uint32_t n = std::min(kStageNodes, b.n - k), h = k / kStageNodes % 2;
+        double* st = reinterpret_cast<double*>(ctx->stage + h * kStageHalf);
+        const size_t bytes = sizeof(double) * 3 * (size_t)n;
+        if (k >= 2 * kStageNodes) XF_HIP(ctx, hipEventSynchronize(ctx->stage_done[h]));
+        if (x) memcpy(st, x + 3 * (size_t)k, bytes);
+        if (v) memcpy(st + 3 * (size_t)kStageNodes, v + 3 * (size_t)k, bytes);
         // positions change; inverse masses keep their current values (pins and
         // kinematic nodes may have dropped theirs to 0)
-        XF_HIP(ctx, hipMemcpyAsync(tmp.data(), s->X + b.node_base, sizeof(double4) * b.n, hipMemcpyDeviceToHost,
-                                   ctx->stream));
-        XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        for (uint32_t i = 0; i < b.n; i++) tmp[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], tmp[i].w);
-        XF_HIP(ctx, hipMemcpyAsync(s->X + b.node_base, tmp.data(), sizeof(double4) * b.n, hipMemcpyHostToDevice,
-                                   ctx->stream));
-        XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        for (uint32_t i = 0; i < b.n; i++) tmp[i].w = s->h_oflags[b.node_base + i];
-        XF_HIP(ctx, hipMemcpyAsync(s->O + b.node_base, tmp.data(), sizeof(double4) * b.n, hipMemcpyHostToDevice,
-                                   ctx->stream));
-        XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        XF_HIP(ctx, xf_launch_unpack_state(ctx->stream, n, x ? st : nullptr, v ? st + 3 * (size_t)kStageNodes : nullptr,
+                                           s->X + b.node_base + k, s->O + b.node_base + k, s->V + b.node_base + k));
+        XF_HIP(ctx, hipEventRecord(ctx->stage_done[h], ctx->stream));
     }
-    if (v) {
-        for (uint32_t i = 0; i < b.n; i++) tmp[i] = make_double4(v[3 * i], v[3 * i + 1], v[3 * i + 2], 0.0);
-        XF_HIP(ctx, hipMemcpyAsync(s->V + b.node_base, tmp.data(), sizeof(double4) * b.n, hipMemcpyHostToDevice,
-                                   ctx->stream));
-        XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    }
+    XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return XF_OK;
 }
 

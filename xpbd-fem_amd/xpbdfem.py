@@ -485,8 +485,8 @@ class Scene:
 
     def get_state(self, body=0):
         n = self.bodies[body][0]
-        x = np.zeros(3 * n, np.float64)
-        v = np.zeros(3 * n, np.float64)
+        x = np.empty(3 * n, np.float64)
+        v = np.empty(3 * n, np.float64)
         self.ctx.check(lib().xf_scene_get_state(self.h, body, x.ctypes.data, v.ctypes.data), "xf_scene_get_state")
         return x, v
 
