@@ -194,8 +194,11 @@ enum {
 
 typedef struct xf_scene_opts {
     uint32_t colour_order;      /* XF_COLOUR_* */
-    uint32_t block_size;        /* workgroup size of per-colour and sweep-block projection
-                                   launches (64, 128, 192, 256), 0 = default (64) */
+    uint32_t block_size;        /* workgroup size of per-colour projection launches and of
+                                   sweep-block launches with tet_lanes 4 (64, 128, 192, 256),
+                                   0 = default (64); other sweep-block launches take 256, or the
+                                   lanes of their largest phase where there are more than two
+                                   workgroups per compute unit */
     uint32_t use_graph;         /* capture each per-colour xf_scene_step call shape in a hipGraph */
     uint32_t launch_mode;       /* XF_LAUNCH_* */
     uint32_t persistent_blocks; /* grid size of the persistent launch, 0 = one per compute unit */
@@ -224,9 +227,9 @@ typedef struct xf_scene_opts {
                                    of a block must fit the LDS of one workgroup (at most 2048). */
     uint32_t block_lanes;       /* sweep blocks: consecutive blocks of a launch colour share one
                                    workgroup while each phase holds at most this many tets (1 to
-                                   256; a block above it gets a workgroup of its own), or 0: the
-                                   largest of 64, 128, 256 that leaves at least 4 workgroups per
-                                   compute unit in every launch colour (else 64) */
+                                   256; a block above it gets a workgroup of its own), or 0: 64,
+                                   or 128 where that would leave more than 11 workgroups per
+                                   compute unit in a launch colour */
     uint32_t separate_finish;   /* sweep blocks: 1 keeps the end of each substep (pinning, contact,
                                    velocity, next prediction) as a node launch of its own; 0: the
                                    last block launch of a substep does it for every node when at

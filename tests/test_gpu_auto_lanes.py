@@ -80,3 +80,29 @@ def test_automatic_lanes_packed_layout(ctx):
     x, v = sc.get_state(0)
     sc.close()
     assert np.array_equal(x, a[0]) and np.array_equal(v, a[1])
+
+
+@pytest.mark.parametrize("dims,lanes,cap", [
+    ((20, 9, 7), 192, 192),     # one slot's phases above 64 tets, few slots: runs of blocks
+    ((112, 33, 31), 0, 64),     # two 64-tet slots per compute unit
+    ((132, 37, 35), 0, 64),     # three, laid out to be so
+    ((132, 37, 35), 200, 200),  # no multiple of the wavefront
+    ((248, 60, 60), 0, 128),    # past the line of the automatic cap
+])
+def test_slot_caps_and_layout(ctx, dims, lanes, cap):
+    """One lane per tet at the edges of the automatic slot cap and with packed
+    layouts of several caps: the reported order is that of a scene of few
+    large slots, and the results are those of per-colour launches."""
+    wl = workloads.beam_yeoh(*dims)
+    wl = dict(wl, substeps=2)
+    a = run(ctx, wl, block_lanes=lanes, tet_lanes=1)
+    b = run(ctx, wl, block_lanes=256, tet_lanes=1)
+    assert a[3]["block_lanes"] == cap
+    assert np.array_equal(a[2], b[2])
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    sc = workloads.make_scene(ctx, wl, sweep_blocks=True, block_lanes=lanes)
+    for _ in range(2):
+        sc.step(wl["substeps"], float(wl["dt"]))
+    x, v = sc.get_state(0)
+    sc.close()
+    assert np.array_equal(x, a[0]) and np.array_equal(v, a[1])

@@ -365,6 +365,7 @@ struct xf_scene {
     // layout index of every block inside its launch colour, per body: the
     // order of the blocks' tets in each colour and of the slots (LayoutBlocks)
     std::vector<std::vector<uint32_t>> blk_lay;
+    uint32_t blk_cap = 0;  // opts.block_lanes, or the automatic slot cap
     uint32_t* blk_fin = nullptr;
     uint2* tloc = nullptr;
     // whole-call launches of small bodies (xf_body.hip; BuildBodyTables):
@@ -901,8 +902,16 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     if (rc) return rc;
     const bool blocks = s->opts.launch_mode == XF_LAUNCH_BLOCKS;
     const bool quad = blocks && TetLanes(s, energy, sim) == 4;
-    // automatic quads: 64 tets a phase on 256 threads (block_size is the workgroup of one-lane launches)
-    const uint32_t blk_threads = quad && s->opts.tet_lanes == 0 ? 256u : block;
+    // Workgroups of the block launches: 256 threads where a launch has at most
+    // two of them per compute unit (loads and write-back in fewer rounds: 96x24x24
+    // beam, one lane per tet, 1.45 ms per frame against 1.53 on 64; 64 mixed
+    // boxes 1.97 against 2.00), else as many as the largest phase has tets
+    // (more idle at the phases' barriers and in nothing else: 192x48x48 beam,
+    // 64-tet slots, 3.2 ms on 64, 4.4 on 256; 288x72x72, 256-tet slots, 9.3 on
+    // 256 threads and 11.9, 12.5 and 15.9 on 192, 128 and 64).
+    uint32_t blk_threads = block;
+    if (blocks && (!quad || s->opts.tet_lanes == 0))
+        blk_threads = quad || s->blk_wide ? 256u : std::min(256u, (std::max(s->blk_pmax, 1u) + 63) / 64 * 64);
     s->blk_tet_lanes = quad ? 4u : 1u;
     // the node phase rides on the substep's last block launch when nothing
     // runs between the sweep and the velocity update (no volume passes), the
@@ -1043,116 +1052,160 @@ struct BlockTables {
 
 // A workgroup of the quad launches sweeps at most this many tets a phase.
 constexpr uint32_t kQuadTets = 64;
+constexpr size_t kResidentSlots = 11;  // and at most so many of them per compute unit, else 128-tet slots
 
-// Layout order of the blocks of every launch colour (blk_lay): body, then
-// block number, or, where slots of kQuadTets tets merged from consecutive
-// blocks would be more than the compute units although the tets would fill
-// no more than all of them, an order in which they are not. Then blocks go,
-// in that order, into the fullest of a few open bins that still holds them
-// (a bin: at most kQuadTets tets in each phase, its nodes within LDS), and the
-// layout is the bins one after another; the few open bins keep a slot's
-// blocks near each other. On the 96x24x24 beam (blocks of 1 to 24 tets a
-// phase) 264 slots a launch become 226 on 256 compute units; the eight
-// compute units that swept two slots took 11 us where the others took 8.
-// Blocks of one launch colour share no node, so their order in memory does
-// not enter the results; the reported sweep order stays body, block, visit.
+// The blocks of one launch colour, for packing them into slots: nph tets per
+// phase and a bound on the nodes of each, by layout index.
+struct BlockSizes {
+    uint32_t nph = 0;
+    std::vector<uint32_t> count, nodes;
+    size_t size() const { return nodes.size(); }
+};
+
+// Slots of consecutive blocks when a slot holds at most cap tets a phase and
+// slot_nodes nodes.
+size_t RunSlots(const BlockSizes& z, uint32_t cap, uint32_t slot_nodes) {
+    std::vector<uint32_t> fill(z.nph, 0);
+    uint32_t nodes = 0;
+    size_t slots = 0;
+    for (size_t m = 0; m < z.size(); m++) {
+        const uint32_t* c = &z.count[m * z.nph];
+        bool fits = slots > 0 && nodes + z.nodes[m] <= slot_nodes;
+        for (uint32_t j = 0; j < z.nph && fits; j++) fits = fill[j] + c[j] <= cap;
+        if (!fits) {
+            slots++;
+            nodes = 0;
+            std::fill(fill.begin(), fill.end(), 0u);
+        }
+        nodes += z.nodes[m];
+        for (uint32_t j = 0; j < z.nph; j++) fill[j] += c[j];
+    }
+    return slots;
+}
+
+// Slots that an order of the blocks can be expected to reach: the fullest
+// phase's tets over the cap, a twentieth more, or runs of consecutive blocks.
+size_t ExpectedSlots(const BlockSizes& z, uint32_t cap, uint32_t slot_nodes) {
+    const size_t runs = RunSlots(z, cap, slot_nodes);
+    std::vector<uint64_t> total(z.nph, 0);
+    for (size_t m = 0; m < z.size(); m++)
+        for (uint32_t j = 0; j < z.nph; j++) total[j] += z.count[m * z.nph + j];
+    const uint64_t most = z.nph ? *std::max_element(total.begin(), total.end()) : 0;
+    return std::min<size_t>(runs, (size_t)((most * 21 + 20 * (uint64_t)cap - 1) / (20 * (uint64_t)cap)));
+}
+
+// An order of the blocks whose runs need few slots: each block, in layout
+// order, goes into the fullest of a few open bins that still holds it; the bins
+// one after another. The few open bins keep a slot's blocks near each other.
+std::vector<uint32_t> BinOrder(const BlockSizes& z, uint32_t cap, uint32_t slot_nodes, size_t* n_bins) {
+    struct Bin {
+        std::vector<uint32_t> fill, members;
+        uint32_t nodes = 0, level = 0;
+    };
+    constexpr size_t kOpen = 16;
+    std::vector<Bin> bins;
+    std::vector<size_t> open;
+    for (size_t m = 0; m < z.size(); m++) {
+        const uint32_t* c = &z.count[m * z.nph];
+        size_t best = open.size();
+        for (size_t o = 0; o < open.size(); o++) {
+            const Bin& b = bins[open[o]];
+            bool fits = b.nodes + z.nodes[m] <= slot_nodes;
+            for (uint32_t j = 0; j < z.nph && fits; j++) fits = b.fill[j] + c[j] <= cap;
+            if (fits && (best == open.size() || b.level > bins[open[best]].level)) best = o;
+        }
+        if (best == open.size()) {
+            if (open.size() == kOpen) {  // close the fullest
+                size_t full = 0;
+                for (size_t o = 1; o < open.size(); o++)
+                    if (bins[open[o]].level > bins[open[full]].level) full = o;
+                open.erase(open.begin() + full);
+            }
+            best = open.size();
+            open.push_back(bins.size());
+            bins.emplace_back();
+            bins.back().fill.assign(z.nph, 0);
+        }
+        Bin& b = bins[open[best]];
+        for (uint32_t j = 0; j < z.nph; j++) {
+            b.fill[j] += c[j];
+            b.level = std::max(b.level, b.fill[j]);
+        }
+        b.nodes += z.nodes[m];
+        b.members.push_back((uint32_t)m);
+    }
+    std::vector<uint32_t> order;
+    order.reserve(z.size());
+    for (const Bin& b : bins) order.insert(order.end(), b.members.begin(), b.members.end());
+    *n_bins = bins.size();
+    return order;
+}
+
+// The automatic slot cap (blk_cap) and the layout order of the blocks of every
+// launch colour (blk_lay).
+//
+// Cap: 64, the tets of one wave or of a quad workgroup, until a compute unit's
+// LDS is full of such slots, then 128, whose larger blocks load a shared node
+// less often. Per 30-substep frame of a beam at 64 and 128: 128x36x36 2.15 and
+// 2.45 ms, 192x48x48 3.21 and 3.34, 216x54x54 (10.97 slots per compute unit
+// and launch) 4.16 and 4.27, 240x60x60 (15.0) 5.69 and 5.34, 288x72x72 10.4 and
+// 9.2; 20-substep frame of 400 mixed boxes (11.5) 6.26 and 6.08.
+//
+// Layout: body, then block number, or BinOrder for the cap where a compute
+// unit then sweeps fewer slots (192x48x48 beam: 3.54 ms as runs, 3.21 so). On the 96x24x24 beam (blocks of 1 to 24 tets a phase) 264 slots
+// a launch become 226 on 256 compute units; the eight compute units that swept
+// two slots took 11 us where the others took 8. Blocks of one launch colour
+// share no node, so their order in memory does not enter the results; the
+// reported sweep order stays body, block, visit.
 void LayoutBlocks(xf_scene* s) {
     const uint32_t slot_nodes = (uint32_t)std::min<size_t>(s->lds_limit / 32, 65535);
     s->blk_lay.assign(s->bodies.size(), std::vector<uint32_t>());
-    struct Block {
-        uint32_t body, k, nodes;
-    };
-    std::vector<Block> blocks[4];
+    BlockSizes z[4];
+    for (int q = 0; q < 4; q++) z[q].nph = s->blk[q].nph;
     for (size_t bi = 0; bi < s->bodies.size(); bi++) {
         const xf::SweepBlocks& sb = s->sweep[bi];
         s->blk_lay[bi].resize(sb.n_blocks);
         for (uint32_t k = 0; k < sb.n_blocks; k++) {
-            s->blk_lay[bi][k] = (uint32_t)blocks[sb.launch[k]].size();
-            blocks[sb.launch[k]].push_back({(uint32_t)bi, k, 0});
+            s->blk_lay[bi][k] = (uint32_t)z[sb.launch[k]].size();
+            z[sb.launch[k]].nodes.push_back(0);
         }
     }
-    // tets per phase of each block, row-major by layout index
-    std::vector<uint32_t> count[4];
-    for (int q = 0; q < 4; q++) count[q].assign(blocks[q].size() * (size_t)s->blk[q].nph, 0);
+    for (BlockSizes& b : z) b.count.assign(b.size() * (size_t)b.nph, 0);
     for (size_t bi = 0; bi < s->bodies.size(); bi++) {
         const xf::SweepBlocks& sb = s->sweep[bi];
         for (uint32_t t = 0; t < s->bodies[bi].t; t++) {
-            const uint32_t k = sb.block[t], q = sb.launch[k];
-            count[q][s->blk_lay[bi][k] * (size_t)s->blk[q].nph + sb.phase[t]]++;
+            const uint32_t k = sb.block[t];
+            BlockSizes& b = z[sb.launch[k]];
+            const size_t m = s->blk_lay[bi][k];
+            b.count[m * b.nph + sb.phase[t]]++;
+            b.nodes[m] = std::min(b.nodes[m] + 4, slot_nodes);  // four a tet bound them
         }
     }
+    const size_t cu = (size_t)s->n_cu;
+    s->blk_cap = s->opts.block_lanes;
+    if (s->blk_cap == 0) {
+        s->blk_cap = kQuadTets;
+        for (const BlockSizes& b : z)
+            if (ExpectedSlots(b, kQuadTets, slot_nodes) > kResidentSlots * cu) s->blk_cap = 128;
+    }
+    std::vector<uint32_t> place[4];  // layout index by position in body, block order
     for (int q = 0; q < 4; q++) {
-        const uint32_t nph = s->blk[q].nph;
-        const size_t nb = blocks[q].size();
-        if (nb <= (size_t)s->n_cu) continue;
-        // slots of consecutive blocks, and the least number of slots any order can reach
-        std::vector<uint64_t> total(nph, 0);
-        std::vector<uint32_t> fill(nph, 0);
-        size_t runs = 1;
-        bool small = true;
-        for (size_t m = 0; m < nb; m++) {
-            const uint32_t* c = &count[q][m * nph];
-            bool fits = true;
-            for (uint32_t j = 0; j < nph; j++) {
-                total[j] += c[j];
-                small = small && c[j] <= kQuadTets;
-                fits = fits && fill[j] + c[j] <= kQuadTets;
-            }
-            if (!fits) {
-                runs++;
-                std::fill(fill.begin(), fill.end(), 0u);
-            }
-            for (uint32_t j = 0; j < nph; j++) fill[j] += c[j];
-        }
-        const uint64_t most = *std::max_element(total.begin(), total.end());
-        if (!small || runs <= (size_t)s->n_cu || most > (uint64_t)kQuadTets * (uint64_t)s->n_cu) continue;
-        // nodes per block: four per tet is enough of a bound here
-        for (size_t m = 0; m < nb; m++)
-            for (uint32_t j = 0; j < nph; j++) blocks[q][m].nodes += 4 * count[q][m * nph + j];
-        struct Bin {
-            std::vector<uint32_t> fill, members;
-            uint32_t nodes = 0, level = 0;
-        };
-        constexpr size_t kOpen = 16;
-        std::vector<Bin> bins;
-        std::vector<size_t> open;
-        for (size_t m = 0; m < nb; m++) {
-            const uint32_t* c = &count[q][m * nph];
-            size_t best = open.size();
-            for (size_t o = 0; o < open.size(); o++) {
-                const Bin& b = bins[open[o]];
-                bool fits = b.nodes + blocks[q][m].nodes <= slot_nodes;
-                for (uint32_t j = 0; j < nph && fits; j++) fits = b.fill[j] + c[j] <= kQuadTets;
-                if (fits && (best == open.size() || b.level > bins[open[best]].level)) best = o;
-            }
-            if (best == open.size()) {
-                if (open.size() == kOpen) {  // close the fullest
-                    size_t full = 0;
-                    for (size_t o = 1; o < open.size(); o++)
-                        if (bins[open[o]].level > bins[open[full]].level) full = o;
-                    open.erase(open.begin() + full);
-                }
-                best = open.size();
-                open.push_back(bins.size());
-                bins.emplace_back();
-                bins.back().fill.assign(nph, 0);
-            }
-            Bin& b = bins[open[best]];
-            for (uint32_t j = 0; j < nph; j++) {
-                b.fill[j] += c[j];
-                b.level = std::max(b.level, b.fill[j]);
-            }
-            b.nodes += blocks[q][m].nodes;
-            b.members.push_back((uint32_t)m);
-        }
-        if (bins.size() > (size_t)s->n_cu) continue;
-        uint32_t next = 0;
-        for (const Bin& b : bins)
-            for (uint32_t m : b.members) s->blk_lay[blocks[q][m].body][blocks[q][m].k] = next++;
+        const size_t runs = RunSlots(z[q], s->blk_cap, slot_nodes);
+        if (runs <= cu) continue;
+        size_t bins = 0;
+        const std::vector<uint32_t> order = BinOrder(z[q], s->blk_cap, slot_nodes, &bins);
+        if ((bins + cu - 1) / cu >= (runs + cu - 1) / cu) continue;
+        place[q].resize(order.size());
+        for (uint32_t i = 0; i < (uint32_t)order.size(); i++) place[q][order[i]] = i;
     }
+    for (size_t bi = 0; bi < s->bodies.size(); bi++)
+        for (uint32_t k = 0; k < s->sweep[bi].n_blocks; k++) {
+            const std::vector<uint32_t>& p = place[s->sweep[bi].launch[k]];
+            if (!p.empty()) s->blk_lay[bi][k] = p[s->blk_lay[bi][k]];
+        }
 }
 
-// Sweep-block tables for the slot cap lanes_opt (0: automatic). Blocks of
+// Sweep-block tables for the slot cap lanes_opt (0: blk_cap). Blocks of
 // launch colour q in layout order (LayoutBlocks: the order of
 // their tets inside each colour q, j) are merged, consecutive ones, into
 // workgroup slots while every phase of the slot holds at most lanes_opt
@@ -1232,21 +1285,8 @@ int PackBlocks(xf_scene* s, uint32_t lanes_opt, BlockTables* bt) {
             gfirst[q].push_back(nblk[q]);
         }
     };
-    const int n_cu = s->n_cu;
-    uint32_t lanes_cap = lanes_opt;
-    if (lanes_cap == 0) {
-        // the largest cap that leaves >= 4 slots per compute unit in every launch colour
-        for (uint32_t cap : {256u, 128u, 64u}) {
-            group(cap);
-            lanes_cap = cap;
-            bool enough = true;
-            for (int q = 0; q < 4; q++)
-                if (nblk[q] && gfirst[q].size() - 1 < 4 * (size_t)n_cu) enough = false;
-            if (enough) break;
-        }
-    } else {
-        group(lanes_cap);
-    }
+    const uint32_t lanes_cap = lanes_opt ? lanes_opt : s->blk_cap;
+    group(lanes_cap);
     s->blk_lanes = lanes_cap;
     uint32_t nslot[4], slot_base[5] = {0, 0, 0, 0, 0};
     std::vector<uint32_t> deal[4];  // per launch colour: slot in layout order -> dispatched slot
