@@ -180,11 +180,12 @@ typedef struct xf_body_desc {
 
 /* Launch modes of xf_scene_step. */
 enum {
-    XF_LAUNCH_PER_COLOUR = 0, /* one launch per colour phase and node phase (hipGraph-captured if use_graph);
-                                 where every body's nodes fit the LDS of a workgroup (64 bytes each: 2,560 on
-                                 gfx950) and that is estimated faster, one launch per step call instead, with
-                                 a workgroup per body (energies 3 to 7 and above 12, no kinematic nodes, no
-                                 manipulator). Same results. */
+    XF_LAUNCH_PER_COLOUR = 0, /* one launch per colour phase and node phase (hipGraph-captured if use_graph).
+                                 Where that is estimated faster, a launch for several colours instead, with
+                                 a workgroup per tile of nodes (energies 3 to 7 and above 12, up to 1,024
+                                 nodes per compute unit, no damping or volume passes, no kinematic nodes,
+                                 no manipulator), or one launch per step call, with a workgroup per body
+                                 (bodies of up to 2,560 nodes on gfx950; passes included). Same results. */
     XF_LAUNCH_PERSISTENT = 1, /* one cooperative launch per step call, grid barriers between phases */
     XF_LAUNCH_BLOCKS = 2      /* needs sweep_blocks: one projection launch per block launch colour
                                  (at most 4 per substep), each workgroup of block_size threads

@@ -129,31 +129,6 @@ __global__ __launch_bounds__(256) void xf_project_colour(
 // schedule position, the tet's four block-local node indices, 16 bits each
 // (x: corners 0 | 1 << 16, y: corners 2 | 3 << 16). The first launch colour
 // of a substep advances the simulation clock (clock != nullptr).
-// A slot's nodes into LDS (stage_nodes) and back (write_nodes), kStage list
-// entries per lane at a time: the batch's id loads are issued together,
-// then its node loads (at clamped in-range positions, so that no branch
-// separates them), so a batch costs two memory round trips whatever its
-// size, where one entry per iteration waits for each id before its node.
-constexpr uint32_t kStage = 4;
-
-template <uint32_t NS>
-__device__ __forceinline__ void stage_nodes(uint32_t tid, uint32_t bs, uint32_t n, const uint32_t* __restrict__ bn,
-                                            const double4* __restrict__ X, NodeLds<NS> xs) {
-    for (uint32_t k0 = tid; k0 < n; k0 += kStage * bs) {
-        uint32_t g[kStage];
-#pragma unroll
-        for (uint32_t u = 0; u < kStage; u++) g[u] = bn[min(k0 + u * bs, n - 1u)];
-        double4 v[kStage];
-#pragma unroll
-        for (uint32_t u = 0; u < kStage; u++) v[u] = X[g[u] != xf::kNoNode ? g[u] : 0u];
-#pragma unroll
-        for (uint32_t u = 0; u < kStage; u++) {
-            const uint32_t k = k0 + u * bs;
-            if (k < n && g[u] != xf::kNoNode) xs.put(k, v[u]);
-        }
-    }
-}
-
 template <uint32_t NS>
 __device__ __forceinline__ void write_nodes(uint32_t tid, uint32_t bs, uint32_t n, const uint32_t* __restrict__ bn,
                                             double4* __restrict__ X, NodeLds<NS> xs) {
@@ -291,8 +266,9 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
 }
 
 #ifndef XF_BLOCKS_ONLY
-// First prediction of a step call from the stored velocity.
-__global__ __launch_bounds__(256) void xf_predict(uint32_t n, double4* __restrict__ X, double4* __restrict__ O,
+// First prediction of a step call from the stored velocity (Xo: X, or the
+// other node array of the tile launches).
+__global__ __launch_bounds__(256) void xf_predict(uint32_t n, const double4* X, double4* Xo, double4* __restrict__ O,
                                                   const double4* __restrict__ V,
                                                   const XfBodyParams* __restrict__ bodies) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -303,7 +279,7 @@ __global__ __launch_bounds__(256) void xf_predict(uint32_t n, double4* __restric
     const XfBodyParams& p = bodies[(uint32_t)oi.w >> 1];
     double v[3] = {vi.x, vi.y, vi.z};
     double x[3] = {xi.x, xi.y, xi.z};
-    predict(p, v, x, &X[i], &O[i], xi.w, oi.w);
+    predict(p, v, x, &Xo[i], &O[i], xi.w, oi.w);
 }
 
 // End of a substep: pin (Geo.cpp:318-322), collisions, velocity
@@ -930,10 +906,10 @@ extern "C" hipError_t xf_launch_volume(hipStream_t s, uint32_t block, uint32_t s
     return hipGetLastError();
 }
 
-extern "C" hipError_t xf_launch_predict(hipStream_t s, uint32_t n, double4* X, double4* O, const double4* V,
-                                        const XfBodyParams* bodies) {
+extern "C" hipError_t xf_launch_predict(hipStream_t s, uint32_t n, const double4* X, double4* Xo, double4* O,
+                                        const double4* V, const XfBodyParams* bodies) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(xf_predict, dim3((n + 255) / 256), dim3(256), 0, s, n, X, O, V, bodies);
+    hipLaunchKernelGGL(xf_predict, dim3((n + 255) / 256), dim3(256), 0, s, n, X, Xo, O, V, bodies);
     return hipGetLastError();
 }
 

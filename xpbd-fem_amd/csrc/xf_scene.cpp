@@ -17,6 +17,7 @@
 
 #include "../../include/xpbdfem.h"
 #include "xf_body.h"
+#include "xf_tile.h"
 #include "xf_device.h"
 #include "xf_host_util.h"
 #include "xf_sched.h"
@@ -68,8 +69,13 @@ extern "C" hipError_t xf_launch_blocks_contract(
     double4* X, double4* O, const XfBodyParams* bodies, float comp1_u, float a_u, float dt, float* clock, bool fin,
     const uint32_t* fextra, uint32_t fmax, const float* tend, bool single_body, bool quad, size_t lds_limit,
     bool wide, uint32_t* nstride);
-extern "C" hipError_t xf_launch_predict(hipStream_t s, uint32_t n, double4* X, double4* O, const double4* V,
-                                        const XfBodyParams* bodies);
+extern "C" hipError_t xf_launch_predict(hipStream_t s, uint32_t n, const double4* X, double4* Xo, double4* O,
+                                        const double4* V, const XfBodyParams* bodies);
+extern "C" hipError_t xf_launch_tile_fill(hipStream_t s, uint32_t n, const uint32_t* pos, float4* const tg[4],
+                                          const float4* taux, float4* const e[4], float4* eaux);
+extern "C" hipError_t xf_launch_tiles(hipStream_t s, int energy, bool sim, bool aux, uint32_t ntile, uint32_t nmax,
+                                      uint32_t lanes, size_t lds_limit, bool advance, const XfTileArgs* args,
+                                      const XfTileData* d);
 extern "C" hipError_t xf_launch_finish(hipStream_t s, bool predict_next, bool single_body, uint32_t n, double4* X,
                                        double4* O, double4* V, const XfBodyParams* bodies, const float* clock);
 extern "C" hipError_t xf_launch_count_nonfinite(hipStream_t s, uint32_t n, const double4* X, uint32_t* count);
@@ -368,9 +374,26 @@ struct xf_scene {
     uint32_t blk_cap = 0;  // opts.block_lanes, or the automatic slot cap
     uint32_t* blk_fin = nullptr;
     uint2* tloc = nullptr;
+    // tile launches (xf_tile.hip; BuildTiles): ntile 0 where the scene has none
+    struct TileSpan {
+        uint32_t nph, nmax;  // colours; most nodes of a tile
+        uint32_t lanes;      // most tets of a tile in one colour, or own nodes
+        size_t meta, rec;    // first in tile_meta and tile_rec
+    };
+    uint32_t ntile = 0, tile_nent = 0;
+    std::vector<TileSpan> tile_spans;
+    double4* X2 = nullptr;  // the other node array
+    uint4* tile_meta = nullptr;
+    uint2* tile_rec = nullptr;
+    uint32_t* tile_node = nullptr;
+    uint32_t* tile_pos = nullptr;
+    uint2* tile_loc = nullptr;
+    float4* tile_tg[4] = {};
+    float4* tile_taux = nullptr;
     // whole-call launches of small bodies (xf_body.hip; BuildBodyTables):
     // usable for per-colour step calls when body_threads != 0
     uint32_t body_threads = 0, body_ncol = 0, body_nmax = 0, body_cmax = 0;
+    double body_us = 0.0;  // estimated time of a sweep
     uint32_t* body_rec = nullptr;
     uint2* body_loc = nullptr;
     uint32_t* tout = nullptr;  // per schedule position: the tet's slot in body-concatenated, body-local order
@@ -523,13 +546,22 @@ void ComputeMaterial(xf_scene* s) {
     }
 }
 
+// Whether per-colour step calls run as tile launches, several colours each:
+// the scene has the plan (BuildTiles), and the sweep is followed by nothing
+// but the node phase.
+bool TileSweeps(const xf_scene* s, int energy) {
+    return s->ntile != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR &&
+           (energy == 0 || (energy >= 3 && energy <= 7)) && s->vpasses == 0 && s->post == 0 && !s->dproj &&
+           s->nkin == 0 && !s->manip_on;
+}
+
 // Whether per-colour step calls run as one launch per call, a workgroup per
 // body (xf_launch_body): the scene has the tables (BuildBodyTables), the
-// energy constrains tets with the terms of energies 3..7, and nothing outside
-// a body moves its nodes.
+// energy constrains tets with the terms of energies 3..7, nothing outside a
+// body moves its nodes, and tile launches are not the shorter way.
 bool WholeCalls(const xf_scene* s, int energy) {
     return s->body_threads != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR &&
-           (energy == 0 || (energy >= 3 && energy <= 7)) && s->nkin == 0 && !s->manip_on;
+           (energy == 0 || (energy >= 3 && energy <= 7)) && s->nkin == 0 && !s->manip_on && !TileSweeps(s, energy);
 }
 
 // Whether the launches of the current settings read the per-tet material
@@ -557,6 +589,14 @@ int UploadMaterial(xf_scene* s) {
     if (need_taux)
         XF_HIP(ctx, hipMemcpyAsync(s->taux, s->h_taux.data(), sizeof(float4) * s->T, hipMemcpyHostToDevice,
                                    ctx->stream));
+    if (s->ntile) {
+        if (need_taux && !s->tile_taux) {
+            int rc = DevAlloc(ctx, &s->tile_taux, s->tile_nent, &s->device_bytes);
+            if (rc) return rc;
+        }
+        XF_HIP(ctx, xf_launch_tile_fill(ctx->stream, s->tile_nent, s->tile_pos, s->tg, need_taux ? s->taux : nullptr,
+                                        s->tile_tg, s->tile_taux));
+    }
     XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s->material_dirty = false;
     return XF_OK;
@@ -775,6 +815,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     hipStream_t st = ctx->stream;
     uint32_t block = s->opts.block_size ? s->opts.block_size : 64;
     uint32_t slabs = s->opts.xcd_slabs;
+    double4* start = s->X;  // where the first prediction goes
     auto node = [&](int kind, bool predict_next) -> int {
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (timer) {
@@ -782,7 +823,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
             XF_HIP(ctx, hipEventCreate(&e1));
             XF_HIP(ctx, hipEventRecord(e0, st));
         }
-        if (kind == 0) XF_HIP(ctx, xf_launch_predict(st, s->N, s->X, s->O, s->V, s->bp));
+        if (kind == 0) XF_HIP(ctx, xf_launch_predict(st, s->N, s->X, start, s->O, s->V, s->bp));
         else
             XF_HIP(ctx, xf_launch_finish(st, predict_next, s->bodies.size() == 1, s->N, s->X, s->O, s->V, s->bp,
                                          s->clock));
@@ -896,6 +937,39 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
             timer->ev_proj.push_back(e0);
             timer->ev_proj.push_back(e1);
         }
+        return XF_OK;
+    }
+    if (TileSweeps(s, energy)) {
+        // the launches alternate between two node arrays and end in X
+        double4* cur = (substeps * s->tile_spans.size()) % 2 ? s->X2 : s->X;
+        start = cur;
+        int rc = node(0, false);
+        if (rc) return rc;
+        for (uint32_t k = 0; k < substeps; k++)
+            for (size_t g = 0; g < s->tile_spans.size(); g++) {
+                const xf_scene::TileSpan& sp = s->tile_spans[g];
+                double4* out = cur == s->X ? s->X2 : s->X;
+                const bool last = g + 1 == s->tile_spans.size();
+                const XfTileArgs args = {sp.nph, s->tile_nent, !last ? 0u : k + 1 < substeps ? 1u : 2u, dt,
+                                         s->comp1_u, s->a_u};
+                const XfTileData data = {s->tile_meta + sp.meta, s->tile_rec + sp.rec, s->tile_node, s->tile_loc,
+                                         s->tile_tg[0], s->tile_tg[1], s->tile_tg[2], s->tile_tg[3], s->tile_taux,
+                                         cur, out, s->O, s->V, s->bp, s->clock};
+                hipEvent_t e0 = nullptr, e1 = nullptr;
+                if (timer) {
+                    XF_HIP(ctx, hipEventCreate(&e0));
+                    XF_HIP(ctx, hipEventCreate(&e1));
+                    XF_HIP(ctx, hipEventRecord(e0, st));
+                }
+                XF_HIP(ctx, xf_launch_tiles(st, energy, sim, s->aux, s->ntile, sp.nmax, sp.lanes,
+                                            s->lds_limit, g == 0, &args, &data));
+                if (timer) {
+                    XF_HIP(ctx, hipEventRecord(e1, st));
+                    timer->ev_proj.push_back(e0);
+                    timer->ev_proj.push_back(e1);
+                }
+                cur = out;
+            }
         return XF_OK;
     }
     int rc = node(0, false);
@@ -1440,9 +1514,10 @@ int UploadBlocks(xf_scene* s, const BlockTables& bt) {
 // sweep over the colours is estimated shorter in a workgroup per body than as
 // a launch per colour. In microseconds (measured): a phase of up to 64 tets
 // 0.85 (quads), a larger one 1.0 plus 0.5 per 256 tets (a wave on each SIMD);
-// a colour launch 2.7 plus 0.2 per thousand tets of its colour. Leaves
+// a colour launch 3.0 plus 0.11 per thousand tets of its colour. Leaves
 // body_threads 0 and the tables empty where the launches per colour are the
 // better choice.
+double ColourLaunchesUs(const xf_scene* s) { return 3.0 * s->ncol + 0.11e-3 * s->T; }
 struct BodyTables {
     std::vector<uint32_t> rec;
     std::vector<uint2> loc;
@@ -1482,9 +1557,8 @@ void BuildBodyTables(xf_scene* s, BodyTables* bt) {
         longest = std::max(longest, us);
         sum += us;
     }
-    const double whole = std::max(longest, sum / s->n_cu);
-    const double launches = 2.7 * s->ncol + 0.2e-3 * s->T;
-    if (whole >= launches) return;
+    s->body_us = std::max(longest, sum / s->n_cu);
+    if (s->body_us >= ColourLaunchesUs(s)) return;
     bt->rec = std::move(rec);
     bt->loc.resize(s->T);
     for (const Body& b : s->bodies)
@@ -1498,6 +1572,65 @@ void BuildBodyTables(xf_scene* s, BodyTables* bt) {
     s->body_nmax = nmax;
     s->body_cmax = cmax;
     s->body_threads = std::min(512u, std::max(256u, (cmax + 63) / 64 * 64));
+}
+
+// Tables of the tile launches where a sweep of them is estimated shorter than
+// whole calls and than a launch per colour.
+int BuildTiles(xf_scene* s, const std::vector<uint4>& tidx) {
+    xf_ctx* ctx = s->ctx;
+    if (s->opts.launch_mode != XF_LAUNCH_PER_COLOUR || s->ncol < 2 || s->bodies.size() > (size_t)s->n_cu ||
+        (uint64_t)s->N > (uint64_t)s->n_cu * 2 * kTileThreads)
+        return XF_OK;
+    // two launches with all phases on quads are the least a plan can come to
+    if (s->body_threads && s->body_us < 9.0 + 0.85 * s->ncol) return XF_OK;
+    XfTileMesh m;
+    m.n_nodes = s->N;
+    m.n_tets = s->T;
+    m.ncol = s->ncol;
+    m.tidx = tidx.data();
+    m.colour_begin = s->colour_begin.data();
+    for (const Body& b : s->bodies) {
+        m.body_begin.push_back(b.node_base);
+        m.xyz.push_back(b.xyz.data());
+    }
+    m.body_begin.push_back(s->N);
+    m.n_cu = (uint32_t)s->n_cu;
+    m.lds_limit = (uint32_t)s->lds_limit;
+    const XfTilePlan plan = PlanTiles(m);
+    if (plan.spans.size() < 2 || plan.n_ent == 0) return XF_OK;
+    const double other = s->body_threads ? s->body_us : ColourLaunchesUs(s);
+    if (plan.us >= other) return XF_OK;
+    int rc;
+    if ((rc = DevAlloc(ctx, &s->X2, s->N, &s->device_bytes)) ||
+        (rc = DevAlloc(ctx, &s->tile_meta, plan.meta.size(), &s->device_bytes)) ||
+        (rc = DevAlloc(ctx, &s->tile_rec, plan.rec.size(), &s->device_bytes)) ||
+        (rc = DevAlloc(ctx, &s->tile_node, plan.n_node, &s->device_bytes)) ||
+        (rc = DevAlloc(ctx, &s->tile_pos, plan.n_ent, &s->device_bytes)) ||
+        (rc = DevAlloc(ctx, &s->tile_loc, plan.n_ent, &s->device_bytes)))
+        return rc;
+    for (float4*& e : s->tile_tg)
+        if ((rc = DevAlloc(ctx, &e, plan.n_ent, &s->device_bytes))) return rc;
+    hipStream_t st = ctx->stream;
+    XF_HIP(ctx, hipMemcpyAsync(s->tile_meta, plan.meta.data(), sizeof(uint4) * plan.meta.size(),
+                               hipMemcpyHostToDevice, st));
+    XF_HIP(ctx, hipMemcpyAsync(s->tile_rec, plan.rec.data(), sizeof(uint2) * plan.rec.size(), hipMemcpyHostToDevice,
+                               st));
+    for (const XfTileSpan& sp : plan.spans) {
+        XF_HIP(ctx, hipMemcpyAsync(s->tile_node + sp.node0, sp.node.get(), sizeof(uint32_t) * sp.n_node,
+                                   hipMemcpyHostToDevice, st));
+        XF_HIP(ctx, hipMemcpyAsync(s->tile_pos + sp.ent0, sp.pos.get(), sizeof(uint32_t) * sp.n_ent,
+                                   hipMemcpyHostToDevice, st));
+        XF_HIP(ctx, hipMemcpyAsync(s->tile_loc + sp.ent0, sp.loc.get(), sizeof(uint2) * sp.n_ent,
+                                   hipMemcpyHostToDevice, st));
+    }
+    XF_HIP(ctx, hipStreamSynchronize(st));
+    s->ntile = plan.ntile;
+    s->tile_nent = plan.n_ent;
+    for (size_t k = plan.spans.size(); k-- > 0;) {  // in sweep order
+        const XfTileSpan& sp = plan.spans[k];
+        s->tile_spans.push_back({sp.nph, sp.nmax, std::max(sp.pmax, plan.own_max), sp.meta, sp.rec});
+    }
+    return XF_OK;
 }
 
 int CheckSettings(xf_ctx* ctx, const xf_settings* st) {
@@ -1599,7 +1732,9 @@ XF_API void xf_scene_destroy(xf_scene* s) {
     void* ptrs[] = {s->X,  s->O,     s->V,     s->tidx,  s->tg[0],         s->tg[1],  s->tg[2],
                     s->tg[3], s->taux, s->bp, s->clock, s->counter, s->colour_begin_d, s->arrive,
                     s->barrier_err, s->tdmp, s->rmeta, s->rinfo, s->rnodes, s->rincb, s->rinc, s->rtet,
-                    s->blk_rec, s->blk_node, s->tloc, s->blk_fin, s->body_rec, s->body_loc, s->tout, s->kin_idx, s->kin_pos, s->manip};
+                    s->blk_rec, s->blk_node, s->tloc, s->blk_fin, s->body_rec, s->body_loc, s->X2, s->tile_meta,
+                    s->tile_rec, s->tile_node, s->tile_pos, s->tile_loc, s->tile_tg[0], s->tile_tg[1], s->tile_tg[2],
+                    s->tile_tg[3], s->tile_taux, s->tout, s->kin_idx, s->kin_pos, s->manip};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (xf_scene::AdjBuf* b : {&s->adj_ck_x, &s->adj_ck_v, &s->adj_tape, &s->adj_xs, &s->adj_o, &s->adj_xb,
@@ -1956,6 +2091,7 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
         XF_HIP(ctx, hipMemcpyAsync(s->body_loc, body.loc.data(), sizeof(uint2) * body.loc.size(),
                                    hipMemcpyHostToDevice, st));
     }
+    if ((rc = BuildTiles(s, h_tidx))) return rc;
     uint32_t uzero = 0;
     static const uint32_t kClockZero[kClockWords] = {0u, 0u};  // time 0.0f, tick 0
     XF_HIP(ctx, hipMemcpyAsync(s->clock, kClockZero, sizeof(kClockZero), hipMemcpyHostToDevice, st));
@@ -2668,7 +2804,7 @@ int ReverseLaunches(xf_scene* s, uint32_t substeps, float dt, int energy, uint32
     auto replay_start = [&](uint32_t w) -> int {
         XF_HIP(ctx, xf_launch_copy2_d4(st, N, s->X, b.ckx + (size_t)N * w, s->V, b.ckv + (size_t)N * w));
         if (fp64) XF_HIP(ctx, xf_launch_predict64(st, N, s->X, s->O, s->V, s->bp, dt, nullptr));
-        else XF_HIP(ctx, xf_launch_predict(st, N, s->X, s->O, s->V, s->bp));
+        else XF_HIP(ctx, xf_launch_predict(st, N, s->X, s->X, s->O, s->V, s->bp));
         return XF_OK;
     };
     // end of replayed substep i of window w (records X and O, then the next prediction)

@@ -700,6 +700,31 @@ struct NodeLds {
     }
 };
 
+// A slot's nodes into LDS (stage_nodes) and back (write_nodes), kStage list
+// entries per lane at a time: the batch's id loads are issued together,
+// then its node loads (at clamped in-range positions, so that no branch
+// separates them), so a batch costs two memory round trips whatever its
+// size, where one entry per iteration waits for each id before its node.
+constexpr uint32_t kStage = 4;
+
+template <uint32_t NS>
+__device__ __forceinline__ void stage_nodes(uint32_t tid, uint32_t bs, uint32_t n, const uint32_t* __restrict__ bn,
+                                            const double4* __restrict__ X, NodeLds<NS> xs) {
+    for (uint32_t k0 = tid; k0 < n; k0 += kStage * bs) {
+        uint32_t g[kStage];
+#pragma unroll
+        for (uint32_t u = 0; u < kStage; u++) g[u] = bn[min(k0 + u * bs, n - 1u)];
+        double4 v[kStage];
+#pragma unroll
+        for (uint32_t u = 0; u < kStage; u++) v[u] = X[g[u] != xf::kNoNode ? g[u] : 0u];
+#pragma unroll
+        for (uint32_t u = 0; u < kStage; u++) {
+            const uint32_t k = k0 + u * bs;
+            if (k < n && g[u] != xf::kNoNode) xs.put(k, v[u]);
+        }
+    }
+}
+
 // One tet of a block phase: nodes from LDS, element data loaded, solved,
 // nodes written back to LDS.
 template <int E, bool SIM, bool AUX, bool DAMP, uint32_t NS>
