@@ -210,8 +210,9 @@ typedef struct xf_scene_opts {
                                    sweeps one spatial slab and node lines are fetched by one L2.
                                    Changes the sweep order inside colours (a valid serial order
                                    still; xf_scene_get_order / xf_scene_get_ring_order report it). */
-    uint32_t ring_lanes;        /* lanes per vertex ring in ring-energy launches: 16, 32, or 0 = 32
-                                   when some ring has more than 16 tets, else 16 */
+    uint32_t ring_lanes;        /* lanes per vertex ring in ring-energy launches: 16, 32, or 0 = by
+                                   the rings of a colour (128 up to two per compute unit, 64 up to
+                                   six, else 32, or 16 when no ring has more than 16 tets) */
     uint32_t sweep_blocks;      /* 1: colour the tets by sweep blocks. Node levels are breadth-first
                                    distances over tet edges from the nodes of least d . p, for a
                                    pair of directions d (x with y, y - z, y + z, z; y with z,

@@ -17,14 +17,19 @@
 //            as uint bits) -- damping passes only
 //   vertex rings in sweep order (colour-major, body-major inside a colour),
 //   built when a body first uses a vertex-ring energy:
-//          rmeta[R] uint4 (node offset, node count, ring-tet offset, tet count)
+//          rmeta[R] uint4 (offset in rnode_more, node count, offset in
+//            rtet_more, tet count)
 //          rinfo[R] uint4 (body id, position in the body's ring sweep order,
 //            ring volume as float bits, 0)
-//          rnodes[]  uint32 global node ids, the ring's own vertex first
-//          rincb[] uint16 per ring node, rinc[4 * ring tets] uint16: each ring
-//            node's (ring tet << 2 | corner) slots in ring-tet order
-//          rtet[2 * ring tets] float4 pairs (QQ0 QQ1 QQ2 QR0 | QR1 QR2 V idx)
-//            idx = four ring-local node indices, one byte each, as float bits
+//          rnode[R][kRingFirst] uint2 (global node id, first | end << 16 of the
+//            node's entries in the incidence lists), the ring's own vertex
+//            first; rnode_more: a ring's nodes beyond those. An entry of the
+//            lists is a (ring tet, corner): node-major, tets ascending.
+//          rtet[R][3][kRingFirst] float4 (QQ0 QQ1 QQ2 QR0 | QR1 QR2 w j | s idx
+//            e01 e23): w = (V_t / 4) / V, j = 1 / V_t * (1/6), s = w / V_t *
+//            (1/6), idx = four ring-local node indices, one byte each, e = the
+//            corners' list entries, 16 bits each; rtet_more: three float4 per
+//            ring tet beyond those
 //   body table  XfBodyParams[B]
 #pragma once
 #include <stdint.h>
@@ -53,7 +58,7 @@ struct XfBodyParams {
     // Vertex-ring energies (SolveSimplex, Geo.cpp:13-64)
     uint32_t n_rings;        // rings of the body (amortized range of the ring damping pass)
     float compliance;        // Settings::compliance
-    float poisson;           // Settings::poissonsRatio
+    float ring_mu, ring_lambda, ring_a;  // material of the ring's constraints (a: J at rest)
     // Node range of the body in the scene (adjoint loss terms)
     uint32_t node_base;
     uint32_t n_nodes;
@@ -68,6 +73,9 @@ struct XfBodyParams {
 // Settings::tickId of the next substep). The first colour launch of a
 // substep advances both; kernels later in the same substep use tick - 1.
 constexpr int kClockWords = 2;
+
+// Nodes and tets of a vertex ring that are found by the ring's index.
+constexpr uint32_t kRingFirst = 32;
 
 // Kernel selector for the projection launch.
 struct XfProjectArgs {

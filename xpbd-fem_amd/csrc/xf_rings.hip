@@ -10,23 +10,33 @@
 // Rings of one colour share no node (the host colours the ring conflict
 // graph), so a colour is one launch with plain gathers and scatters, and
 // colours in order equal the reference's serial sweep over the colour-major
-// ring order. Inside a launch a team of 16 or 32 lanes (a launch option)
-// works on one ring, in LDS, in phases separated by workgroup barriers:
-//   0  load the ring's FP64 node positions and its incidence lists (the ring
-//      volume, a sum of rest volumes, comes precomputed in the same order);
+// ring order. Inside a launch a team of 16, 32, 64 or 128 lanes works on one
+// ring, in LDS, in phases (no barrier between them for a team of one
+// wavefront):
+//   0  load the ring's FP64 node positions and its tets (the ring volume, a
+//      sum of rest volumes, comes precomputed in the same order);
 //   1  per ring tet (lanes in parallel): I1 and J of the tet and their
 //      weighted gradient contributions at its 4 corners;
-//   2  per ring node (lanes in parallel): the contributions of the node's
-//      tets added in ring-tet order (host-built incidence lists; phase 1
-//      wrote them in that order); two lanes add the two energy terms in
-//      ring-tet order;
-//   3  per ring node: SolveSimplex's scaling; then the terms of the
-//      constraint sums (all lanes), one lane per sum adding them in ring-node
-//      order, and one lane the Lagrange multipliers;
+//   2  the contributions of each node's tets added in ring-tet order, a lane
+//      per node and component (host-built incidence lists; phase 1 wrote them
+//      in that order), beside two lanes that add the energy terms;
+//   3  per ring node: SolveSimplex's scaling and the terms of the constraint
+//      sums; then every lane adds the sums in ring-node order and forms the
+//      Lagrange multipliers;
 //   4  per ring node: the position (or velocity) update.
 // Every sum keeps the reference's order (ring tets in OneRing order, ring
 // nodes in OneRing order), compiled with -ffp-contract=off: a serial CPU
 // sweep of the same ring order reproduces the result bit for bit.
+//
+// What bounds it: a colour holds few rings (376 of 24 tets on the 48x12x12
+// beam) and each is one chain of instructions, four cycles apiece, on a
+// wavefront that is alone on its SIMD. With 32 lanes a ring, a lane per node in
+// phase 2 and workgroup barriers it took 14,200 cycles (a colour launch 7.15
+// us): 2,900 in three dependent loads (now two: a ring's first kRingFirst nodes
+// and tets are found by its index), 3,650 in phase 2 (the ring's own vertex has
+// every tet: 24 times six values for one lane), 4,100 in scaling, terms and
+// sums through LDS, 930 in multipliers formed by one lane. Now 9,800 with 32
+// lanes (5.13 us), 8,900 with 64, 8,400 with 128 (4.63).
 #include <hip/hip_runtime.h>
 
 #include "xf_device.h"
@@ -35,87 +45,131 @@
 
 namespace {
 
-// Floats per ring tet in LDS: weighted I1 and J, then the I1 and J gradient
-// contributions at its 4 corners (4 x 6), stored at the corners' entries of
-// the incidence lists.
-constexpr uint32_t kTetFloats = 2 + 12 + 12;
-constexpr uint32_t kScalars = 16;
-// Incidence entries per lane whose loads phase 0 issues up front.
-constexpr uint32_t kIncLoads = 4;
+// Floats per ring tet in LDS: five entries of six, four of the tet's I1 and J
+// gradient contributions at its corners, at the corners' entries of the
+// incidence lists, and one that starts with its weighted I1 and J.
+constexpr uint32_t kTetFloats = 6 * 5;
 
-// LDS of one ring team: positions [3][nmax] double, inverse masses [nmax],
-// gradients [6][nmax] (g0 xyz, g1 xyz), per-node velocity-like vectors
-// [3][nmax] (X - O, or V), per-tet contributions [tmax * kTetFloats]
-// (energy terms [tmax][2], then gradient contributions [4 tmax][6] in
-// incidence-entry order; reused for the constraint-sum terms), scalars
-// [kScalars], incidence lists: per-node starts [nmax + 1], entries [4 tmax]
-// and their inverse [4 tmax] (uint16).
+// LDS of one ring team: entries [5 tmax][6] (corners in incidence-entry order,
+// then the tets; reused for the terms of the constraint sums), positions
+// [3][nmax] double, inverse masses [nmax], gradients [6][nmax] (g0 xyz, g1
+// xyz), the nodes' incidence lists (first entry, end) [nmax], the two energy
+// sums.
+__host__ __device__ inline size_t ring_round16(size_t b) { return (b + 15) & ~(size_t)15; }
+__host__ __device__ inline size_t ring_entry_bytes(uint32_t nmax, uint32_t tmax) {
+    const size_t e = (size_t)tmax * kTetFloats, t = 5 * ring_round16(nmax);
+    return ring_round16(4 * (e > t ? e : t));
+}
 __host__ __device__ inline size_t ring_team_bytes(uint32_t nmax, uint32_t tmax) {
-    size_t b = 8 * 3 * (size_t)nmax + 4 * ((size_t)nmax * (1 + 6 + 3) + (size_t)tmax * kTetFloats + kScalars) +
-               2 * ((size_t)nmax + 1 + 8 * (size_t)tmax);
-    return (b + 7) & ~(size_t)7;
+    return ring_entry_bytes(nmax, tmax) + ring_round16(8 * 3 * (size_t)nmax + 4 * ((size_t)nmax * (1 + 6 + 1) + 2));
 }
 
 struct Team {
     double* xs;
-    float *ws, *g, *v, *c, *sc;
-    uint16_t *incb, *inc, *inv;
+    float *ws, *g, *c, *sc;
+    uint32_t* seg;
     uint32_t nmax;
     __device__ double& x(uint32_t r, uint32_t n) const { return xs[r * nmax + n]; }
-    __device__ float& gr(uint32_t k, uint32_t r, uint32_t n) const { return g[(k * 3 + r) * nmax + n]; }
-    __device__ float& vr(uint32_t r, uint32_t n) const { return v[r * nmax + n]; }
 };
+
+// LDS writes of a team's lanes before, reads after. The lanes of up to 64 are
+// of one wavefront, whose LDS accesses complete in order: only the compiler is
+// held. Every lane of a workgroup reaches every barrier.
+template <uint32_t LANES>
+__device__ __forceinline__ void team_sync() {
+    if constexpr (LANES > 64u) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+// A value that the lanes of a team share, in a scalar register where a team is
+// of whole wavefronts (its loads and branches are then scalar too).
+template <uint32_t LANES>
+__device__ __forceinline__ uint32_t team_value(uint32_t v) {
+    return LANES >= 64u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)v) : v;
+}
+
+// a[0] + a[6] + a[12] + ... (n terms), in order from 0. Eight loads are in
+// flight at a time, those past the last term in a remainder (LDS of the
+// workgroup or past its end, where reads give 0) not used; adding 0 in their
+// place is exact, as the sum is never -0.
+__device__ __forceinline__ float ordered_sum(const float* a, uint32_t n) {
+    float s = 0.0f;
+    for (; n >= 8u; n -= 8u, a += 48) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = a[6 * u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s = s + v[u];
+    }
+    if (n > 0u) {
+        float v[7];
+#pragma unroll
+        for (int u = 0; u < 7; u++) v[u] = a[6 * u];
+#pragma unroll
+        for (uint32_t u = 0; u < 7; u++) s = s + (u < n ? v[u] : 0.0f);
+    }
+    return s;
+}
 
 using xf::adjdet;
 using xf::dot3;
 
 // Phase 1 for ring tet k (CalculateElementEnergyAndGradients for a linear
-// tet, Fem.cpp:941-973): c[2 k] = w_t I1, c[2 k + 1] = w_t J and, for corner
-// j at incidence entry e = inv[4 k + j], c[2 tmax + 6 e + r] = w_t dI1/dx_j
-// and c[2 tmax + 6 e + 3 + r] = w_t dJ/dx_j, with w_t = (V_t / 4) / V. The
-// node sums of phase 2 then read each node's entries contiguously.
-__device__ void ring_tet(const Team& T, float4 a, float4 b, float vsum, uint32_t k, uint32_t tmax) {
-    uint32_t bits = __float_as_uint(b.w);
-    uint32_t li[4] = {bits & 255u, (bits >> 8) & 255u, (bits >> 16) & 255u, bits >> 24};
+// tet, Fem.cpp:941-973): entry 4 nt + k holds w_t I1 and w_t J and, for corner
+// j, its incidence entry w_t dI1/dx_j and w_t dJ/dx_j, with w_t = (V_t / 4) /
+// V. The sums of phase 2 then read each node's entries, and the energies, at
+// one stride. a, b, d: the tet's record. I, V: the I1 half, the J half.
+template <bool I, bool V>
+__device__ __forceinline__ void ring_tet(const Team& T, float4 a, float4 b, float4 d, uint32_t k, uint32_t nt) {
+    const uint32_t bits = __float_as_uint(d.y), e01 = __float_as_uint(d.z), e23 = __float_as_uint(d.w);
+    const uint32_t li[4] = {bits & 255u, (bits >> 8) & 255u, (bits >> 16) & 255u, bits >> 24};
+    const uint32_t en[4] = {e01 & 0xFFFFu, e01 >> 16, e23 & 0xFFFFu, e23 >> 16};
     float P[3][3];
     for (int i = 0; i < 3; i++)
         for (uint32_t r = 0; r < 3; r++) P[i][r] = (float)(T.x(r, li[i]) - T.x(r, li[3]));
-    const float QQ[3] = {a.x, a.y, a.z}, QR[3] = {a.w, b.x, b.y};
-    float vt = b.z;
-    float ew = (vt / 4.0f) / vsum;
-    // CalculateIncompressibleNeoHookeanEnergyAndGradients (Fem.cpp:164-190)
-    float I1 = 0.0f, gI[4][3];
-    for (int i = 0; i < 3; i++) {
-        I1 = I1 + QQ[i] * dot3(P[i], P[i]);
-        for (int r = 0; r < 3; r++) gI[i][r] = (2.0f * QQ[i]) * P[i][r];
-    }
-    int q = 0;
-    for (int i = 0; i < 3; i++)
-        for (int j = i + 1; j < 3; j++) {
-            I1 = I1 + QR[q] * dot3(P[i], P[j]);
-            for (int r = 0; r < 3; r++) gI[i][r] = gI[i][r] + QR[q] * P[j][r];
-            for (int r = 0; r < 3; r++) gI[j][r] = gI[j][r] + QR[q] * P[i][r];
-            ++q;
-        }
-    for (int r = 0; r < 3; r++) gI[3][r] = ((0.0f - gI[0][r]) - gI[1][r]) - gI[2][r];
-    // energy terms at c[2 k + q]; corner j's gradients at the entry the
-    // incidence lists give (tet k, corner j): c[2 tmax + 6 e + 0..5]
+    const float ew = b.z;
     float* slot[4];
-    for (int n = 0; n < 4; n++) slot[n] = T.c + 2 * tmax + 6 * (uint32_t)T.inv[4 * k + n];
-    T.c[2 * k] = ew * I1;
-    for (int n = 0; n < 4; n++)
-        for (int r = 0; r < 3; r++) slot[n][r] = ew * gI[n][r];
-    // J of the tet from mat3 PP with rows P_i (Fem.cpp:960-970)
-    float M[3][3], adj[3][3];
-    for (int j = 0; j < 3; j++)
-        for (int r = 0; r < 3; r++) M[j][r] = P[r][j];
-    float det = adjdet(M, adj);
-    float J = ((1.0f / vt) * (1.0f / 6.0f)) * det;
-    T.c[2 * k + 1] = ew * J;
-    float sJ = (ew / vt) * (1.0f / 6.0f);
-    for (int n = 0; n < 3; n++)
-        for (int r = 0; r < 3; r++) slot[n][3 + r] = sJ * adj[n][r];
-    for (int r = 0; r < 3; r++) slot[3][3 + r] = sJ * (((-adj[0][r]) - adj[1][r]) - adj[2][r]);
+    for (int n = 0; n < 4; n++) slot[n] = T.c + 6 * en[n];
+    float* sum = T.c + 6 * (4 * nt + k);
+    if constexpr (I) {
+        // CalculateIncompressibleNeoHookeanEnergyAndGradients (Fem.cpp:164-190)
+        const float QQ[3] = {a.x, a.y, a.z}, QR[3] = {a.w, b.x, b.y};
+        float I1 = 0.0f, gI[4][3];
+        for (int i = 0; i < 3; i++) {
+            I1 = I1 + QQ[i] * dot3(P[i], P[i]);
+            for (int r = 0; r < 3; r++) gI[i][r] = (2.0f * QQ[i]) * P[i][r];
+        }
+        int q = 0;
+        for (int i = 0; i < 3; i++)
+            for (int j = i + 1; j < 3; j++) {
+                I1 = I1 + QR[q] * dot3(P[i], P[j]);
+                for (int r = 0; r < 3; r++) gI[i][r] = gI[i][r] + QR[q] * P[j][r];
+                for (int r = 0; r < 3; r++) gI[j][r] = gI[j][r] + QR[q] * P[i][r];
+                ++q;
+            }
+        for (int r = 0; r < 3; r++) gI[3][r] = ((0.0f - gI[0][r]) - gI[1][r]) - gI[2][r];
+        sum[0] = ew * I1;
+        for (int n = 0; n < 4; n++)
+            for (int r = 0; r < 3; r++) slot[n][r] = ew * gI[n][r];
+    }
+    if constexpr (V) {
+        // J of the tet from mat3 PP with rows P_i (Fem.cpp:960-970)
+        float M[3][3], adj[3][3];
+        for (int j = 0; j < 3; j++)
+            for (int r = 0; r < 3; r++) M[j][r] = P[r][j];
+        float det = adjdet(M, adj);
+        float J = b.w * det;
+        sum[1] = ew * J;
+        const float sJ = d.x;
+        for (int n = 0; n < 3; n++)
+            for (int r = 0; r < 3; r++) slot[n][3 + r] = sJ * adj[n][r];
+        for (int r = 0; r < 3; r++) slot[3][3 + r] = sJ * (((-adj[0][r]) - adj[1][r]) - adj[2][r]);
+    }
 }
 
 // One colour of the ring sweep. POST = false: project positions
@@ -127,11 +181,11 @@ __device__ void ring_tet(const Team& T, float4 a, float4 b, float vsum, uint32_t
 template <bool POST, uint32_t LANES>
 __global__ __launch_bounds__(256) void xf_ring_colour(
     uint32_t begin, uint32_t count, uint32_t slabs, uint32_t nmax, uint32_t tmax, const uint4* __restrict__ rmeta,
-    const uint4* __restrict__ rinfo, const uint32_t* __restrict__ rnodes, const uint16_t* __restrict__ rincb,
-    const uint16_t* __restrict__ rinc, const float4* __restrict__ rtet, double4* __restrict__ X,
+    const uint4* __restrict__ rinfo, const uint2* __restrict__ rnode, const float4* __restrict__ rtet,
+    const uint2* __restrict__ rnode_more, const float4* __restrict__ rtet_more, double4* __restrict__ X,
     const double4* __restrict__ O, double4* __restrict__ V, const XfBodyParams* __restrict__ bodies, float dt,
     float* __restrict__ clock) {
-    extern __shared__ double xf_ring_lds[];
+    extern __shared__ double2 xf_ring_lds[];
     if (!POST && clock != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
         clock[0] = clock[0] + dt;
         uint32_t* tick = reinterpret_cast<uint32_t*>(clock) + 1;
@@ -140,36 +194,35 @@ __global__ __launch_bounds__(256) void xf_ring_colour(
     const uint32_t lane = threadIdx.x % LANES, team = threadIdx.x / LANES;
     Team T;
     T.nmax = nmax;
-    T.xs = reinterpret_cast<double*>(reinterpret_cast<char*>(xf_ring_lds) + team * ring_team_bytes(nmax, tmax));
+    T.c = reinterpret_cast<float*>(reinterpret_cast<char*>(xf_ring_lds) + team * ring_team_bytes(nmax, tmax));
+    T.xs = reinterpret_cast<double*>(reinterpret_cast<char*>(T.c) + ring_entry_bytes(nmax, tmax));
     T.ws = reinterpret_cast<float*>(T.xs + 3 * nmax);
     T.g = T.ws + nmax;
-    T.v = T.g + 6 * nmax;
-    T.c = T.v + 3 * nmax;
-    T.sc = T.c + tmax * kTetFloats;
-    T.incb = reinterpret_cast<uint16_t*>(T.sc + kScalars);
-    T.inc = T.incb + nmax + 1;
-    T.inv = T.inc + 4 * tmax;
+    T.seg = reinterpret_cast<uint32_t*>(T.g + 6 * nmax);
+    T.sc = reinterpret_cast<float*>(T.seg + nmax);
 
-    // Every lane reaches every barrier; a team without a ring (colour tail,
-    // or a body the damping pass skips) has nn = nt = 0.
-    uint32_t i = xf::colour_slot(begin, count, slabs, LANES);
-    uint4 m = make_uint4(0, 0, 0, 0);
-    float volume = 0.0f;
-    uint32_t energy = 0, rtype = 0;
-    float damp = 0.0f, nu = 0.0f, compliance = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
-    if (i != xf::kNoSlot) {
-        m = rmeta[i];
-        uint4 info = rinfo[i];
-        volume = __uint_as_float(info.z);
-        const XfBodyParams& bp = bodies[info.x];
-        energy = bp.energy;
-        rtype = bp.rtype;
-        damp = bp.damping;
-        nu = bp.poisson;
-        compliance = bp.compliance;
-        C0 = bp.yeoh[0];
-        C1 = bp.yeoh[1];
-        C2 = bp.yeoh[2];
+    // Phase 0. A lane's first node and tet are found by the ring's index, so
+    // only the node's position waits for another load. A team without a ring
+    // (colour tail, or a body the damping pass skips) loads the colour's first
+    // and has nn = nt = 0.
+    const uint32_t i = team_value<LANES>(xf::colour_slot(begin, count, slabs, LANES));
+    const uint32_t ic = i == xf::kNoSlot ? begin : i;
+    uint4 m = rmeta[ic];
+    const uint4 info = rinfo[ic];
+    uint2 nd = rnode[(size_t)ic * kRingFirst + min(lane, kRingFirst - 1u)];
+    // with 128 lanes the second wavefront takes the J halves of the tets
+    const uint32_t tl = LANES > 64u ? lane & 63u : lane, lf = min(tl, kRingFirst - 1u);
+    const float4* tf = rtet + (size_t)ic * 3 * kRingFirst;
+    float4 ta = tf[lf], tb = tf[kRingFirst + lf], td = tf[2 * kRingFirst + lf];
+    double4 x0 = X[nd.x];
+    const float volume = __uint_as_float(info.z);
+    const XfBodyParams& bp = bodies[team_value<LANES>(info.x)];
+    const uint32_t energy = bp.energy, rtype = bp.rtype;
+    const float compliance = bp.compliance, C0 = bp.yeoh[0], C1 = bp.yeoh[1], C2 = bp.yeoh[2];
+    float damp = bp.damping;
+    if (i == xf::kNoSlot) {
+        m = make_uint4(0, 0, 0, 0);
+    } else {
         if (POST) {
             bool on = rtype >= 2u && damp > 0.0f;
             if (on && rtype == 3u) {
@@ -181,179 +234,184 @@ __global__ __launch_bounds__(256) void xf_ring_colour(
             if (!on) m = make_uint4(0, 0, 0, 0);
         }
     }
-    const uint32_t nn = m.y, nt = m.w;
-    const uint32_t* nodes = rnodes + m.x;
-
-    // Phase 0: positions, inverse masses and incidence lists. The loads of a
-    // lane's first node, its first kIncLoads incidence entries and its first
-    // ring tet (for phase 1) are issued before any of them is used, at
-    // clamped in-range positions (a team without a ring reads entry 0), so
-    // the phase waits for two dependent round trips (node id, position), not
-    // one per loop iteration; rings beyond those counts loop as before.
-    const uint32_t ne = 4u * nt;
-    const uint32_t n0 = min(lane, nn > 0u ? nn - 1u : 0u);
-    const uint32_t g0 = nodes[n0];
-    const uint16_t b0 = rincb[m.x + n0];
-    uint16_t code[kIncLoads];
-#pragma unroll
-    for (uint32_t u = 0; u < kIncLoads; u++) code[u] = rinc[4 * m.z + min(lane + u * LANES, ne > 0u ? ne - 1u : 0u)];
-    const uint32_t k0 = min(lane, nt > 0u ? nt - 1u : 0u);
-    float4 ta = rtet[2 * (m.z + k0)], tb = rtet[2 * (m.z + k0) + 1];
-    const double4 x0 = X[g0];
-    if (lane < nn) {
-        T.x(0, lane) = x0.x;
-        T.x(1, lane) = x0.y;
-        T.x(2, lane) = x0.z;
-        T.ws[lane] = (float)x0.w;
-        T.incb[lane] = b0;
-    }
-    for (uint32_t n = lane + LANES; n < nn; n += LANES) {
-        double4 x = X[nodes[n]];
+    const uint32_t nn = team_value<LANES>(m.y), nt = team_value<LANES>(m.w);
+    auto node_of = [&](uint32_t n) {
+        return n < kRingFirst ? rnode[(size_t)ic * kRingFirst + n] : rnode_more[m.x + n - kRingFirst];
+    };
+    auto put_node = [&](uint32_t n, const uint2& d, const double4& x) {
         T.x(0, n) = x.x;
         T.x(1, n) = x.y;
         T.x(2, n) = x.z;
         T.ws[n] = (float)x.w;
-        T.incb[n] = rincb[m.x + n];
+        T.seg[n] = d.y;
+    };
+    if (lane < nn) {
+        if (LANES > kRingFirst && lane >= kRingFirst) {
+            nd = node_of(lane);
+            x0 = X[nd.x];
+        }
+        put_node(lane, nd, x0);
     }
-    if (lane == 0) T.incb[nn] = (uint16_t)ne;
-#pragma unroll
-    for (uint32_t u = 0; u < kIncLoads; u++) {
-        const uint32_t e = lane + u * LANES;
-        if (e < ne) {
-            T.inc[e] = code[u];
-            T.inv[code[u]] = (uint16_t)e;  // entry e of the lists holds (tet, corner) = code
+    for (uint32_t n = lane + LANES; n < nn; n += LANES) {
+        const uint2 d = node_of(n);
+        put_node(n, d, X[d.x]);
+    }
+    team_sync<LANES>();
+
+    // Phase 1: per ring tet.
+    for (uint32_t k = tl; k < nt; k += LANES > 64u ? 64u : LANES) {
+        if (k >= kRingFirst) {
+            const float4* t = rtet_more + 3 * (size_t)(m.z + k - kRingFirst);
+            ta = t[0];
+            tb = t[1];
+            td = t[2];
+        } else if (k != tl) {
+            ta = tf[k];
+            tb = tf[kRingFirst + k];
+            td = tf[2 * kRingFirst + k];
+        }
+        if constexpr (LANES > 64u) {
+            if (threadIdx.x & 64u) ring_tet<false, true>(T, ta, tb, td, k, nt);
+            else ring_tet<true, false>(T, ta, tb, td, k, nt);
+        } else {
+            ring_tet<true, true>(T, ta, tb, td, k, nt);
         }
     }
-    for (uint32_t e = lane + kIncLoads * LANES; e < ne; e += LANES) {
-        const uint16_t c = rinc[4 * m.z + e];
-        T.inc[e] = c;
-        T.inv[c] = (uint16_t)e;
-    }
-    __syncthreads();
+    team_sync<LANES>();
 
-    // Phase 1: per ring tet (the lane's first from the phase-0 loads).
-    for (uint32_t k = lane; k < nt; k += LANES) {
-        if (k != lane) {
-            ta = rtet[2 * (m.z + k)];
-            tb = rtet[2 * (m.z + k) + 1];
-        }
-        ring_tet(T, ta, tb, volume, k, tmax);
-    }
-    __syncthreads();
-
-    // Phase 2: ring-node gradients in ring-tet order (a node's entries are
-    // contiguous: no dependent index load); energy terms.
-    for (uint32_t n = lane; n < nn; n += LANES) {
-        const uint32_t e0 = T.incb[n], e1 = T.incb[n + 1];
-        const float* sl = T.c + 2 * tmax;
-        float a[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-        for (uint32_t e = e0; e < e1; e++)
-#pragma unroll
-            for (uint32_t r = 0; r < 6; r++) a[r] = a[r] + sl[6 * e + r];
-        for (uint32_t r = 0; r < 3; r++) {
-            T.gr(0, r, n) = a[r];
-            T.gr(1, r, n) = a[3 + r];
-        }
-    }
-    if (lane >= LANES - 2 && nt > 0) {
-        uint32_t q = lane - (LANES - 2);  // 0: I1 term, 1: J term
-        float u = 0.0f;
-#pragma unroll 4
-        for (uint32_t k = 0; k < nt; k++) u = u + T.c[2 * k + q];
-        T.sc[1 + q] = u;
-    }
-    __syncthreads();
-
-    // Phase 3: SolveSimplex (Geo.cpp:13-64): constants, gradient scaling and
-    // the per-node vectors of the damping terms.
-    float I1 = 0.0f, J = 0.0f, U0 = 0.0f, U1 = 0.0f, comp0 = 0.0f, comp1 = 0.0f;
-    bool two = energy != 8u;
-    bool damped_proj = !POST && damp > 0.0f && rtype < 2u;
+    // Phase 2. Items 0 to 5: the components of the ring's own vertex, which is
+    // a corner of every tet; 6 and 7: the energies; then node 1's components
+    // and so on. The first eight lanes take one of the long ones each, the
+    // others go on through the rest.
     if (nt > 0) {
-        I1 = T.sc[1];
-        J = T.sc[2];
+        const uint32_t items = 6u * nn + 2u;
+        for (uint32_t it = lane; it < items; it += lane < 8u ? items : LANES - 8u) {
+            const bool energy_sum = it == 6u || it == 7u;
+            const uint32_t q = it < 6u ? it : it - 2u, n = energy_sum ? 0u : q / 6u, r = energy_sum ? it - 6u : q - 6u * n;
+            const uint32_t e = T.seg[n], e0 = energy_sum ? 4u * nt : e & 0xFFFFu, e1 = energy_sum ? 5u * nt : e >> 16;
+            const float sum = ordered_sum(T.c + 6 * e0 + r, e1 - e0);
+            (energy_sum ? T.sc : T.g + n)[r * (energy_sum ? 1u : nmax)] = sum;
+        }
+    }
+    team_sync<LANES>();
+
+    // Phase 3: SolveSimplex (Geo.cpp:13-64): constants and gradient scaling.
+    float I1 = 0.0f, J = 0.0f, U0 = 0.0f, U1 = 0.0f, comp0 = 0.0f, comp1 = 0.0f;
+    float sc = 1.0f, s1 = 0.0f;
+    const float mu = bp.ring_mu, lambda = bp.ring_lambda, a = bp.ring_a;
+    const bool two = energy != 8u, skin = energy == 10u;
+    const bool damped_proj = !POST && damp > 0.0f && rtype < 2u;
+    if (nt > 0) {
+        I1 = T.sc[0];
+        J = T.sc[1];
         if (!two) {
-            float mu = 2.0f;
-            float lambda = mu / (1.0f - 2.0f * nu);
-            float a = 1.0f + mu / lambda;
             comp0 = compliance / volume;
             U0 = fmaxf(0.0000001f, (mu / 2.0f) * I1 + (lambda / 2.0f) * (J - a) * (J - a));
-            for (uint32_t n = lane; n < nn; n += LANES)
-                for (uint32_t r = 0; r < 3; r++)
-                    T.gr(0, r, n) = (mu / 2.0f) * T.gr(0, r, n) + (lambda / 2.0f) * 2.0f * (J - a) * T.gr(1, r, n);
         } else {
-            float mu = 1.0f / compliance;
-            float lambda = (2.0f * mu * nu) / (1.0f - 2.0f * nu);
-            float a = 1.0f + mu / lambda;
             comp0 = 1.0f / (mu * volume);
             comp1 = 1.0f / (lambda * volume);
             U0 = I1;
-            float sc = 1.0f;
-            bool skin = energy == 10u;
             if (skin) {
                 float IM = I1 - 3.0f;
                 U0 = fmaxf(0.0001f, C0 * IM + C1 * IM * IM + C2 * IM * IM * IM);
                 sc = C0 + 2.0f * C1 * IM + 3.0f * C2 * IM * IM;
             }
             U1 = (J - a) * (J - a);
-            float s1 = 2.0f * (J - a);
-            for (uint32_t n = lane; n < nn; n += LANES)
-                for (uint32_t r = 0; r < 3; r++) {
-                    if (skin) T.gr(0, r, n) = T.gr(0, r, n) * sc;
-                    T.gr(1, r, n) = T.gr(1, r, n) * s1;
-                }
+            s1 = 2.0f * (J - a);
         }
-        if (POST || damped_proj)
-            for (uint32_t n = lane; n < nn; n += LANES) {
-                if (POST) {
-                    double4 vd = V[nodes[n]];
-                    T.vr(0, n) = (float)vd.x;
-                    T.vr(1, n) = (float)vd.y;
-                    T.vr(2, n) = (float)vd.z;
-                } else {
-                    double4 o = O[nodes[n]];
-                    for (uint32_t r = 0; r < 3; r++) T.vr(r, n) = (float)(T.x(r, n) - (r == 0 ? o.x : r == 1 ? o.y : o.z));
+    }
+    // the scaled gradients of ring node n
+    auto scaled = [&](uint32_t n, float g0[3], float g1[3]) {
+        for (uint32_t r = 0; r < 3; r++) {
+            const float u = T.g[r * nmax + n], v = T.g[(3 + r) * nmax + n];
+            if (!two) {
+                g0[r] = (mu / 2.0f) * u + (lambda / 2.0f) * 2.0f * (J - a) * v;
+                g1[r] = v;
+            } else {
+                g0[r] = skin ? u * sc : u;
+                g1[r] = v * s1;
+            }
+        }
+    };
+
+    // The constraint sums, each in ring-node order (the sums of
+    // Xpbd.h:87-263):
+    //   wgg[0] = 1e-22 + sum w g0.g0     wgg[1] = 1e-22 + sum w g1.g0
+    //   wgg[2] = 1e-22 + sum w g1.g1     gV[0] = sum +-g0.v, gV[1] = sum +-g1.v
+    // with v = X - O (projection) or V (damping pass, where the two-constraint
+    // RayleighDamp sums -g.v). A lane per node forms the terms, into the
+    // entries, free after phase 2; then every lane adds them. Multiplying by 1 and negating are
+    // exact, so each sum rounds as the reference's does; the padding to sixteen
+    // terms adds 0 to sums that are never -0.
+    const bool with_v = POST || damped_proj;
+    const uint32_t n16 = (nn + 15u) & ~15u;
+    float g0[3] = {0.0f, 0.0f, 0.0f}, g1[3] = {0.0f, 0.0f, 0.0f};  // of the lane's first node
+    if (nt > 0)
+        for (uint32_t n = lane; n < n16; n += LANES) {
+            float h0[3], h1[3], t[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            if (n < nn) {
+                scaled(n, h0, h1);
+                if (n == lane)
+                    for (int r = 0; r < 3; r++) {
+                        g0[r] = h0[r];
+                        g1[r] = h1[r];
+                    }
+                const float w = T.ws[n];
+                t[0] = w * dot3(h0, h0);
+                t[1] = w * dot3(h1, h0);
+                t[2] = w * dot3(h1, h1);
+                if (with_v) {
+                    const uint32_t id = n == lane ? nd.x : node_of(n).x;
+                    float v[3];
+                    if (POST) {
+                        const double4 vd = V[id];
+                        v[0] = (float)vd.x;
+                        v[1] = (float)vd.y;
+                        v[2] = (float)vd.z;
+                    } else {
+                        const double4 o = O[id];
+                        v[0] = (float)(T.x(0, n) - o.x);
+                        v[1] = (float)(T.x(1, n) - o.y);
+                        v[2] = (float)(T.x(2, n) - o.z);
+                    }
+                    t[3] = dot3(h0, v);
+                    t[4] = dot3(h1, v);
+                    if (POST && two) {
+                        t[3] = -1.0f * t[3];
+                        t[4] = -1.0f * t[4];
+                    }
                 }
             }
-    }
-    __syncthreads();
-
-    // Phase 3b: the constraint sums, each in ring-node order (the sums of
-    // Xpbd.h:87-263):
-    //   sc[5] = 1e-22 + sum w g0.g0     sc[6] = 1e-22 + sum w g1.g0
-    //   sc[7] = 1e-22 + sum w g1.g1     sc[8] = sum +-g0.v, sc[9] = sum +-g1.v
-    // with v = X - O (projection) or V (damping pass, where the two-constraint
-    // RayleighDamp sums -g.v). Their terms are formed by all lanes (one
-    // (sum, node) pair at a time) into the per-tet area, free after phase 2;
-    // then one lane per sum adds them in order. Multiplying by 1 and negating
-    // are exact, so each sum rounds as the reference's does.
-    const uint32_t nsum = POST || damped_proj ? 5u : 3u;
-    float* terms = T.c;  // nsum x nn floats (nn <= 3 nt + 1 fits the 26 nt floats)
-    if (nt > 0)
-        for (uint32_t it = lane; it < nsum * nn; it += LANES) {
-            const uint32_t q = it / nn, n = it - q * nn;
-            const float* a = T.g + (q == 1 || q == 2 || q == 4 ? 3 * nmax : 0);
-            const float* b = q <= 1 ? T.g : q == 2 ? T.g + 3 * nmax : T.v;
-            float d = a[n] * b[n] + a[nmax + n] * b[nmax + n] + a[2 * nmax + n] * b[2 * nmax + n];
-            float term = q <= 2 ? T.ws[n] * d : d;
-            terms[it] = q >= 3 && POST && two ? -1.0f * term : term;
+            for (uint32_t q = 0; q < 3; q++) T.c[q * n16 + n] = t[q];
+            if (with_v)
+                for (uint32_t q = 3; q < 5; q++) T.c[q * n16 + n] = t[q];
         }
-    __syncthreads();
-    if (nt > 0 && lane < nsum) {
-        const float* tq = terms + lane * nn;
-        float acc = lane <= 2 ? 1.0e-22f : 0.0f;
-#pragma unroll 8
-        for (uint32_t n = 0; n < nn; n++) acc = acc + tq[n];
-        T.sc[5 + lane] = acc;
+    team_sync<LANES>();
+    float wgg[3] = {1.0e-22f, 1.0e-22f, 1.0e-22f}, gV[2] = {0.0f, 0.0f};
+    auto add4 = [&](uint32_t q, uint32_t n, float& acc) {
+        const float4 t = *reinterpret_cast<const float4*>(T.c + q * n16 + n);
+        acc = acc + t.x;
+        acc = acc + t.y;
+        acc = acc + t.z;
+        acc = acc + t.w;
+    };
+    if (nt > 0) {
+        for (uint32_t n = 0; n < n16; n += 16)
+#pragma unroll
+            for (uint32_t u = 0; u < 16; u += 4)
+#pragma unroll
+                for (uint32_t q = 0; q < 3; q++) add4(q, n + u, wgg[q]);
+        if (with_v)
+            for (uint32_t n = 0; n < n16; n += 16)
+#pragma unroll
+                for (uint32_t u = 0; u < 16; u += 4)
+#pragma unroll
+                    for (uint32_t q = 0; q < 2; q++) add4(3 + q, n + u, gV[q]);
     }
-    __syncthreads();
 
-    // Phase 3c: one lane forms the Lagrange multipliers.
-    if (lane == 0 && nt > 0) {
-        float l0 = 0.0f, l1 = 0.0f;
-        float wgg[3] = {T.sc[5], T.sc[6], T.sc[7]};
-        float gV[2] = {T.sc[8], T.sc[9]};
+    // The Lagrange multipliers, in every lane.
+    float l0 = 0.0f, l1 = 0.0f;
+    if (nt > 0) {
         if (!two && !POST) {
             // EnergyXpbdConstrain (Xpbd.h:87-120)
             float alpha = comp0 / (dt * dt);
@@ -428,41 +486,39 @@ __global__ __launch_bounds__(256) void xf_ring_colour(
             l0 = invDet * ((b0 * invA00) - (A1 * invA00) * (b1 * invA11));
             l1 = invDet * ((b1 * invA11) - (b0 * invA00) * (A1 * invA11));
         }
-        T.sc[3] = l0;
-        T.sc[4] = l1;
     }
-    __syncthreads();
 
     // Phase 4: node updates.
     if (nt > 0) {
-        float l0 = T.sc[3], l1 = T.sc[4];
         for (uint32_t n = lane; n < nn; n += LANES) {
-            float wn = T.ws[n];
+            const float wn = T.ws[n];
+            const uint32_t id = n == lane ? nd.x : node_of(n).x;
+            if (n != lane) scaled(n, g0, g1);
             if (!POST) {
                 double xr[3];
                 for (uint32_t r = 0; r < 3; r++) {
                     if (!two) {
                         float s = wn * l0;
-                        xr[r] = T.x(r, n) + (double)(s * T.gr(0, r, n));
+                        xr[r] = T.x(r, n) + (double)(s * g0[r]);
                     } else {
-                        float acc = 0.0f + l0 * T.gr(0, r, n);
-                        acc = acc + l1 * T.gr(1, r, n);
+                        float acc = 0.0f + l0 * g0[r];
+                        acc = acc + l1 * g1[r];
                         xr[r] = T.x(r, n) + (double)(wn * acc);
                     }
                 }
                 // x, y, z only: w (the inverse mass) stays as stored
-                double* xn = reinterpret_cast<double*>(X + nodes[n]);
+                double* xn = reinterpret_cast<double*>(X + id);
                 xn[0] = xr[0];
                 xn[1] = xr[1];
                 xn[2] = xr[2];
             } else {
-                double4 vd = V[nodes[n]];
+                double4 vd = V[id];
                 double* vr[3] = {&vd.x, &vd.y, &vd.z};
                 for (uint32_t r = 0; r < 3; r++) {
-                    if (!two) *vr[r] = *vr[r] + (double)((wn * l0) * T.gr(0, r, n));
-                    else *vr[r] = *vr[r] + (double)(wn * (l0 * T.gr(0, r, n) + l1 * T.gr(1, r, n)));
+                    if (!two) *vr[r] = *vr[r] + (double)((wn * l0) * g0[r]);
+                    else *vr[r] = *vr[r] + (double)(wn * (l0 * g0[r] + l1 * g1[r]));
                 }
-                V[nodes[n]] = vd;
+                V[id] = vd;
             }
         }
     }
@@ -474,22 +530,27 @@ __global__ __launch_bounds__(256) void xf_ring_colour(
 extern "C" size_t xf_ring_team_bytes(uint32_t nmax, uint32_t tmax) { return ring_team_bytes(nmax, tmax); }
 
 // One colour of the ring sweep (post = false) or of the ring damping pass
-// (post = true), `teams` rings per workgroup and `lanes` (16 or 32) lanes per
-// ring. clock: advanced by the first colour of a substep (pass it for that
+// (post = true), `teams` rings per workgroup and `lanes` (16, 32, 64 or 128)
+// lanes per ring. clock: advanced by the first colour of a substep (pass it for that
 // launch only); read by the damping pass for the amortized range.
 extern "C" hipError_t xf_launch_rings(hipStream_t s, bool post, uint32_t lanes, uint32_t teams, uint32_t slabs,
                                       uint32_t begin, uint32_t count, uint32_t nmax, uint32_t tmax,
-                                      const uint4* rmeta, const uint4* rinfo, const uint32_t* rnodes,
-                                      const uint16_t* rincb, const uint16_t* rinc, const float4* rtet, double4* X,
-                                      const double4* O, double4* V, const XfBodyParams* bodies, float dt,
-                                      float* clock) {
+                                      const uint4* rmeta, const uint4* rinfo, const uint2* rnode, const float4* rtet,
+                                      const uint2* rnode_more, const float4* rtet_more, double4* X, const double4* O,
+                                      double4* V, const XfBodyParams* bodies, float dt, float* clock) {
     if (count == 0) return hipSuccess;
-    if ((lanes != 16 && lanes != 32) || teams == 0 || teams * lanes > 256) return hipErrorInvalidValue;
+    if ((lanes != 16 && lanes != 32 && lanes != 64 && lanes != 128) || teams == 0 || teams * lanes > 256) return hipErrorInvalidValue;
     size_t lds = (size_t)teams * ring_team_bytes(nmax, tmax);
     dim3 grid(xf::colour_grid(count, teams, slabs)), block(teams * lanes);
-    auto k = post ? (lanes == 16 ? xf_ring_colour<true, 16> : xf_ring_colour<true, 32>)
-                  : (lanes == 16 ? xf_ring_colour<false, 16> : xf_ring_colour<false, 32>);
-    hipLaunchKernelGGL(k, grid, block, lds, s, begin, count, slabs, nmax, tmax, rmeta, rinfo, rnodes, rincb, rinc,
-                       rtet, X, O, V, bodies, dt, clock);
+    auto k = post ? (lanes == 16   ? xf_ring_colour<true, 16>
+                     : lanes == 32 ? xf_ring_colour<true, 32>
+                     : lanes == 64 ? xf_ring_colour<true, 64>
+                                   : xf_ring_colour<true, 128>)
+                  : (lanes == 16   ? xf_ring_colour<false, 16>
+                     : lanes == 32 ? xf_ring_colour<false, 32>
+                     : lanes == 64 ? xf_ring_colour<false, 64>
+                                   : xf_ring_colour<false, 128>);
+    hipLaunchKernelGGL(k, grid, block, lds, s, begin, count, slabs, nmax, tmax, rmeta, rinfo, rnode, rtet, rnode_more,
+                       rtet_more, X, O, V, bodies, dt, clock);
     return hipGetLastError();
 }

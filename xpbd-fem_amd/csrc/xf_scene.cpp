@@ -43,8 +43,8 @@ extern "C" hipError_t xf_launch_volume(hipStream_t s, uint32_t block, uint32_t s
                                        const float4* taux, double4* X, const XfBodyParams* bodies, float dt);
 extern "C" hipError_t xf_launch_rings(hipStream_t s, bool post, uint32_t lanes, uint32_t teams, uint32_t slabs,
                                       uint32_t begin, uint32_t count, uint32_t nmax, uint32_t tmax,
-                                      const uint4* rmeta, const uint4* rinfo, const uint32_t* rnodes,
-                                      const uint16_t* rincb, const uint16_t* rinc, const float4* rtet, double4* X,
+                                      const uint4* rmeta, const uint4* rinfo, const uint2* rnode, const float4* rtet,
+                                      const uint2* rnode_more, const float4* rtet_more, double4* X,
                                       const double4* O, double4* V, const XfBodyParams* bodies, float dt,
                                       float* clock);
 extern "C" size_t xf_ring_team_bytes(uint32_t nmax, uint32_t tmax);
@@ -332,10 +332,8 @@ struct xf_scene {
     std::vector<uint32_t> ring_colour_begin;
     uint4* rmeta = nullptr;
     uint4* rinfo = nullptr;  // body id, position in the body's ring order, ring volume bits, 0
-    uint32_t* rnodes = nullptr;
-    uint16_t* rincb = nullptr;  // per ring node: first entry of its incidence list (ring-local)
-    uint16_t* rinc = nullptr;   // per ring: (ring tet << 2 | corner) of each node, node-major, tets ascending
-    float4* rtet = nullptr;
+    uint2 *rnode = nullptr, *rnode_more = nullptr;  // node ids and incidence lists (xf_device.h)
+    float4 *rtet = nullptr, *rtet_more = nullptr;
     // sweep blocks (opts.sweep_blocks): per launch colour q, nslot blocks
     // (body-major, then block number) and nph phases; blk_rec + rec_off holds
     // per block nph (first schedule position, count) pairs, blk_node +
@@ -634,7 +632,12 @@ int UploadParams(xf_scene* s, float dt) {
         p.simultaneous = st.simultaneous ? 1u : 0u;
         p.n_rings = s->bodies[i].rings.n;
         p.compliance = st.compliance;
-        p.poisson = st.poissons_ratio;
+        // SolveSimplex's material (Geo.cpp:13-64): one constraint (Pixar) or two
+        p.ring_mu = st.energy == XF_ENERGY_CONTINUOUS_PIXAR ? 2.0f : 1.0f / st.compliance;
+        p.ring_lambda = st.energy == XF_ENERGY_CONTINUOUS_PIXAR
+                            ? p.ring_mu / (1.0f - 2.0f * st.poissons_ratio)
+                            : (2.0f * p.ring_mu * st.poissons_ratio) / (1.0f - 2.0f * st.poissons_ratio);
+        p.ring_a = 1.0f + p.ring_mu / p.ring_lambda;
         p.node_base = s->bodies[i].node_base;
         p.n_nodes = s->bodies[i].n;
         p.unlock = st.unlock_pins;
@@ -697,9 +700,8 @@ int UploadRings(xf_scene* s) {
     xf_ctx* ctx = s->ctx;
     std::vector<uint4> meta(s->R);
     std::vector<uint4> info(s->R);
-    std::vector<uint32_t> nodes;
-    std::vector<uint16_t> incb, inc;
-    std::vector<float4> rtet;
+    std::vector<uint2> node((size_t)s->R * kRingFirst, make_uint2(0u, 0u)), node_more;
+    std::vector<float4> tet((size_t)s->R * 3 * kRingFirst, make_float4(0.0f, 0.0f, 0.0f, 0.0f)), tet_more;
     s->ring_colour_begin.assign(s->rcol + 1, 0);
     std::vector<uint32_t> cursor(s->bodies.size(), 0);
     uint32_t pos = 0;
@@ -712,33 +714,44 @@ int UploadRings(xf_scene* s) {
             while (k < r.n && b.ring_colour[b.ring_order[k]] == c) {
                 uint32_t v = b.ring_order[k++];
                 uint32_t n0 = r.node_off[v], n1 = r.node_off[v + 1], t0 = r.tet_off[v], t1 = r.tet_off[v + 1];
-                meta[pos] = make_uint4((uint32_t)nodes.size(), n1 - n0, (uint32_t)(rtet.size() / 2), t1 - t0);
+                meta[pos] = make_uint4((uint32_t)node_more.size(), n1 - n0, (uint32_t)(tet_more.size() / 3), t1 - t0);
                 // ring volume: sum of V_t / 4 in ring-tet order (SolveRing, Geo.cpp:160-163)
                 float vsum = 0.0f;
                 for (uint32_t q = t0; q < t1; q++) vsum = vsum + 0.25f * b.ec.vol[r.tets[q]];
                 uint32_t vbits;
                 memcpy(&vbits, &vsum, 4);
                 info[pos] = make_uint4((uint32_t)bi, k - 1, vbits, 0u);
-                for (uint32_t q = n0; q < n1; q++) nodes.push_back(b.node_base + r.nodes[q]);
                 // incidence lists: for each ring node, its (tet, corner) slots in ring-tet order
-                std::vector<uint16_t> cnt(n1 - n0 + 1, 0);
-                for (uint32_t q = 4 * t0; q < 4 * t1; q++) cnt[r.idx[q] + 1]++;
-                for (uint32_t n = 0; n < n1 - n0; n++) cnt[n + 1] += cnt[n];
-                incb.insert(incb.end(), cnt.begin(), cnt.end() - 1);
-                size_t base = inc.size();
-                inc.resize(base + 4 * (size_t)(t1 - t0));
-                for (uint32_t q = 4 * t0; q < 4 * t1; q++) inc[base + cnt[r.idx[q]]++] = (uint16_t)(q - 4 * t0);
+                std::vector<uint32_t> at(n1 - n0 + 1, 0);
+                for (uint32_t q = 4 * t0; q < 4 * t1; q++) at[r.idx[q] + 1]++;
+                for (uint32_t n = 0; n < n1 - n0; n++) at[n + 1] += at[n];
+                for (uint32_t n = 0; n < n1 - n0; n++) {
+                    const uint2 d = make_uint2(b.node_base + r.nodes[n0 + n], at[n] | (at[n + 1] << 16));
+                    if (n < kRingFirst) node[(size_t)pos * kRingFirst + n] = d;
+                    else node_more.push_back(d);
+                }
                 for (uint32_t q = t0; q < t1; q++) {
                     uint32_t t = r.tets[q];
                     const float* qq = &b.ec.qq[3 * (size_t)t];
                     const float* qr = &b.ec.qr[3 * (size_t)t];
                     const uint8_t* li = &r.idx[4 * (size_t)q];
-                    uint32_t bits = (uint32_t)li[0] | ((uint32_t)li[1] << 8) | ((uint32_t)li[2] << 16) |
-                                    ((uint32_t)li[3] << 24);
-                    float bitsf;
-                    memcpy(&bitsf, &bits, 4);
-                    rtet.push_back(make_float4(qq[0], qq[1], qq[2], qr[0]));
-                    rtet.push_back(make_float4(qr[1], qr[2], b.ec.vol[t], bitsf));
+                    const uint32_t bits = (uint32_t)li[0] | ((uint32_t)li[1] << 8) | ((uint32_t)li[2] << 16) |
+                                          ((uint32_t)li[3] << 24);
+                    uint32_t e[4];
+                    for (int j = 0; j < 4; j++) e[j] = at[li[j]]++;
+                    const uint32_t words[3] = {bits, e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+                    float f[3];
+                    memcpy(f, words, sizeof(f));
+                    // the weights of CalculateElementEnergyAndGradients (Fem.cpp:941-973)
+                    const float vt = b.ec.vol[t], w = (vt / 4.0f) / vsum;
+                    const float4 rec[3] = {
+                        make_float4(qq[0], qq[1], qq[2], qr[0]),
+                        make_float4(qr[1], qr[2], w, (1.0f / vt) * (1.0f / 6.0f)),
+                        make_float4((w / vt) * (1.0f / 6.0f), f[0], f[1], f[2])};
+                    for (uint32_t j = 0; j < 3; j++) {
+                        if (q - t0 < kRingFirst) tet[((size_t)pos * 3 + j) * kRingFirst + q - t0] = rec[j];
+                        else tet_more.push_back(rec[j]);
+                    }
                 }
                 ++pos;
             }
@@ -746,31 +759,24 @@ int UploadRings(xf_scene* s) {
     }
     s->ring_colour_begin[s->rcol] = pos;
     if (pos != s->R) return Fail(ctx, XF_E_INVALID, "internal: ring schedule covers %u of %u rings", pos, s->R);
-    // One padding entry past the end of each list: the ring kernel loads a
-    // lane's first entries at clamped positions, which for a ring without
-    // nodes or tets (or a lane without a ring) is the ring's start offset.
-    nodes.push_back(0u);
-    incb.push_back(0u);
-    inc.insert(inc.end(), 4, (uint16_t)0u);
-    rtet.push_back(make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-    rtet.push_back(make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     rc = DevAlloc(ctx, &s->rmeta, s->R, &s->device_bytes);
     if (!rc) rc = DevAlloc(ctx, &s->rinfo, s->R, &s->device_bytes);
-    if (!rc) rc = DevAlloc(ctx, &s->rnodes, nodes.size(), &s->device_bytes);
-    if (!rc) rc = DevAlloc(ctx, &s->rincb, incb.size(), &s->device_bytes);
-    if (!rc) rc = DevAlloc(ctx, &s->rinc, inc.size(), &s->device_bytes);
-    if (!rc) rc = DevAlloc(ctx, &s->rtet, rtet.size(), &s->device_bytes);
+    if (!rc) rc = DevAlloc(ctx, &s->rnode, node.size(), &s->device_bytes);
+    if (!rc) rc = DevAlloc(ctx, &s->rtet, tet.size(), &s->device_bytes);
+    if (!rc) rc = DevAlloc(ctx, &s->rnode_more, node_more.size(), &s->device_bytes);
+    if (!rc) rc = DevAlloc(ctx, &s->rtet_more, tet_more.size(), &s->device_bytes);
     if (rc) return rc;
-    XF_HIP(ctx, hipMemcpyAsync(s->rincb, incb.data(), sizeof(uint16_t) * incb.size(), hipMemcpyHostToDevice,
-                               ctx->stream));
-    XF_HIP(ctx, hipMemcpyAsync(s->rinc, inc.data(), sizeof(uint16_t) * inc.size(), hipMemcpyHostToDevice,
-                               ctx->stream));
-    XF_HIP(ctx, hipMemcpyAsync(s->rmeta, meta.data(), sizeof(uint4) * s->R, hipMemcpyHostToDevice, ctx->stream));
-    XF_HIP(ctx, hipMemcpyAsync(s->rinfo, info.data(), sizeof(uint4) * s->R, hipMemcpyHostToDevice, ctx->stream));
-    XF_HIP(ctx, hipMemcpyAsync(s->rnodes, nodes.data(), sizeof(uint32_t) * nodes.size(), hipMemcpyHostToDevice,
-                               ctx->stream));
-    XF_HIP(ctx, hipMemcpyAsync(s->rtet, rtet.data(), sizeof(float4) * rtet.size(), hipMemcpyHostToDevice,
-                               ctx->stream));
+    hipStream_t st = ctx->stream;
+    XF_HIP(ctx, hipMemcpyAsync(s->rmeta, meta.data(), sizeof(uint4) * s->R, hipMemcpyHostToDevice, st));
+    XF_HIP(ctx, hipMemcpyAsync(s->rinfo, info.data(), sizeof(uint4) * s->R, hipMemcpyHostToDevice, st));
+    XF_HIP(ctx, hipMemcpyAsync(s->rnode, node.data(), sizeof(uint2) * node.size(), hipMemcpyHostToDevice, st));
+    XF_HIP(ctx, hipMemcpyAsync(s->rtet, tet.data(), sizeof(float4) * tet.size(), hipMemcpyHostToDevice, st));
+    if (!node_more.empty())
+        XF_HIP(ctx, hipMemcpyAsync(s->rnode_more, node_more.data(), sizeof(uint2) * node_more.size(),
+                                   hipMemcpyHostToDevice, st));
+    if (!tet_more.empty())
+        XF_HIP(ctx, hipMemcpyAsync(s->rtet_more, tet_more.data(), sizeof(float4) * tet_more.size(),
+                                   hipMemcpyHostToDevice, st));
     XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s->rings_dev = true;
     s->params_dirty = true;  // n_rings per body
@@ -838,11 +844,19 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
         // Geo3d::Substep with a vertex-ring energy: ring colours (the first
         // advances the clock), velocity, then GeoLinear3d::Damp's ring pass
         // and PBD tet pass (Geo.cpp:790-811), then the next prediction.
-        // lanes per ring: the option, else 32 when rings have more than 16
-        // tets (a tet per lane in the gather); rings per workgroup: the
-        // scene's workgroup size over the lanes, halved until the rings' LDS
-        // fits the budget
-        uint32_t lanes = s->opts.ring_lanes ? s->opts.ring_lanes : (s->rtmax > 16 ? 32u : 16u);
+        // Lanes per ring: the option, else by the rings of a colour: two
+        // wavefronts a ring while a compute unit has at most two rings, one
+        // while it has six, then half of one (of 16 tets, a quarter). Per
+        // colour of 24-tet rings with 128, 64 and 32 lanes: 376 rings
+        // (48x12x12 beam) 4.63, 4.85 and 5.13 us, 2,425 (96x24x24) 7.47, 6.91
+        // and 6.64, 11,000 (160x40x40) 20.8, 15.7 and 14.1. Rings per
+        // workgroup: the scene's workgroup size over the lanes, halved until
+        // the rings' LDS fits the budget.
+        uint32_t lanes = s->opts.ring_lanes;
+        if (lanes == 0) {
+            const uint64_t per_cu = (uint64_t)s->rcol * s->n_cu;
+            lanes = s->R <= 2 * per_cu ? 128u : s->R <= 6 * per_cu ? 64u : s->rtmax > 16 ? 32u : 16u;
+        }
         uint32_t rb = std::max(1u, block / lanes);
         while (rb > 1 && rb * xf_ring_team_bytes(s->rnmax, s->rtmax) > kRingLdsLimit) rb /= 2;
         int rc = node(0, false);
@@ -857,7 +871,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
                     XF_HIP(ctx, hipEventRecord(e0, st));
                 }
                 XF_HIP(ctx, xf_launch_rings(st, false, lanes, rb, slabs, begin, count, s->rnmax, s->rtmax, s->rmeta,
-                                            s->rinfo, s->rnodes, s->rincb, s->rinc, s->rtet, s->X, s->O, s->V,
+                                            s->rinfo, s->rnode, s->rtet, s->rnode_more, s->rtet_more, s->X, s->O, s->V,
                                             s->bp, dt, c == 0 ? s->clock : nullptr));
                 if (timer) {
                     XF_HIP(ctx, hipEventRecord(e1, st));
@@ -878,7 +892,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
                 for (uint32_t c = 0; c < s->rcol; c++) {
                     uint32_t begin = s->ring_colour_begin[c], count = s->ring_colour_begin[c + 1] - begin;
                     XF_HIP(ctx, xf_launch_rings(st, true, lanes, rb, slabs, begin, count, s->rnmax, s->rtmax, s->rmeta,
-                                                s->rinfo, s->rnodes, s->rincb, s->rinc, s->rtet, s->X, s->O, s->V,
+                                                s->rinfo, s->rnode, s->rtet, s->rnode_more, s->rtet_more, s->X, s->O, s->V,
                                                 s->bp, dt, s->clock));
                 }
             if (s->post & 2u)
@@ -1731,7 +1745,7 @@ XF_API void xf_scene_destroy(xf_scene* s) {
     DropAdjGraph(s);
     void* ptrs[] = {s->X,  s->O,     s->V,     s->tidx,  s->tg[0],         s->tg[1],  s->tg[2],
                     s->tg[3], s->taux, s->bp, s->clock, s->counter, s->colour_begin_d, s->arrive,
-                    s->barrier_err, s->tdmp, s->rmeta, s->rinfo, s->rnodes, s->rincb, s->rinc, s->rtet,
+                    s->barrier_err, s->tdmp, s->rmeta, s->rinfo, s->rnode, s->rtet, s->rnode_more, s->rtet_more,
                     s->blk_rec, s->blk_node, s->tloc, s->blk_fin, s->body_rec, s->body_loc, s->X2, s->tile_meta,
                     s->tile_rec, s->tile_node, s->tile_pos, s->tile_loc, s->tile_tg[0], s->tile_tg[1], s->tile_tg[2],
                     s->tile_tg[3], s->tile_taux, s->tout, s->kin_idx, s->kin_pos, s->manip};
