@@ -106,3 +106,32 @@ def test_slot_caps_and_layout(ctx, dims, lanes, cap):
     x, v = sc.get_state(0)
     sc.close()
     assert np.array_equal(x, a[0]) and np.array_equal(v, a[1])
+
+
+@pytest.mark.parametrize("dims,lanes", [((132, 36, 36), 128), ((156, 38, 41), 192), ((172, 41, 42), 256)])
+def test_workgroups_sharing_compute_units(ctx, dims, lanes):
+    """Two workgroups on some compute units with phases of two, three and four
+    wavefronts: the lanes that hold a phase's tets differ between them."""
+    wl = workloads.beam_yeoh(*dims)
+    wl = dict(wl, substeps=2)
+    a = run(ctx, wl, block_lanes=lanes, tet_lanes=1)
+    b = run(ctx, wl, block_lanes=64, tet_lanes=1, separate_finish=1)
+    assert 256 < a[3]["n_block_slots"] / 4 <= 512
+    assert all(np.array_equal(p, q) for p, q in zip(a[:3], b[:3]))
+
+
+@pytest.mark.parametrize("lanes,tet_lanes", [(64, 0), (64, 4), (128, 1), (256, 1)])
+@pytest.mark.parametrize("n", [3, 40])
+def test_bodies_of_mixed_energies(ctx, n, lanes, tet_lanes):
+    """Bodies of both energies side by side in the slots, per-tet material:
+    the energy term that a lane uses is that of its tet's body."""
+    wl = workloads.boxes_batch(n_bodies=n)
+    dt, out = float(wl["dt"]), []
+    for blocks in (True, False):
+        sc = workloads.make_batch_scene(ctx, wl, sweep_blocks=True, block_lanes=lanes, tet_lanes=tet_lanes,
+                                        launch_mode=xf.LAUNCH_BLOCKS if blocks else xf.LAUNCH_PER_COLOUR)
+        sc.step(3, dt)
+        sc.step(2, dt)
+        out.append([a for i in range(n) for a in sc.get_state(i)])
+        sc.close()
+    assert all(np.array_equal(p, q) for p, q in zip(*out))

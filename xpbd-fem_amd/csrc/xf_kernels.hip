@@ -157,6 +157,7 @@ __device__ __forceinline__ void write_nodes(uint32_t tid, uint32_t bs, uint32_t 
 // colour touches. All are staged in LDS with their O and finished from there
 // after the last phase. No other workgroup of the launch reads or writes
 // those nodes, and O is not read by the projection (FIN excludes DAMP).
+// ncu: compute units; pwaves: wavefronts of the largest phase, at most 4.
 // tend: the clock, read for the end time of the substep (advanced by an
 // earlier launch). fsingle: the scene has one body.
 // PF: register sets of element data, loaded PF - 1 phases ahead. One lane per
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
     const float4* __restrict__ tg1, const float4* __restrict__ tg2, const float4* __restrict__ tg3,
     const float4* __restrict__ taux, double4* __restrict__ X, double4* __restrict__ O,
     const XfBodyParams* __restrict__ bodies, float comp1_u, float a_u, float dt, float* __restrict__ clock,
-    const uint32_t* __restrict__ fextra, uint32_t fmax, const float* __restrict__ tend, uint32_t fsingle) {
+    const uint32_t* __restrict__ fextra, uint32_t fmax, const float* __restrict__ tend, uint32_t fsingle, uint32_t ncu, uint32_t pwaves) {
     static_assert(!(FIN && (DAMP || E == 30)), "the fused node phase needs a projection that leaves O unread");
     static_assert(!QUAD || (SIM && !DAMP && (E == 0 || E == 4 || E == 7)),
                   "quad lanes take the simultaneous MixedSel / YeohSkinFast projection without damping");
@@ -191,31 +192,61 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
     const uint32_t ftot = FIN ? nmax + fmax : 0u;
     double4* os = FIN ? reinterpret_cast<double4*>(xs.base + (NS / 16u) * ftot) : nullptr;
     uint32_t* fs = FIN ? reinterpret_cast<uint32_t*>(os + ftot) : nullptr;
-    // QUAD: four lanes per tet (block_tet_quad), bs / 4 tets
-    // at a time; else one lane per tet
-    const uint32_t lt = QUAD ? tid >> 2 : tid, per = QUAD ? bs >> 2 : bs;
+    // QUAD: four lanes per tet (block_tet_quad), bs / 4 tets at a time; else
+    // one lane per tet. Where few workgroups share a compute unit (NS 48), the
+    // lanes are turned by whole wavefronts so that their busy ones do not share
+    // a SIMD: of the g-th workgroup of a compute unit, wavefront k was seen on
+    // SIMD (k + g) mod 4, and its first tets go to the wavefront on SIMD pwaves
+    // * g mod 4, pwaves wavefronts having tets in the largest phase. 269
+    // workgroups of 128-tet phases on 256 compute units (64 mixed boxes): those
+    // that share one took 22.6 us where the others took 15; without sharing
+    // SIMDs a substep of four such launches takes 85 us, 107 before. 128x36x36
+    // beam, 128-tet slots: 1.95 ms per frame, 2.35 before.
+    constexpr bool TURN = NS == 48 && !QUAD;
+    const uint32_t turned = TURN ? (tid + 64u * (blockIdx.x / ncu) * (5u - pwaves)) % bs : tid;
+    const uint32_t lt = QUAD ? tid >> 2 : turned, per = QUAD ? bs >> 2 : bs;
     constexpr uint32_t PF = QUAD ? 3 : 2;
+    // AUX: the material (ax), and with it the body, of a lane's tet is loaded
+    // two phases ahead and the body's energy term one, so that neither is
+    // waited for behind the element data
+    auto at = [&](uint32_t j) { return min(r[2 * j] + lt, last); };
     auto load = [&](uint32_t j) {
-        return load_block_tet<AUX>(min(r[2 * j] + lt, last), tloc, tg0, tg1, tg2, tg3, taux);
+        return load_block_tet<false>(at(j), tloc, tg0, tg1, tg2, tg3, taux);
     };
-    auto solve = [&](const BlockTet& t, uint32_t i) {
-        if constexpr (QUAD) {
+    auto load_ax = [&](uint32_t j) { return AUX ? taux[at(j)] : make_float4(0.0f, 0.0f, 0.0f, 0.0f); };
+    struct Term {
+        float C[3];
+        uint32_t energy;
+    };
+    auto term = [&](const float4& ax) {
+        const XfBodyParams& bp = bodies[tet_material<AUX>(ax, comp1_u, a_u).body];
+        return Term{{bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]}, bp.energy};
+    };
+    auto solve = [&](const BlockTet& t, const Term& p, uint32_t i) {
+        if constexpr (DAMP) {
+            lds_tet_damped<E, SIM, AUX, NS>(t, tidx[i], xs, O, bodies, comp1_u, a_u, dt);
+        } else {
             const TetMaterial m = tet_material<AUX>(t.ax, comp1_u, a_u);
-            const XfBodyParams& bp = bodies[m.body];
-            const float C[3] = {bp.yeoh[0], bp.yeoh[1], bp.yeoh[2]};
-            block_tet_quad<NS>(t, tid & 3u, xs, E == 7 || (E == 0 && bp.energy == 7), C, m.comp1, m.a, dt);
-        } else block_tet<E, SIM, AUX, DAMP, NS>(t, i, xs, tidx, O, bodies, comp1_u, a_u, dt);
+            const bool yf = E == 7 || (E == 0 && p.energy == 7u);
+            if constexpr (QUAD) block_tet_quad<NS>(t, tid & 3u, xs, yf, p.C, m.comp1, m.a, dt);
+            else lds_tet<E, SIM, NS>(t, xs, yf, p.C, m.comp1, m.a, dt);
+        }
     };
     // each lane's first tet of the phase is t; with OVER, lanes go on to the
     // tets beyond the workgroup's lanes
-    auto phase = [&](uint32_t j, const BlockTet& t) {
+    auto phase = [&](uint32_t j, BlockTet& t, const float4& ax, const Term& p) {
         const uint32_t b = r[2 * j], cnt = r[2 * j + 1];
-        if (lt < cnt) solve(t, b + lt);
+        t.ax = ax;
+        if (lt < cnt) solve(t, p, b + lt);
         if constexpr (OVER)
-            for (uint32_t k = lt + per; k < cnt; k += per)
-                solve(load_block_tet<AUX>(b + k, tloc, tg0, tg1, tg2, tg3, taux), b + k);
+            for (uint32_t k = lt + per; k < cnt; k += per) {
+                const BlockTet o = load_block_tet<AUX>(b + k, tloc, tg0, tg1, tg2, tg3, taux);
+                solve(o, term(o.ax), b + k);
+            }
         __syncthreads();
     };
+    float4 ax = load_ax(0), ax_next = load_ax(min(1u, jl));
+    Term tm = term(ax);
     BlockTet t[PF];
     t[0] = load(0);
     if constexpr (FIN) {
@@ -240,8 +271,13 @@ __global__ __launch_bounds__(256) void xf_project_blocks(
     for (uint32_t j = 0; j < nph; j += PF) {
 #pragma unroll
         for (uint32_t k = 0; k < PF; k++) {
+            const Term tm_next = term(ax_next);
+            const float4 ax_after = load_ax(min(j + k + 2, jl));
             t[(k + PF - 1) % PF] = load(min(j + k + PF - 1, jl));
-            if (k == 0 || j + k < nph) phase(j + k, t[k]);
+            if (k == 0 || j + k < nph) phase(j + k, t[k], ax, tm);
+            ax = ax_next;
+            ax_next = ax_after;
+            tm = tm_next;
         }
     }
     if constexpr (FIN) {
@@ -707,7 +743,7 @@ extern "C" hipError_t xf_launch_project(hipStream_t s, int energy, bool sim, boo
 typedef void (*XfBlocksFn)(uint32_t, uint32_t, uint32_t, const uint32_t*, const uint32_t*, const uint2*,
                            const uint4*, const float4*, const float4*, const float4*, const float4*, const float4*,
                            double4*, double4*, const XfBodyParams*, float, float, float, float*, const uint32_t*,
-                           uint32_t, const float*, uint32_t);
+                           uint32_t, const float*, uint32_t, uint32_t, uint32_t);
 
 namespace {
 template <int E, bool OVER>
@@ -786,7 +822,8 @@ extern "C" size_t xf_block_fin_lds_bytes(uint32_t nmax, uint32_t fmax, uint32_t 
 // nodes and fmax extra nodes; tend: the clock, not advanced by this launch;
 // single_body: the scene has one body); not with damp or energy 30. quad:
 // four lanes per tet (simultaneous MixedSel / YeohSkinFast without damping,
-// energies 0, 4 and 7; anything else is hipErrorInvalidValue). lds_limit:
+// energies 0, 4 and 7; anything else is hipErrorInvalidValue). ncu: the
+// device's compute units. lds_limit:
 // the device's LDS bytes per workgroup (more than 64 KiB is granted to the
 // kernel with hipFuncAttributeMaxDynamicSharedMemorySize). wide: the launch
 // may keep 48 bytes per node in LDS (NodeLds) where a 48-byte kernel exists
@@ -800,7 +837,7 @@ extern "C" hipError_t XF_BLOCKS_LAUNCH(hipStream_t s, int energy, bool sim, bool
                                        const float4* taux, double4* X, double4* O,
                                        const XfBodyParams* bodies, float comp1_u, float a_u, float dt,
                                        float* clock, bool fin, const uint32_t* fextra, uint32_t fmax,
-                                       const float* tend, bool single_body, bool quad, size_t lds_limit,
+                                       const float* tend, bool single_body, bool quad, uint32_t ncu, size_t lds_limit,
                                        bool wide, uint32_t* nstride) {
     XfBlocksFn fn = nullptr;
     const bool over = pmax > (quad ? threads / 4 : threads);
@@ -828,7 +865,8 @@ extern "C" hipError_t XF_BLOCKS_LAUNCH(hipStream_t s, int energy, bool sim, bool
         default: return hipErrorInvalidValue;
     }
     size_t lds = fin ? xf_block_fin_lds_bytes(nmax, fmax, ns) : xf_block_lds_bytes(nmax, ns);
-    if (fn == nullptr || threads == 0 || threads > 256 || threads % 64 || nph == 0 || ntet == 0 || lds > lds_limit)
+    if (fn == nullptr || threads == 0 || threads > 256 || threads % 64 || nph == 0 || ntet == 0 || ncu == 0 ||
+        lds > lds_limit)
         return hipErrorInvalidValue;
     if (fin && (tend == nullptr || clock != nullptr || fextra == nullptr)) return hipErrorInvalidValue;
     if (nslot == 0) return hipSuccess;
@@ -839,7 +877,7 @@ extern "C" hipError_t XF_BLOCKS_LAUNCH(hipStream_t s, int energy, bool sim, bool
     }
     hipLaunchKernelGGL(fn, dim3(nslot), dim3(threads), lds, s, nph, nmax, ntet, rec, bnode, tloc, tidx, tg0, tg1,
                        tg2, tg3, taux, X, O, bodies, comp1_u, a_u, dt, clock, fextra, fmax, tend,
-                       single_body ? 1u : 0u);
+                       single_body ? 1u : 0u, ncu, std::min(4u, (pmax + 63u) / 64u));
     return hipGetLastError();
 }
 

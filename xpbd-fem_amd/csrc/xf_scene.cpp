@@ -58,7 +58,7 @@ extern "C" hipError_t xf_launch_blocks(hipStream_t s, int energy, bool sim, bool
                                        const float4* taux, double4* X, double4* O,
                                        const XfBodyParams* bodies, float comp1_u, float a_u, float dt,
                                        float* clock, bool fin, const uint32_t* fextra, uint32_t fmax,
-                                       const float* tend, bool single_body, bool quad, size_t lds_limit,
+                                       const float* tend, bool single_body, bool quad, uint32_t ncu, size_t lds_limit,
                                        bool wide, uint32_t* nstride);
 // the same launch with the kernels compiled with multiply-add contraction
 // (xf_blocks_contract.hip)
@@ -67,7 +67,7 @@ extern "C" hipError_t xf_launch_blocks_contract(
     uint32_t nmax, uint32_t ntet, uint32_t pmax, const uint32_t* rec, const uint32_t* bnode, const uint2* tloc,
     const uint4* tidx, const float4* tg0, const float4* tg1, const float4* tg2, const float4* tg3, const float4* taux,
     double4* X, double4* O, const XfBodyParams* bodies, float comp1_u, float a_u, float dt, float* clock, bool fin,
-    const uint32_t* fextra, uint32_t fmax, const float* tend, bool single_body, bool quad, size_t lds_limit,
+    const uint32_t* fextra, uint32_t fmax, const float* tend, bool single_body, bool quad, uint32_t ncu, size_t lds_limit,
     bool wide, uint32_t* nstride);
 extern "C" hipError_t xf_launch_predict(hipStream_t s, uint32_t n, const double4* X, double4* Xo, double4* O,
                                         const double4* V, const XfBodyParams* bodies);
@@ -1027,7 +1027,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
                                s->tg[0], s->tg[1], s->tg[2], s->tg[3], s->taux, s->X, s->O, s->bp, s->comp1_u,
                                s->a_u, dt, first ? s->clock : nullptr, fin && q == s->blk_last, s->blk_fin,
                                s->blk_fmax, s->clock, s->bodies.size() == 1, quad,
-                               s->lds_limit, s->blk_wide, &s->blk_nstride));
+                               (uint32_t)s->n_cu, s->lds_limit, s->blk_wide, &s->blk_nstride));
             first = false;
             if (timer) {
                 XF_HIP(ctx, hipEventRecord(e1, st));

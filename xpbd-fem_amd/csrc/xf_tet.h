@@ -725,19 +725,41 @@ __device__ __forceinline__ void stage_nodes(uint32_t tid, uint32_t bs, uint32_t 
     }
 }
 
-// One tet of a block phase: nodes from LDS, element data loaded, solved,
-// nodes written back to LDS.
-template <int E, bool SIM, bool AUX, bool DAMP, uint32_t NS>
-__device__ __forceinline__ void block_tet(const BlockTet& t, uint32_t i, NodeLds<NS> xs, const uint4* __restrict__ tidx,
-                                          const double4* __restrict__ O, const XfBodyParams* __restrict__ bodies,
-                                          float comp1_u, float a_u, float dt) {
+// One tet of a phase in LDS, one lane: nodes from LDS, projected, written back.
+// yf, C: the energy term and coefficients of its body.
+template <int E, bool SIM, uint32_t NS>
+__device__ __forceinline__ void lds_tet(const BlockTet& t, NodeLds<NS> xs, bool yf, const float C[3], float comp1,
+                                        float a, float dt) {
+    const uint32_t id[4] = {t.loc.x & 0xFFFFu, t.loc.x >> 16, t.loc.y & 0xFFFFu, t.loc.y >> 16};
+    double x[4][3];
+    float w[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double4 v = xs.get(id[k]);
+        x[k][0] = v.x;
+        x[k][1] = v.y;
+        x[k][2] = v.z;
+        w[k] = (float)v.w;
+    }
+    const float Qi[3][3] = {{t.q0.x, t.q0.y, t.q0.z}, {t.q0.w, t.q1.x, t.q1.y}, {t.q1.z, t.q1.w, t.q2.x}};
+    const float QQ[3] = {t.q2.y, t.q2.z, t.q2.w};
+    const float QR[3] = {t.q3.x, t.q3.y, t.q3.z};
+    solve_tet<E, SIM>(yf, C, x, w, Qi, QQ, QR, t.q3.w, comp1, a, dt);
+#pragma unroll
+    for (int k = 0; k < 4; k++) xs.put_xyz(id[k], x[k][0], x[k][1], x[k][2]);
+}
+
+// The same with damping inside the projection (reads O of the tet's nodes,
+// global ids gid, and the body's damping).
+template <int E, bool SIM, bool AUX, uint32_t NS>
+__device__ __forceinline__ void lds_tet_damped(const BlockTet& t, const uint4& gid, NodeLds<NS> xs,
+                                               const double4* __restrict__ O, const XfBodyParams* __restrict__ bodies,
+                                               float comp1_u, float a_u, float dt) {
     uint32_t ia = t.loc.x & 0xFFFFu, ib = t.loc.x >> 16, ic = t.loc.y & 0xFFFFu, id = t.loc.y >> 16;
     double4 na = xs.get(ia), nb = xs.get(ib), nc = xs.get(ic), nd = xs.get(id);
     double x[4][3] = {{na.x, na.y, na.z}, {nb.x, nb.y, nb.z}, {nc.x, nc.y, nc.z}, {nd.x, nd.y, nd.z}};
     float w[4] = {(float)na.w, (float)nb.w, (float)nc.w, (float)nd.w};
-    uint4 gid = make_uint4(0u, 0u, 0u, 0u);
-    if constexpr (DAMP) gid = tidx[i];
-    project_loaded<E, SIM, AUX, DAMP>(t.q0, t.q1, t.q2, t.q3, t.ax, gid, x, w, O, bodies, comp1_u, a_u, dt);
+    project_loaded<E, SIM, AUX, true>(t.q0, t.q1, t.q2, t.q3, t.ax, gid, x, w, O, bodies, comp1_u, a_u, dt);
     xs.put_xyz(ia, x[0][0], x[0][1], x[0][2]);
     xs.put_xyz(ib, x[1][0], x[1][1], x[1][2]);
     xs.put_xyz(ic, x[2][0], x[2][1], x[2][2]);

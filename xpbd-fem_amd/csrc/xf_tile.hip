@@ -44,24 +44,8 @@ __global__ __launch_bounds__(512) void xf_tile_span(XfTileArgs A, XfTileData D, 
                                    D.tg2, D.tg3, D.taux);
     };
     auto project = [&](const BlockTet& t) {
-        const uint32_t id[4] = {t.loc.x & 0xFFFFu, t.loc.x >> 16, t.loc.y & 0xFFFFu, t.loc.y >> 16};
-        double x[4][3];
-        float w[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const double4 v = xs.get(id[k]);
-            x[k][0] = v.x;
-            x[k][1] = v.y;
-            x[k][2] = v.z;
-            w[k] = (float)v.w;
-        }
         const TetMaterial mt = tet_material<AUX>(t.ax, A.comp1, A.a);
-        const float Qi[3][3] = {{t.q0.x, t.q0.y, t.q0.z}, {t.q0.w, t.q1.x, t.q1.y}, {t.q1.z, t.q1.w, t.q2.x}};
-        const float QQ[3] = {t.q2.y, t.q2.z, t.q2.w};
-        const float QR[3] = {t.q3.x, t.q3.y, t.q3.z};
-        solve_tet<E, SIM>(yf, C, x, w, Qi, QQ, QR, t.q3.w, mt.comp1, mt.a, A.dt);
-#pragma unroll
-        for (int k = 0; k < 4; k++) xs.put_xyz(id[k], x[k][0], x[k][1], x[k][2]);
+        lds_tet<E, SIM>(t, xs, yf, C, mt.comp1, mt.a, A.dt);
     };
     auto phase = [&](uint32_t j, const BlockTet& t) {
         const uint2 e = r[j];
@@ -74,7 +58,8 @@ __global__ __launch_bounds__(512) void xf_tile_span(XfTileArgs A, XfTileData D, 
             }
         } else {
             if (tid < e.y) project(t);
-            for (uint32_t k = tid + bs; k < e.y; k += bs) project(load_block_tet<AUX>(e.x + k, D.loc, D.tg0, D.tg1, D.tg2, D.tg3, D.taux));
+            for (uint32_t k = tid + bs; k < e.y; k += bs)
+                project(load_block_tet<AUX>(e.x + k, D.loc, D.tg0, D.tg1, D.tg2, D.tg3, D.taux));
         }
         __syncthreads();
     };
