@@ -104,17 +104,43 @@ __device__ __forceinline__ void reverse_one(uint32_t i, const uint4* __restrict_
     for (int n = 0; n < 4; n++) Xb[nid[n]] = make_double4(xb[n][0], xb[n][1], xb[n][2], 0.0);
 }
 
-// Reverse sweep of one colour: tets [begin, begin+count) of the sweep order.
+// reverse_one on four lanes (adjoint_quad): lane q holds component q of the
+// four nodes, lane 3 nothing.
 template <bool AUX, class R>
-__global__ __launch_bounds__(64) void xf_project_reverse(
-    uint32_t begin, uint32_t count, const uint4* __restrict__ tidx, const float4* __restrict__ tg0,
-    const float4* __restrict__ tg1, const float4* __restrict__ tg2, const float4* __restrict__ tg3,
-    const float4* __restrict__ taux, const double* __restrict__ tape, const double4* __restrict__ W,
-    double4* __restrict__ Xb, R* __restrict__ gacc, const XfBodyParams* __restrict__ bodies, float comp1_u,
-    float a_u, float dt) {
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < count)
-        reverse_one<AUX, R>(begin + k, tidx, tg0, tg1, tg2, tg3, taux, tape, W, Xb, gacc, bodies, comp1_u, a_u, dt);
+__device__ __forceinline__ void reverse_quad(uint32_t i, uint32_t q, const uint4* __restrict__ tidx,
+                                             const float4* __restrict__ tg0, const float4* __restrict__ tg1,
+                                             const float4* __restrict__ tg2, const float4* __restrict__ tg3,
+                                             const float4* __restrict__ taux, const double* __restrict__ tape,
+                                             const double4* __restrict__ W, double4* __restrict__ Xb,
+                                             R* __restrict__ gacc, const XfBodyParams* __restrict__ bodies,
+                                             float comp1_u, float a_u, float dt) {
+    const uint4 id = tidx[i];
+    BlockTet t;
+    t.q0 = tg0[i];
+    t.q1 = tg1[i];
+    t.q2 = tg2[i];
+    t.q3 = tg3[i];
+    t.ax = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (AUX) t.ax = taux[i];
+    t.loc = make_uint2(0u, 0u);
+    const uint32_t nid[4] = {id.x, id.y, id.z, id.w}, c = min(q, 2u);
+    const double* tp = tape + 12 * (size_t)i + c;
+    double x[4], xb[4];
+    float w[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+        x[n] = tp[3 * n];
+        w[n] = (float)W[nid[n]].w;
+        xb[n] = reinterpret_cast<const double*>(Xb + nid[n])[c];
+    }
+    const R g = gacc[i];
+    const TetMaterial m = tet_material<AUX>(t.ax, comp1_u, a_u);
+    const XfBodyParams& bp = bodies[m.body];
+    const R C[3] = {(R)bp.yeoh[0], (R)bp.yeoh[1], (R)bp.yeoh[2]};
+    const R gl = adjoint_quad<R>(quad_tet<R>(t), q, bp.energy == 7, C, x, w, (R)m.comp1, (R)m.a, (R)dt, xb);
+    if (q == 0u) gacc[i] = g + gl;
+#pragma unroll
+    for (int n = 0; n < 4; n++) reinterpret_cast<double*>(Xb + nid[n])[q] = q < 3u ? xb[n] : 0.0;
 }
 
 // Projection of the tet at schedule position i in element precision R
@@ -163,13 +189,20 @@ __device__ __forceinline__ void project_one(uint32_t i, const uint4* __restrict_
 // window replay (on X, into tape_rec); the rest take the reverse of colour
 // [vbegin, vbegin + vcount) of the later window (tape_rev, inverse masses
 // from W, adjoint Xb, gacc). The two touch disjoint arrays.
-template <bool AUX, class R>
+template <bool AUX, class R, bool QUAD>
 __global__ __launch_bounds__(64) void xf_adj_pair(
     uint32_t rbegin, uint32_t rcount, uint32_t rblocks, double4* __restrict__ X, double* __restrict__ tape_rec,
     uint32_t vbegin, uint32_t vcount, const double* __restrict__ tape_rev, const double4* __restrict__ W,
     double4* __restrict__ Xb, R* __restrict__ gacc, const uint4* __restrict__ tidx, const float4* __restrict__ tg0,
     const float4* __restrict__ tg1, const float4* __restrict__ tg2, const float4* __restrict__ tg3,
     const float4* __restrict__ taux, const XfBodyParams* __restrict__ bodies, float comp1_u, float a_u, float dt) {
+    if (QUAD && blockIdx.x >= rblocks) {
+        const uint32_t k = (blockIdx.x - rblocks) * 16u + (threadIdx.x >> 2);
+        if (k < vcount)
+            reverse_quad<AUX, R>(vbegin + k, threadIdx.x & 3u, tidx, tg0, tg1, tg2, tg3, taux, tape_rev, W, Xb, gacc,
+                                 bodies, comp1_u, a_u, dt);
+        return;
+    }
     if (blockIdx.x < rblocks) {
         uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
         if (k < rcount)
@@ -400,47 +433,22 @@ __global__ __launch_bounds__(256) void xf_copy2_d4(uint32_t n, double4* __restri
 
 // ------------------------------------------------------ launch wrappers
 
-// fp64: the FP64 element model (gacc then holds doubles).
-extern "C" hipError_t xf_launch_project_reverse(hipStream_t s, bool aux, bool fp64, uint32_t begin, uint32_t count,
-                                                const uint4* tidx, const float4* tg0, const float4* tg1,
-                                                const float4* tg2, const float4* tg3, const float4* taux,
-                                                const double* tape, const double4* W, double4* Xb, void* gacc,
-                                                const XfBodyParams* bodies, float comp1_u, float a_u, float dt) {
-    if (count == 0) return hipSuccess;
-    dim3 grid((count + 63) / 64), block(64);
-    float* g32 = static_cast<float*>(gacc);
-    double* g64 = static_cast<double*>(gacc);
-    if (fp64 && aux)
-        hipLaunchKernelGGL((xf_project_reverse<true, double>), grid, block, 0, s, begin, count, tidx, tg0, tg1, tg2,
-                           tg3, taux, tape, W, Xb, g64, bodies, comp1_u, a_u, dt);
-    else if (fp64)
-        hipLaunchKernelGGL((xf_project_reverse<false, double>), grid, block, 0, s, begin, count, tidx, tg0, tg1, tg2,
-                           tg3, taux, tape, W, Xb, g64, bodies, comp1_u, a_u, dt);
-    else if (aux)
-        hipLaunchKernelGGL((xf_project_reverse<true, float>), grid, block, 0, s, begin, count, tidx, tg0, tg1, tg2,
-                           tg3, taux, tape, W, Xb, g32, bodies, comp1_u, a_u, dt);
-    else
-        hipLaunchKernelGGL((xf_project_reverse<false, float>), grid, block, 0, s, begin, count, tidx, tg0, tg1, tg2,
-                           tg3, taux, tape, W, Xb, g32, bodies, comp1_u, a_u, dt);
-    return hipGetLastError();
-}
-
 // Record of colour [rbegin, rbegin + rcount) and reverse of colour
 // [vbegin, vbegin + vcount) in one launch (xf_adj_pair); either count may
-// be 0.
-extern "C" hipError_t xf_launch_adj_pair(hipStream_t s, bool aux, bool fp64, uint32_t rbegin, uint32_t rcount,
+// be 0. fp64: the FP64 element model (gacc then holds doubles). quad: four lanes per tet of the reverse.
+extern "C" hipError_t xf_launch_adj_pair(hipStream_t s, bool aux, bool fp64, bool quad, uint32_t rbegin, uint32_t rcount,
                                          double4* X, double* tape_rec, uint32_t vbegin, uint32_t vcount,
                                          const double* tape_rev, const double4* W, double4* Xb, void* gacc,
                                          const uint4* tidx, const float4* tg0, const float4* tg1, const float4* tg2,
                                          const float4* tg3, const float4* taux, const XfBodyParams* bodies,
                                          float comp1_u, float a_u, float dt) {
-    const uint32_t rblocks = (rcount + 63) / 64, vblocks = (vcount + 63) / 64;
+    const uint32_t rblocks = (rcount + 63) / 64, vblocks = quad ? (vcount + 15) / 16 : (vcount + 63) / 64;
     if (rblocks + vblocks == 0) return hipSuccess;
     dim3 grid(rblocks + vblocks), block(64);
 #define XF_PAIR(A, R, G)                                                                                         \
-    hipLaunchKernelGGL((xf_adj_pair<A, R>), grid, block, 0, s, rbegin, rcount, rblocks, X, tape_rec, vbegin,   \
-                       vcount, tape_rev, W, Xb, static_cast<R*>(G), tidx, tg0, tg1, tg2, tg3, taux, bodies, comp1_u, \
-                       a_u, dt)
+    hipLaunchKernelGGL((quad ? xf_adj_pair<A, R, true> : xf_adj_pair<A, R, false>), grid, block, 0, s, rbegin,   \
+                       rcount, rblocks, X, tape_rec, vbegin, vcount, tape_rev, W, Xb, static_cast<R*>(G), tidx, tg0, \
+                       tg1, tg2, tg3, taux, bodies, comp1_u, a_u, dt)
     if (fp64) {
         if (aux) XF_PAIR(true, double, gacc);
         else XF_PAIR(false, double, gacc);
