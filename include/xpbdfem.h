@@ -185,12 +185,25 @@ enum {
                                  a workgroup per tile of nodes (energies 3 to 7 and above 12, up to 1,024
                                  nodes per compute unit, no damping or volume passes, no kinematic nodes,
                                  no manipulator), or one launch per step call, with a workgroup per body
-                                 (bodies of up to 2,560 nodes on gfx950; passes included). Same results. */
+                                 (bodies of up to 2,560 nodes on gfx950; passes included). Same results;
+                                 xf_scene_get_route tells which, xf_scene_set_colour_launches keeps one
+                                 launch per colour. */
     XF_LAUNCH_PERSISTENT = 1, /* one cooperative launch per step call, grid barriers between phases */
     XF_LAUNCH_BLOCKS = 2      /* needs sweep_blocks: one projection launch per block launch colour
-                                 (at most 4 per substep), each workgroup of block_size threads
-                                 sweeping one block through its phases with the block's nodes in
-                                 LDS; other passes run per colour */
+                                 (at most 4 per substep), each workgroup sweeping one block through
+                                 its phases with the block's nodes in LDS (threads: see block_size);
+                                 other passes run per colour */
+};
+
+/* How the sweeps of a step call were launched (xf_scene_get_route). */
+enum {
+    XF_ROUTE_NONE = 0,       /* no step call yet */
+    XF_ROUTE_COLOURS = 1,    /* a launch per colour */
+    XF_ROUTE_TILES = 2,      /* a launch for several colours, a workgroup per tile of nodes */
+    XF_ROUTE_BODIES = 3,     /* a launch per step call, a workgroup per body */
+    XF_ROUTE_PERSISTENT = 4, /* XF_LAUNCH_PERSISTENT */
+    XF_ROUTE_BLOCKS = 5,     /* XF_LAUNCH_BLOCKS */
+    XF_ROUTE_RINGS = 6       /* a launch per ring colour */
 };
 
 typedef struct xf_scene_opts {
@@ -319,6 +332,15 @@ XF_API int xf_scene_set_tet_mu(xf_scene* scene, uint32_t body, const float* tet_
  * Returns when the work is enqueued; xf_scene_sync waits for it. */
 XF_API int xf_scene_step(xf_scene* scene, uint32_t substeps, float dt);
 XF_API int xf_scene_sync(xf_scene* scene);
+/* The route of the last step call (XF_ROUTE_*; also of xf_scene_profile and
+ * the forward of xf_scene_adjoint) and the most threads of a workgroup of its
+ * sweep launches (0 before the first one); either nullable. */
+XF_API int xf_scene_get_route(const xf_scene* scene, uint32_t* route, uint32_t* threads);
+/* 1: step calls in XF_LAUNCH_PER_COLOUR take one launch per colour whatever is
+ * estimated faster (to compare the routes, which give the same results); 0
+ * (default): the estimate decides. Any time; not part of the state that the
+ * autotuner chooses. */
+XF_API int xf_scene_set_colour_launches(xf_scene* scene, uint32_t on);
 
 /* Node state of one body: x[3*n], v[3*n] (either nullable). The state is
  * FP64 like the reference's dvec3 X, V (Geo.h:61-64). Synchronous. */

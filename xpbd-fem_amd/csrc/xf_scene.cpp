@@ -404,6 +404,8 @@ struct xf_scene {
     std::vector<XfBodyParams> h_bp;  // body table staging (sized at finalize)
     bool material_dirty = true, params_dirty = true;
     bool aux = false;
+    bool colours_only = false;  // xf_scene_set_colour_launches
+    uint32_t route = XF_ROUTE_NONE, route_threads = 0;  // of the last step call
     uint32_t vpasses = 0;  // max volume passes over bodies (taux is then always present)
     bool dproj = false;    // some body damps inside the projection (Rayleigh Paper / Limit)
     uint32_t post = 0;     // damping passes after the velocity update: bit 0 Rayleigh post, bit 1 PBD
@@ -427,6 +429,7 @@ struct xf_scene {
     bool graph_sim = false, graph_aux = false, graph_dproj = false;
     uint32_t graph_vpasses = 0, graph_post = 0, graph_nkin = 0;
     bool graph_manip = false;
+    uint32_t graph_route = XF_ROUTE_NONE, graph_threads = 0;
     // graph of the adjoint's reverse pass (window replays and reverse
     // sweeps), kept for the call shape in adj_key (sizes, loss substeps,
     // precision, scene constants baked into the launches, buffer addresses)
@@ -543,7 +546,7 @@ void ComputeMaterial(xf_scene* s) {
 // the scene has the plan (BuildTiles), and the sweep is followed by nothing
 // but the node phase.
 bool TileSweeps(const xf_scene* s, int energy) {
-    return s->ntile != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR &&
+    return s->ntile != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR && !s->colours_only &&
            (energy == 0 || (energy >= 3 && energy <= 7)) && s->vpasses == 0 && s->post == 0 && !s->dproj &&
            s->nkin == 0 && !s->manip_on;
 }
@@ -553,7 +556,7 @@ bool TileSweeps(const xf_scene* s, int energy) {
 // energy constrains tets with the terms of energies 3..7, nothing outside a
 // body moves its nodes, and tile launches are not the shorter way.
 bool WholeCalls(const xf_scene* s, int energy) {
-    return s->body_threads != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR &&
+    return s->body_threads != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR && !s->colours_only &&
            (energy == 0 || (energy >= 3 && energy <= 7)) && s->nkin == 0 && !s->manip_on && !TileSweeps(s, energy);
 }
 
@@ -817,6 +820,10 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     uint32_t block = s->opts.block_size ? s->opts.block_size : 64;
     uint32_t slabs = s->opts.xcd_slabs;
     double4* start = s->X;  // where the first prediction goes
+    auto took = [&](uint32_t route, uint32_t threads) {
+        s->route = route;
+        s->route_threads = threads;
+    };
     auto node = [&](int kind, bool predict_next) -> int {
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (timer) {
@@ -854,6 +861,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
         }
         uint32_t rb = std::max(1u, block / lanes);
         while (rb > 1 && rb * xf_ring_team_bytes(s->rnmax, s->rtmax) > kRingLdsLimit) rb /= 2;
+        took(XF_ROUTE_RINGS, rb * lanes);
         int rc = node(0, false);
         if (rc) return rc;
         for (uint32_t k = 0; k < substeps; k++) {
@@ -915,6 +923,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
             XF_HIP(ctx, hipEventCreate(&e1));
         }
         s->ran_persistent = true;
+        took(XF_ROUTE_PERSISTENT, 256);
         XF_HIP(ctx, hipMemsetAsync(s->arrive, 0, sizeof(uint32_t), st));
         if (timer) XF_HIP(ctx, hipEventRecord(e0, st));
         XF_HIP(ctx, xf_launch_frame(st, energy, sim, s->aux, s->dproj, blocks, substeps, s->ncol, s->vpasses, s->post,
@@ -929,6 +938,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
         return XF_OK;
     }
     if (WholeCalls(s, energy)) {
+        took(XF_ROUTE_BODIES, s->body_threads);
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (timer) {
             XF_HIP(ctx, hipEventCreate(&e0));
@@ -951,6 +961,9 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     if (TileSweeps(s, energy)) {
         // the launches alternate between two node arrays and end in X
         double4* cur = (substeps * s->tile_spans.size()) % 2 ? s->X2 : s->X;
+        took(XF_ROUTE_TILES, 0);
+        for (const xf_scene::TileSpan& sp : s->tile_spans)
+            s->route_threads = std::max(s->route_threads, xf_tile_threads(sp.lanes));
         start = cur;
         int rc = node(0, false);
         if (rc) return rc;
@@ -996,6 +1009,7 @@ int Enqueue(xf_scene* s, uint32_t substeps, float dt, int energy, bool sim, Laun
     if (blocks && (!quad || s->opts.tet_lanes == 0))
         blk_threads = quad || s->blk_wide ? 256u : std::min(256u, (std::max(s->blk_pmax, 1u) + 63) / 64 * 64);
     s->blk_tet_lanes = quad ? 4u : 1u;
+    took(blocks ? XF_ROUTE_BLOCKS : XF_ROUTE_COLOURS, blocks ? blk_threads : block);
     // the node phase rides on the substep's last block launch when nothing
     // runs between the sweep and the velocity update (no volume passes), the
     // velocities need not be stored (no damping passes, not the call's last
@@ -2145,6 +2159,22 @@ XF_API int xf_scene_info_get(const xf_scene* s, xf_scene_info* info) {
     return XF_OK;
 }
 
+XF_API int xf_scene_get_route(const xf_scene* s, uint32_t* route, uint32_t* threads) {
+    if (!s) return XF_E_INVALID;
+    if (route) *route = s->route;
+    if (threads) *threads = s->route_threads;
+    return XF_OK;
+}
+
+XF_API int xf_scene_set_colour_launches(xf_scene* s, uint32_t on) {
+    if (!s) return XF_E_INVALID;
+    if (on > 1) return Fail(s->ctx, XF_E_INVALID, "colour_launches must be 0 or 1");
+    if (s->colours_only == (on != 0)) return XF_OK;
+    DropGraph(s);
+    s->colours_only = on != 0;
+    return XF_OK;
+}
+
 XF_API int xf_scene_set_settings(xf_scene* s, uint32_t body, const xf_settings* st) {
     if (!s || !st) return XF_E_INVALID;
     if (body >= s->bodies.size()) return Fail(s->ctx, XF_E_INVALID, "body %u out of range", body);
@@ -2213,7 +2243,11 @@ XF_API int xf_scene_step(xf_scene* s, uint32_t substeps, float dt) {
             s->graph_post = s->post;
             s->graph_nkin = s->nkin;
             s->graph_manip = s->manip_on;
+            s->graph_route = s->route;
+            s->graph_threads = s->route_threads;
         }
+        s->route = s->graph_route;
+        s->route_threads = s->graph_threads;
         XF_HIP(ctx, hipGraphLaunch(s->graph_exec, ctx->stream));
     }
     if (rc) return rc;
@@ -2510,6 +2544,7 @@ XF_API int xf_scene_autotune(xf_scene* s, uint32_t substeps, float dt, uint32_t 
     if (he == hipSuccess) he = hipEventCreate(&e1);
     float time_keep = s->time_host;
     uint32_t tick_keep = s->tick_host;
+    const uint32_t route_keep = s->route, threads_keep = s->route_threads;
     uint32_t packed = cap_keep;  // the slot cap the uploaded tables hold
     auto repack = [&](uint32_t cap) -> int {
         if (cap == packed) return XF_OK;
@@ -2552,6 +2587,8 @@ XF_API int xf_scene_autotune(xf_scene* s, uint32_t substeps, float dt, uint32_t 
     for (void* p : {(void*)sx, (void*)so, (void*)sv, (void*)sc}) (void)hipFree(p);
     s->time_host = time_keep;
     s->tick_host = tick_keep;
+    s->route = route_keep;
+    s->route_threads = threads_keep;
     s->opts = keep;
     s->opts.launch_mode = best_c.mode;
     s->opts.tet_lanes = best_c.lanes;

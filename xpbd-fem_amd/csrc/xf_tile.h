@@ -58,6 +58,10 @@ constexpr uint32_t kTileThreads = 512;     // most lanes
 constexpr uint32_t kTileQuadTets = 64;     // a phase of up to so many tets runs on quads
 constexpr uint32_t kTileNodeBytes = 48;    // LDS per node
 
+// Threads of a launch whose tiles have at most `lanes` tets in a colour and
+// own at most as many nodes.
+inline uint32_t xf_tile_threads(uint32_t lanes) { return lanes <= 256 ? 256u : kTileThreads; }
+
 struct XfTileArgs {
     uint32_t nph, nent;
     uint32_t end;  // 0: store the nodes; 1: end the substep and predict the next; 2: end it and store velocities

@@ -161,7 +161,7 @@ extern "C" hipError_t xf_launch_tiles(hipStream_t s, int energy, bool sim, bool 
         default: break;
     }
     const size_t lds = (size_t)nmax * kTileNodeBytes;
-    const uint32_t threads = lanes <= 256 ? 256u : kTileThreads;
+    const uint32_t threads = xf_tile_threads(lanes);
     if (fn == nullptr || lds > lds_limit || args->nph == 0 || args->nent == 0 ||
         ((aux || energy == 0) && d->taux == nullptr))
         return hipErrorInvalidValue;

@@ -23,6 +23,7 @@ COLLIDE_GROUND, COLLIDE_SPHERE = 1, 2
 RAYLEIGH_PAPER, RAYLEIGH_LIMIT, RAYLEIGH_POST, RAYLEIGH_POST_AMORTIZED = 0, 1, 2, 3
 COLOUR_NATURAL, COLOUR_MINSTD = 0, 1
 LAUNCH_PER_COLOUR, LAUNCH_PERSISTENT, LAUNCH_BLOCKS = 0, 1, 2
+ROUTE_NONE, ROUTE_COLOURS, ROUTE_TILES, ROUTE_BODIES, ROUTE_PERSISTENT, ROUTE_BLOCKS, ROUTE_RINGS = range(7)
 SKIN_YEOH = (0.1095, 14.95, 4.595)  # Fem.cpp:526
 
 _f32p = np.ctypeslib.ndpointer(dtype=np.float32, flags="C_CONTIGUOUS")
@@ -132,6 +133,8 @@ def lib():
         "xf_scene_info_get": ([vp, C.POINTER(SceneInfo)], C.c_int),
         "xf_scene_set_settings": ([vp, C.c_uint32, C.POINTER(Settings)], C.c_int),
         "xf_scene_set_tet_mu": ([vp, C.c_uint32, _f32p], C.c_int),
+        "xf_scene_get_route": ([vp, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)], C.c_int),
+        "xf_scene_set_colour_launches": ([vp, C.c_uint32], C.c_int),
         "xf_scene_step": ([vp, C.c_uint32, C.c_float], C.c_int),
         "xf_scene_sync": ([vp], C.c_int),
         "xf_scene_get_state": ([vp, C.c_uint32, vp, vp], C.c_int),
@@ -191,7 +194,8 @@ def exported_symbols():
         "xf_mesh_colour", "xf_scene_autotune", "xf_scene_adjoint", "xf_mesh_tet_block_colours",
         "xf_scene_get_tick", "xf_scene_set_tick", "xf_mesh_read_tetgen", "xf_mesh_tets_from_stream", "xf_mesh_error",
         "xf_mesh_rings", "xf_mesh_sweep_blocks", "xf_scene_time_steps", "xf_scene_adjoint_noalloc",
-        "xf_scene_set_kinematic", "xf_scene_set_manip", "xf_scene_adjoint_fp64",
+        "xf_scene_set_kinematic", "xf_scene_set_manip", "xf_scene_adjoint_fp64", "xf_scene_get_route",
+        "xf_scene_set_colour_launches",
     ]
 
 
@@ -556,6 +560,18 @@ class Scene:
         t = np.ascontiguousarray(target, np.float32)
         self.ctx.check(lib().xf_scene_set_manip(self.h, body, 0xFFFFFFFF if node is None else node, t),
                        "xf_scene_set_manip")
+
+    def route(self):
+        """(route, threads) of the last step call: ROUTE_*, and the most
+        threads of a workgroup of its sweep launches."""
+        r, t = C.c_uint32(), C.c_uint32()
+        self.ctx.check(lib().xf_scene_get_route(self.h, C.byref(r), C.byref(t)), "xf_scene_get_route")
+        return r.value, t.value
+
+    def set_colour_launches(self, on=True):
+        """Step calls in LAUNCH_PER_COLOUR take one launch per colour, also
+        where another route is estimated faster (same results)."""
+        self.ctx.check(lib().xf_scene_set_colour_launches(self.h, int(on)), "xf_scene_set_colour_launches")
 
     def time_steps(self, calls, substeps, dt):
         """Device ms of `calls` step calls between two HIP events on the
