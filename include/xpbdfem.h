@@ -187,7 +187,10 @@ enum {
                                  no manipulator), or one launch per step call, with a workgroup per body
                                  (bodies of up to 2,560 nodes on gfx950; passes included). Same results;
                                  xf_scene_get_route tells which, xf_scene_set_colour_launches keeps one
-                                 launch per colour. */
+                                 launch per colour. The tables of the tiles (76 to 92 bytes each time a
+                                 tile projects a tet, 2 to 4 times a tet on large meshes, up to 20 on
+                                 small ones; 32 a node) are made by the first step call that may use
+                                 them; without memory for them the other routes stay. */
     XF_LAUNCH_PERSISTENT = 1, /* one cooperative launch per step call, grid barriers between phases */
     XF_LAUNCH_BLOCKS = 2      /* needs sweep_blocks: one projection launch per block launch colour
                                  (at most 4 per substep), each workgroup sweeping one block through

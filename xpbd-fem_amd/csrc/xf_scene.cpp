@@ -367,7 +367,11 @@ struct xf_scene {
     uint32_t blk_cap = 0;  // opts.block_lanes, or the automatic slot cap
     uint32_t* blk_fin = nullptr;
     uint2* tloc = nullptr;
-    // tile launches (xf_tile.hip; BuildTiles): ntile 0 where the scene has none
+    // tile launches (xf_tile.hip): planned by the first step call that could
+    // use them (PlanSweeps), ntile 0 where none did or another route is
+    // estimated faster. tile_taux is there when taux is.
+    bool tiles_tried = false;
+    uint64_t tile_bytes = 0;
     struct TileSpan {
         uint32_t nph, nmax;  // colours; most nodes of a tile
         uint32_t lanes;      // most tets of a tile in one colour, or own nodes
@@ -542,14 +546,16 @@ void ComputeMaterial(xf_scene* s) {
     }
 }
 
-// Whether per-colour step calls run as tile launches, several colours each:
-// the scene has the plan (BuildTiles), and the sweep is followed by nothing
-// but the node phase.
-bool TileSweeps(const xf_scene* s, int energy) {
-    return s->ntile != 0 && s->opts.launch_mode == XF_LAUNCH_PER_COLOUR && !s->colours_only &&
+// Whether per-colour step calls may run as tile launches, several colours
+// each: nothing but the node phase follows the sweep.
+bool MayTile(const xf_scene* s, int energy) {
+    return s->opts.launch_mode == XF_LAUNCH_PER_COLOUR && !s->colours_only &&
            (energy == 0 || (energy >= 3 && energy <= 7)) && s->vpasses == 0 && s->post == 0 && !s->dproj &&
            s->nkin == 0 && !s->manip_on;
 }
+
+// Whether they do: the scene has the plan (PlanSweeps).
+bool TileSweeps(const xf_scene* s, int energy) { return s->ntile != 0 && MayTile(s, energy); }
 
 // Whether per-colour step calls run as one launch per call, a workgroup per
 // body (xf_launch_body): the scene has the tables (BuildBodyTables), the
@@ -571,6 +577,54 @@ bool NeedSlots(xf_scene* s) {
            xf_body_needs_slots(energy, st.simultaneous != 0, s->dproj, s->vpasses != 0 || s->post != 0);
 }
 
+// Gives the tables of the tile launches back.
+void FreeTiles(xf_scene* s) {
+    (void)hipStreamSynchronize(s->ctx->stream);
+    DropGraph(s);
+    auto drop = [](auto*& p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    };
+    drop(s->X2);
+    drop(s->tile_meta);
+    drop(s->tile_rec);
+    drop(s->tile_node);
+    drop(s->tile_pos);
+    drop(s->tile_loc);
+    for (float4*& e : s->tile_tg) drop(e);
+    drop(s->tile_taux);
+    s->device_bytes -= s->tile_bytes;
+    s->tile_bytes = 0;
+    s->ntile = 0;
+    s->tile_nent = 0;
+    s->tile_spans.clear();
+}
+
+// Device memory of the tile launches, which a scene can do without: false
+// where there is none left.
+template <typename T>
+bool TileAlloc(xf_scene* s, T** p, size_t count) {
+    if (hipMalloc((void**)p, sizeof(T) * count) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
+    }
+    s->tile_bytes += sizeof(T) * count;
+    s->device_bytes += sizeof(T) * count;
+    return true;
+}
+
+// Element data and material of the tile entries, from the schedule's.
+int FillTiles(xf_scene* s) {
+    xf_ctx* ctx = s->ctx;
+    if (s->taux && !s->tile_taux && !TileAlloc(s, &s->tile_taux, s->tile_nent)) {
+        FreeTiles(s);
+        return XF_OK;
+    }
+    XF_HIP(ctx, xf_launch_tile_fill(ctx->stream, s->tile_nent, s->tile_pos, s->tg, s->taux, s->tile_tg, s->tile_taux));
+    return XF_OK;
+}
+
 int UploadMaterial(xf_scene* s) {
     xf_ctx* ctx = s->ctx;
     bool had_aux = s->aux;
@@ -586,12 +640,8 @@ int UploadMaterial(xf_scene* s) {
         XF_HIP(ctx, hipMemcpyAsync(s->taux, s->h_taux.data(), sizeof(float4) * s->T, hipMemcpyHostToDevice,
                                    ctx->stream));
     if (s->ntile) {
-        if (need_taux && !s->tile_taux) {
-            int rc = DevAlloc(ctx, &s->tile_taux, s->tile_nent, &s->device_bytes);
-            if (rc) return rc;
-        }
-        XF_HIP(ctx, xf_launch_tile_fill(ctx->stream, s->tile_nent, s->tile_pos, s->tg, need_taux ? s->taux : nullptr,
-                                        s->tile_tg, s->tile_taux));
+        int rc = FillTiles(s);
+        if (rc) return rc;
     }
     XF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s->material_dirty = false;
@@ -1597,15 +1647,23 @@ void BuildBodyTables(xf_scene* s, BodyTables* bt) {
     s->body_threads = std::min(512u, std::max(256u, (cmax + 63) / 64 * 64));
 }
 
-// Tables of the tile launches where a sweep of them is estimated shorter than
-// whole calls and than a launch per colour.
-int BuildTiles(xf_scene* s, const std::vector<uint4>& tidx) {
+// The plan of the tile launches, by the first step call that could use them (a
+// scene that never can keeps neither the time nor the memory): their tables
+// where a sweep of them is estimated shorter than whole calls and than a
+// launch per colour. Device memory: 32 bytes a node, 76 (with material slots
+// 92) each time that a tile projects a tet: 3.9 times on a 64x16x16 beam of 24
+// colours (29 MB), 3.0 on 96x24x24 (76 MB), 2.2 on 128x36x36 (170 MB). A scene
+// that finds no memory for them stays with the other routes.
+int PlanSweeps(xf_scene* s, int energy) {
     xf_ctx* ctx = s->ctx;
-    if (s->opts.launch_mode != XF_LAUNCH_PER_COLOUR || s->ncol < 2 || s->bodies.size() > (size_t)s->n_cu ||
+    if (s->tiles_tried || !MayTile(s, energy)) return XF_OK;
+    s->tiles_tried = true;
+    if (s->ncol < 2 || s->bodies.size() > (size_t)s->n_cu ||
         (uint64_t)s->N > (uint64_t)s->n_cu * 2 * kTileThreads)
         return XF_OK;
     // two launches with all phases on quads are the least a plan can come to
     if (s->body_threads && s->body_us < 9.0 + 0.85 * s->ncol) return XF_OK;
+    std::vector<uint4> tidx(s->T);
     XfTileMesh m;
     m.n_nodes = s->N;
     m.n_tets = s->T;
@@ -1615,6 +1673,11 @@ int BuildTiles(xf_scene* s, const std::vector<uint4>& tidx) {
     for (const Body& b : s->bodies) {
         m.body_begin.push_back(b.node_base);
         m.xyz.push_back(b.xyz.data());
+        for (uint32_t t = 0; t < b.t; t++) {
+            const uint32_t* is = &b.tets[4 * (size_t)t];
+            tidx[b.sched_pos[t]] =
+                make_uint4(b.node_base + is[0], b.node_base + is[1], b.node_base + is[2], b.node_base + is[3]);
+        }
     }
     m.body_begin.push_back(s->N);
     m.n_cu = (uint32_t)s->n_cu;
@@ -1623,16 +1686,14 @@ int BuildTiles(xf_scene* s, const std::vector<uint4>& tidx) {
     if (plan.spans.size() < 2 || plan.n_ent == 0) return XF_OK;
     const double other = s->body_threads ? s->body_us : ColourLaunchesUs(s);
     if (plan.us >= other) return XF_OK;
-    int rc;
-    if ((rc = DevAlloc(ctx, &s->X2, s->N, &s->device_bytes)) ||
-        (rc = DevAlloc(ctx, &s->tile_meta, plan.meta.size(), &s->device_bytes)) ||
-        (rc = DevAlloc(ctx, &s->tile_rec, plan.rec.size(), &s->device_bytes)) ||
-        (rc = DevAlloc(ctx, &s->tile_node, plan.n_node, &s->device_bytes)) ||
-        (rc = DevAlloc(ctx, &s->tile_pos, plan.n_ent, &s->device_bytes)) ||
-        (rc = DevAlloc(ctx, &s->tile_loc, plan.n_ent, &s->device_bytes)))
-        return rc;
-    for (float4*& e : s->tile_tg)
-        if ((rc = DevAlloc(ctx, &e, plan.n_ent, &s->device_bytes))) return rc;
+    bool got = TileAlloc(s, &s->X2, s->N) && TileAlloc(s, &s->tile_meta, plan.meta.size()) &&
+               TileAlloc(s, &s->tile_rec, plan.rec.size()) && TileAlloc(s, &s->tile_node, plan.n_node) &&
+               TileAlloc(s, &s->tile_pos, plan.n_ent) && TileAlloc(s, &s->tile_loc, plan.n_ent);
+    for (float4*& e : s->tile_tg) got = got && TileAlloc(s, &e, plan.n_ent);
+    if (!got) {
+        FreeTiles(s);
+        return XF_OK;
+    }
     hipStream_t st = ctx->stream;
     XF_HIP(ctx, hipMemcpyAsync(s->tile_meta, plan.meta.data(), sizeof(uint4) * plan.meta.size(),
                                hipMemcpyHostToDevice, st));
@@ -1646,9 +1707,11 @@ int BuildTiles(xf_scene* s, const std::vector<uint4>& tidx) {
         XF_HIP(ctx, hipMemcpyAsync(s->tile_loc + sp.ent0, sp.loc.get(), sizeof(uint2) * sp.n_ent,
                                    hipMemcpyHostToDevice, st));
     }
-    XF_HIP(ctx, hipStreamSynchronize(st));
-    s->ntile = plan.ntile;
     s->tile_nent = plan.n_ent;
+    int rc = FillTiles(s);
+    XF_HIP(ctx, hipStreamSynchronize(st));
+    if (rc || s->tile_nent == 0) return rc;
+    s->ntile = plan.ntile;
     for (size_t k = plan.spans.size(); k-- > 0;) {  // in sweep order
         const XfTileSpan& sp = plan.spans[k];
         s->tile_spans.push_back({sp.nph, sp.nmax, std::max(sp.pmax, plan.own_max), sp.meta, sp.rec});
@@ -2114,7 +2177,6 @@ XF_API int xf_scene_finalize(xf_scene* s, const xf_scene_opts* opts) {
         XF_HIP(ctx, hipMemcpyAsync(s->body_loc, body.loc.data(), sizeof(uint2) * body.loc.size(),
                                    hipMemcpyHostToDevice, st));
     }
-    if ((rc = BuildTiles(s, h_tidx))) return rc;
     uint32_t uzero = 0;
     static const uint32_t kClockZero[kClockWords] = {0u, 0u};  // time 0.0f, tick 0
     XF_HIP(ctx, hipMemcpyAsync(s->clock, kClockZero, sizeof(kClockZero), hipMemcpyHostToDevice, st));
@@ -2212,6 +2274,7 @@ XF_API int xf_scene_step(xf_scene* s, uint32_t substeps, float dt) {
     int energy;
     bool sim;
     int rc = Prepare(s, dt, &energy, &sim);
+    if (!rc) rc = PlanSweeps(s, energy);
     if (rc) return rc;
     // one launch per call needs no graph
     if (!s->opts.use_graph || s->opts.launch_mode == XF_LAUNCH_PERSISTENT || WholeCalls(s, energy)) {
@@ -2430,6 +2493,7 @@ XF_API int xf_scene_profile(xf_scene* s, uint32_t substeps, float dt, float* ms_
     int energy;
     bool sim;
     int rc = Prepare(s, dt, &energy, &sim);
+    if (!rc) rc = PlanSweeps(s, energy);
     if (rc) return rc;
     LaunchTimer timer;
     rc = Enqueue(s, substeps, dt, energy, sim, &timer);
@@ -2595,6 +2659,10 @@ XF_API int xf_scene_autotune(xf_scene* s, uint32_t substeps, float dt, uint32_t 
     if (best_c.mode == XF_LAUNCH_PERSISTENT) s->opts.persistent_blocks = best_c.size;
     else s->opts.block_size = best_c.size;
     DropGraph(s);
+    if (best_c.mode != XF_LAUNCH_PER_COLOUR && s->tiles_tried) {  // planned for the trials
+        FreeTiles(s);
+        s->tiles_tried = false;
+    }
     if (!rc && s->opts.sweep_blocks) {
         rc = repack(best_c.cap);
         if (!rc && best_c.cap != cap_keep) s->opts.block_lanes = best_c.cap;
