@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <new>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1647,17 +1648,8 @@ void BuildBodyTables(xf_scene* s, BodyTables* bt) {
     s->body_threads = std::min(512u, std::max(256u, (cmax + 63) / 64 * 64));
 }
 
-// The plan of the tile launches, by the first step call that could use them (a
-// scene that never can keeps neither the time nor the memory): their tables
-// where a sweep of them is estimated shorter than whole calls and than a
-// launch per colour. Device memory: 32 bytes a node, 76 (with material slots
-// 92) each time that a tile projects a tet: 3.9 times on a 64x16x16 beam of 24
-// colours (29 MB), 3.0 on 96x24x24 (76 MB), 2.2 on 128x36x36 (170 MB). A scene
-// that finds no memory for them stays with the other routes.
-int PlanSweeps(xf_scene* s, int energy) {
+int MakeTiles(xf_scene* s) {
     xf_ctx* ctx = s->ctx;
-    if (s->tiles_tried || !MayTile(s, energy)) return XF_OK;
-    s->tiles_tried = true;
     if (s->ncol < 2 || s->bodies.size() > (size_t)s->n_cu ||
         (uint64_t)s->N > (uint64_t)s->n_cu * 2 * kTileThreads)
         return XF_OK;
@@ -1717,6 +1709,24 @@ int PlanSweeps(xf_scene* s, int energy) {
         s->tile_spans.push_back({sp.nph, sp.nmax, std::max(sp.pmax, plan.own_max), sp.meta, sp.rec});
     }
     return XF_OK;
+}
+
+// The plan of the tile launches, by the first step call that could use them (a
+// scene that never can keeps neither the time nor the memory): their tables
+// where a sweep of them is estimated shorter than whole calls and than a
+// launch per colour. Device memory: 32 bytes a node, 76 (with material slots
+// 92) each time that a tile projects a tet: 3.9 times on a 64x16x16 beam of 24
+// colours (29 MB), 3.0 on 96x24x24 (76 MB), 2.2 on 128x36x36 (170 MB). A scene
+// that finds no memory for them stays with the other routes.
+int PlanSweeps(xf_scene* s, int energy) {
+    if (s->tiles_tried || !MayTile(s, energy)) return XF_OK;
+    s->tiles_tried = true;
+    try {
+        return MakeTiles(s);
+    } catch (const std::bad_alloc&) {  // no host memory for it either
+        FreeTiles(s);
+        return XF_OK;
+    }
 }
 
 int CheckSettings(xf_ctx* ctx, const xf_settings* st) {

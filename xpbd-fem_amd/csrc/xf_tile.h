@@ -50,7 +50,8 @@ struct XfTileMesh {
     uint32_t n_cu = 0, lds_limit = 0;
 };
 
-// Empty (no spans) when a tile of one colour is larger than a workgroup takes.
+// Empty (no spans) when a tile of one colour is larger than a workgroup takes,
+// or when memory runs out.
 XfTilePlan PlanTiles(const XfTileMesh& mesh);
 
 // Limits of a tile launch.

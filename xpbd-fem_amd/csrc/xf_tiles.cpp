@@ -143,7 +143,8 @@ uint32_t Workers(uint32_t n_tets) {
 }
 
 // f(k) for k < n on a thread each (on this one where there is one, or no
-// thread to be had); the least of the results, 0 if one ran out of memory.
+// thread or memory for one to be had); the least of the results, 0 if one ran
+// out of memory.
 template <class F>
 uint32_t Share(uint32_t n, F f) {
     std::vector<uint32_t> out(n, 0u);
@@ -160,6 +161,7 @@ uint32_t Share(uint32_t n, F f) {
     try {
         for (; started < n; started++) threads.emplace_back(run, started);
     } catch (const std::system_error&) {
+    } catch (const std::bad_alloc&) {  // the threads that run are still joined
     }
     run(0);
     for (uint32_t k = started; k < n; k++) run(k);
@@ -167,9 +169,7 @@ uint32_t Share(uint32_t n, F f) {
     return *std::min_element(out.begin(), out.end());
 }
 
-}  // namespace
-
-XfTilePlan PlanTiles(const XfTileMesh& m) {
+XfTilePlan Plan(const XfTileMesh& m) {
     XfTilePlan plan;
     const uint32_t B = (uint32_t)m.xyz.size();
     // tiles per body: one to a compute unit, each next one to the body whose
@@ -289,4 +289,14 @@ XfTilePlan PlanTiles(const XfTileMesh& m) {
         end -= best;
     }
     return plan;
+}
+
+}  // namespace
+
+XfTilePlan PlanTiles(const XfTileMesh& m) {
+    try {
+        return Plan(m);
+    } catch (const std::bad_alloc&) {
+        return XfTilePlan();
+    }
 }
