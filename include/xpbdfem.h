@@ -395,11 +395,12 @@ XF_API int xf_scene_time_steps(xf_scene* scene, uint32_t calls, uint32_t substep
  * launch shape -- per-colour launches with workgroup sizes 64, 128, 256 and
  * the persistent launch with 64, 128, 256 and 512 blocks (where co-resident),
  * and, when the scene has sweep_blocks, sweep-block launches with
- * workgroup sizes 64, 128, 256, 1 or 4 lanes per tet (4 where the
- * projection allows it) and slot caps (block_lanes) 32, 64, 128 and 256,
- * the slots repacked for each cap -- and keeps the fastest in the scene
- * options (block_lanes is set when the chosen cap differs from the one in
- * use). The node state and clock are restored afterwards, so tuning does
+ * one lane per tet, or four (where the projection allows it) with workgroup
+ * sizes 64, 128, 256, and slot caps (block_lanes) 32, 64, 128 and 256, the
+ * slots repacked for each cap -- and keeps the fastest in the scene options
+ * (block_lanes is set when the chosen cap differs from the one in use;
+ * block_size stays the caller's where the launches choose their own: whole
+ * calls, tiles, blocks with one lane per tet). The node state and clock are restored afterwards, so tuning does
  * not advance the simulation. chosen / best_ms (ms per call) nullable.
  * No reference counterpart (the reference is single-threaded). */
 XF_API int xf_scene_autotune(xf_scene* scene, uint32_t substeps, float dt, uint32_t reps, xf_scene_opts* chosen,

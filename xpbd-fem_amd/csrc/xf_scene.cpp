@@ -2592,18 +2592,30 @@ XF_API int xf_scene_autotune(xf_scene* s, uint32_t substeps, float dt, uint32_t 
     };
     // Candidates: launch mode and workgroup size; for sweep blocks also
     // lanes per tet and the slot cap (block_lanes: the slots are repacked
-    // for each cap, caps outermost).
+    // for each cap, caps outermost). Where the launches take their own
+    // workgroup size (whole calls, tiles, blocks with one lane per tet) there is
+    // one candidate, with the caller's. Blocks with automatic lanes are always
+    // one of the others: one lane per tet, or four on 256 threads.
     struct Cand {
         uint32_t mode, size, lanes, cap;
     };
+    const xf_scene_opts keep = s->opts;
+    s->opts.launch_mode = XF_LAUNCH_PER_COLOUR;
+    rc = PlanSweeps(s, energy);
+    const bool sized = !WholeCalls(s, energy) && !TileSweeps(s, energy);
+    s->opts.launch_mode = keep.launch_mode;
     std::vector<Cand> candidates;
-    for (uint32_t size : {64u, 128u, 256u}) candidates.push_back({XF_LAUNCH_PER_COLOUR, size, 1, 0});
+    auto add = [&](uint32_t mode, uint32_t lanes, uint32_t cap, bool sizes) {
+        if (!sizes) candidates.push_back({mode, keep.block_size, lanes, cap});
+        else for (uint32_t size : {64u, 128u, 256u}) candidates.push_back({mode, size, lanes, cap});
+    };
+    add(XF_LAUNCH_PER_COLOUR, 1, 0, sized);
     for (uint32_t size : {64u, 128u, 256u, 512u}) candidates.push_back({XF_LAUNCH_PERSISTENT, size, 1, 0});
     if (s->opts.sweep_blocks && energy != kRingMode)
-        for (uint32_t cap : {32u, 64u, 128u, 256u})
-            for (uint32_t lanes : {1u, 4u})
-                for (uint32_t size : {64u, 128u, 256u}) candidates.push_back({XF_LAUNCH_BLOCKS, size, lanes, cap});
-    xf_scene_opts keep = s->opts;
+        for (uint32_t cap : {32u, 64u, 128u, 256u}) {
+            add(XF_LAUNCH_BLOCKS, 1, cap, false);
+            add(XF_LAUNCH_BLOCKS, 4, cap, true);
+        }
     const uint32_t cap_keep = s->blk_lanes;
     Cand best_c = {keep.launch_mode, keep.launch_mode == XF_LAUNCH_PERSISTENT ? keep.persistent_blocks : keep.block_size,
                    keep.tet_lanes, cap_keep};
