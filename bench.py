@@ -58,8 +58,32 @@ BYTES_FUSED_NODE = 32 + 32
 SCHEDULES = {"blocks": dict(sweep_blocks=True, launch_mode=xf.LAUNCH_BLOCKS), "slabs": dict(xcd_slabs=True),
              "plain": {}}
 MODE_NAMES = {xf.LAUNCH_PER_COLOUR: "per-colour", xf.LAUNCH_PERSISTENT: "persistent", xf.LAUNCH_BLOCKS: "blocks"}
-KERNELS = {xf.LAUNCH_PER_COLOUR: "xf_project_colour", xf.LAUNCH_PERSISTENT: "xf_frame_persistent",
-           xf.LAUNCH_BLOCKS: "xf_project_blocks"}
+ROUTE_KERNELS = {xf.ROUTE_COLOURS: "xf_project_colour", xf.ROUTE_TILES: "xf_tile_span",
+                 xf.ROUTE_BODIES: "xf_body_steps", xf.ROUTE_PERSISTENT: "xf_frame_persistent",
+                 xf.ROUTE_BLOCKS: "xf_project_blocks", xf.ROUTE_RINGS: "xf_ring_colour"}
+
+
+def launched_size(sc, mode, size):
+    """Threads of a workgroup of the scene's launches (their own choice in some
+    routes, whatever block_size is), or the blocks of the persistent grid."""
+    return size if mode == xf.LAUNCH_PERSISTENT else sc.route()[1]
+
+
+def recorded_traffic(rec, info, route, threads, schedule):
+    """HBM bytes per projection launch that the counter passes recorded
+    (profiles/traffic_beam96x24x24.json) for the launch shape that ran, or
+    None: block launches match by blocks, slots, cap, lanes per tet and
+    threads, launches per colour by the tets of a colour."""
+    if route == xf.ROUTE_BLOCKS:
+        for b in rec.get("blocks_shapes", []):
+            if (b["n_blocks"], b["n_block_slots"], b["block_lanes"], b["tet_lanes"], b["block_size"]) == \
+                    (info["n_blocks"], info["n_block_slots"], info["block_lanes"], info["tet_lanes"], threads):
+                return float(b["traffic_bytes_per_dispatch"])
+    elif route == xf.ROUTE_COLOURS and schedule != "blocks" and \
+            rec.get("tets_per_dispatch") == info["n_tets"] // max(info["n_colours"], 1):
+        return float(rec["traffic_bytes_per_dispatch"] if schedule == "slabs" else
+                     rec["plain_schedule"]["traffic_bytes_per_dispatch"])
+    return None
 
 
 def fp32_valu(tet_projections, ms):
@@ -199,6 +223,7 @@ def batched_leg(ctx, frames=3, schedule="blocks"):
     el_b = time.perf_counter() - t0
     finite = sc.count_nonfinite() == 0
     info = sc.info()
+    threads = launched_size(sc, mode, size)
     ncol = info["n_colours"]
     sc.close()
     singles = [workloads.make_batch_scene(ctx, b, bodies=[i]) for i in range(len(b["bodies"]))]
@@ -220,7 +245,7 @@ def batched_leg(ctx, frames=3, schedule="blocks"):
     out = {"workload": f"{b['name']}: {len(b['bodies'])} bodies, {T} tets, {S} substeps/frame, {ncol} colours",
            "batched_tet_substeps_per_s": batched, "plain_loop_tet_substeps_per_s": plain,
            "batched_over_plain": batched / plain, "frames": frames,
-           "launch": {"mode": MODE_NAMES[mode], "size": size, "schedule": schedule,
+           "launch": {"mode": MODE_NAMES[mode], "size": threads, "schedule": schedule,
                       "block_lanes": info["block_lanes"], "tet_lanes": info["tet_lanes"]},
            "finite": finite}
     out["check"] = batch_check(ctx, b, schedule, mode, size, block_lanes=info["block_lanes"],
@@ -426,16 +451,17 @@ def large_leg(ctx, frames=2, cells=(288, 72, 72), schedule="blocks"):
     ms = timed_frames(sc, S, dt, frames)
     finite = sc.count_nonfinite() == 0
     ms_proj, _, n_launch = sc.profile(S, dt)
+    threads, kernel = launched_size(sc, mode, size), ROUTE_KERNELS[sc.route()[0]]
     sc.close()
     bytes_proj = projection_bytes(info, mode, S)
     achieved = bytes_proj / (ms_proj * 1e-3) / 1e9 if mode != xf.LAUNCH_PERSISTENT else None
     out = {"workload": f"{wl['name']}: {T} tets, {info['n_nodes']} nodes, {info['n_colours']} colours, "
                        f"{info['n_blocks']} sweep blocks, {S} substeps/frame",
            "tet_substeps_per_s": T * S / (ms * 1e-3), "ms_per_frame": ms, "finite": finite,
-           "launch": {"mode": MODE_NAMES[mode], "size": size, "schedule": schedule,
+           "launch": {"mode": MODE_NAMES[mode], "size": threads, "schedule": schedule,
                       "block_lanes": info["block_lanes"], "tet_lanes": info["tet_lanes"],
                       "node_phase": "in the last projection launch" if info["fused_finish"] else "own launch"},
-           "roofline": {"bound": "hbm", "kernel": KERNELS[mode], "achieved": achieved, "peak": HBM_PEAK_GBS,
+           "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS if achieved else None,
                         "launches": n_launch, "avg_launch_us": 1e3 * ms_proj / max(n_launch, 1),
                         "bytes_per_launch": bytes_proj / max(n_launch, 1),
@@ -636,6 +662,7 @@ def beam_profile(schedule="blocks", block=64, tet_lanes=1, frames=1, graph=False
     wl = workloads.beam_yeoh_96x24x24()
     sc = workloads.make_scene(ctx, wl, block_size=block, tet_lanes=tet_lanes, use_graph=graph, contract=contract,
                               **SCHEDULES[schedule])
+    sc.set_colour_launches(schedule != "blocks")
     for _ in range(frames):
         sc.step(wl["substeps"], float(wl["dt"]))
     sc.sync()
@@ -734,6 +761,9 @@ def main():
     ctx = xf.Context(0)
     opts = SCHEDULES[args.schedule]
     sc = workloads.make_scene(ctx, wl, use_graph=True, **opts)
+    # the slabs and plain schedules are one launch per colour, whose bytes the
+    # roofline counts
+    sc.set_colour_launches(args.schedule != "blocks")
     info = sc.info()
     T, N, S = info["n_tets"], info["n_nodes"], wl["substeps"]
     dt = float(wl["dt"])
@@ -779,20 +809,12 @@ def main():
     # HBM traffic per projection launch: calibrated FETCH_SIZE + WRITE_SIZE of the
     # rocprofv3 --pmc passes recorded for this workload and schedule (profiles/),
     # when the launch shape matches.
+    threads = launched_size(sc, mode, size)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "traffic_beam96x24x24.json")
     if os.path.exists(tpath):
         with open(tpath) as f:
-            rec = json.load(f)
-        shapes = rec.get("blocks_shapes", [])
-        match = [b for b in shapes if b.get("n_blocks") == info["n_blocks"] and b.get("block_size") == size and
-                 b.get("block_lanes") == info["block_lanes"]]
-        if mode == xf.LAUNCH_BLOCKS and match and info["tet_lanes"] == 1:
-            traffic = float(match[0]["traffic_bytes_per_dispatch"])
-        elif mode == xf.LAUNCH_PER_COLOUR and args.schedule != "blocks" and \
-                rec.get("tets_per_dispatch") == T // max(info["n_colours"], 1):
-            traffic = float(rec["traffic_bytes_per_dispatch"] if args.schedule == "slabs" else
-                            rec["plain_schedule"]["traffic_bytes_per_dispatch"])
+            traffic = recorded_traffic(json.load(f), info, sc.route()[0], threads, args.schedule)
 
     out = {
         "metric": METRIC,
@@ -809,12 +831,12 @@ def main():
         "data": "synthetic",
         "config": {"workload": f"{wl['name']}: {T} tets, {N} nodes, {S} substeps/frame, {info['n_colours']} "
                                f"colours, {info['n_blocks']} sweep blocks, ground + sphere", "step": "one frame",
-                   "launch": {"mode": MODE_NAMES[mode], "size": size, "schedule": args.schedule,
+                   "launch": {"mode": MODE_NAMES[mode], "size": threads, "schedule": args.schedule,
                               "tet_lanes": sc.info()["tet_lanes"] if mode == xf.LAUNCH_BLOCKS else 1,
                               "block_lanes": info["block_lanes"],
                               "node_phase": "in the last projection launch" if fused_now else "own launch"}},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": KERNELS[mode],
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": ROUTE_KERNELS[sc.route()[0]],
                      "launches": n_launch, "avg_launch_us": 1e3 * ms_proj / max(n_launch, 1),
                      "bytes_per_launch": bytes_proj / max(n_launch, 1),
                      "frac_196B_model": bytes_model / (ms_proj * 1e-3) / 1e9 / HBM_PEAK_GBS,
@@ -827,8 +849,11 @@ def main():
         pc = workloads.make_scene(ctx, wl, **SCHEDULES["slabs"])
         pc.autotune(S, dt, reps=2)
         ms_pc = timed_frames(pc, S, dt, 10)
+        out["per_colour_slabs"] = {"ms_per_frame": ms_pc, "tet_substeps_per_s": T * S / (ms_pc * 1e-3),
+                                   "kernel": ROUTE_KERNELS[pc.route()[0]]}
+        pc.set_colour_launches()
+        out["per_colour_slabs"]["ms_per_frame_launch_per_colour"] = timed_frames(pc, S, dt, 10)
         pc.close()
-        out["per_colour_slabs"] = {"ms_per_frame": ms_pc, "tet_substeps_per_s": T * S / (ms_pc * 1e-3)}
         if mode == xf.LAUNCH_BLOCKS:
             try:
                 out["contracted"] = contracted_leg(
