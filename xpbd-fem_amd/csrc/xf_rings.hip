@@ -94,8 +94,9 @@ __device__ __forceinline__ uint32_t team_value(uint32_t v) {
 }
 
 // a[0] + a[6] + a[12] + ... (n terms), in order from 0. Eight loads are in
-// flight at a time, those past the last term in a remainder (LDS of the
-// workgroup or past its end, where reads give 0) not used; adding 0 in their
+// flight at a time, those past the last term in a remainder not used (they lie
+// in the team's own LDS: up to 32 floats past its entries, where the nodes'
+// part follows with 14 floats a node, four nodes and more); adding 0 in their
 // place is exact, as the sum is never -0.
 __device__ __forceinline__ float ordered_sum(const float* a, uint32_t n) {
     float s = 0.0f;

@@ -1294,13 +1294,18 @@ std::vector<uint32_t> BinOrder(const BlockSizes& z, uint32_t cap, uint32_t slot_
 //
 // Cap: 64, the tets of one wave or of a quad workgroup, until a compute unit's
 // LDS is full of such slots, then 128, whose larger blocks load a shared node
-// less often. Per 30-substep frame of a beam at 64 and 128: 128x36x36 2.15 and
-// 2.45 ms, 192x48x48 3.21 and 3.34, 216x54x54 (10.97 slots per compute unit
-// and launch) 4.16 and 4.27, 240x60x60 (15.0) 5.69 and 5.34, 288x72x72 10.4 and
-// 9.2; 20-substep frame of 400 mixed boxes (11.5) 6.26 and 6.08.
+// less often. ms per 30-substep frame of a beam at 64 and 128: 112x30x30 1.65
+// and 1.73, 160x40x40 2.68 and 2.78, 192x48x48 3.23 and 3.38, 216x54x54 (10.97
+// slots per compute unit and launch) 4.23 and 4.30, 240x60x60 (15.0) 5.67 and
+// 5.41, 288x72x72 10.5 and 9.17; per 20-substep frame of 64, 128 and 400 mixed
+// boxes (1.9, 3.8 and 11.5 slots) 1.83 and 1.89, 2.30 and 2.57, 5.85 and 5.43.
+// The line by slots misses a few: 128 is ahead on 128x36x36 (2.12 and 1.93),
+// 144x40x40 (2.37 and 2.15) and 256 boxes (3.69 and 3.32), where it leaves 1.5,
+// 2.0 and 3.8 workgroups per compute unit, but not on the 128 boxes with 1.9.
 //
 // Layout: body, then block number, or BinOrder for the cap where a compute
-// unit then sweeps fewer slots (192x48x48 beam: 3.54 ms as runs, 3.21 so). On the 96x24x24 beam (blocks of 1 to 24 tets a phase) 264 slots
+// unit then sweeps fewer slots (192x48x48 beam: 3.54 ms as runs, 3.21 so). On
+// the 96x24x24 beam (blocks of 1 to 24 tets a phase) 264 slots
 // a launch become 226 on 256 compute units; the eight compute units that swept
 // two slots took 11 us where the others took 8. Blocks of one launch colour
 // share no node, so their order in memory does not enter the results; the
@@ -2961,7 +2966,11 @@ int ReverseLaunches(xf_scene* s, uint32_t substeps, float dt, int energy, uint32
         const uint32_t vb = s->colour_begin[v], vc = rev_tape ? s->colour_begin[v + 1] - vb : 0;
         // four lanes per tet of the reverse while its lanes fill no more than
         // the device's SIMDs (colours of 6,133 tets, with the record of as many:
-        // 4.6 us against 5.56 with one lane)
+        // 4.6 us against 5.56 with one lane). The line holds for both precisions:
+        // adjoint of 12 substeps, one lane and four, FP32 and FP64 elements, 480
+        // tets a colour (FP64; FP32 goes by windows) 3.01 and 2.78 ms, 1,152 2.47
+        // and 2.26, 3.15 and 2.93, 4,000 3.12 and 2.95, 3.81 and 3.61, 9,464 4.60
+        // and 4.33, 5.36 and 5.15, 12,544 5.37 and 5.35, 6.09 and 6.06
         const bool quad = vc <= 64u * (uint32_t)s->n_cu;
         if (vc) {
             XF_HIP(ctx, xf_launch_adj_pair(st, s->aux, fp64, quad, rb, rc, s->X, rec_tape, vb, vc, rev_tape, W, b.Xb,

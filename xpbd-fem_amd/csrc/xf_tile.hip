@@ -6,10 +6,12 @@
 // of the chip idle). Here one launch pays them for a span of colours, whose
 // chains follow each other out of LDS; the halo tets that neighbours project
 // too run on lanes that would be idle. Per substep, launches per colour
-// against tiles, one to a compute unit: 24x12x12 beam of 24 colours 84 us and
-// 34.9 (2 spans of 12 colours, 17 own nodes a tile and 950 in LDS), 64x16x16
-// 86 and 44 (3 spans of 8), 128x36x36 184 and 107, the same with 31 greedy
-// colours 261 and 137; 64 mixed boxes 203 and 93. The element data of a tile's
+// against tiles, one to a compute unit: 24x12x12 beam of 24 colours 85 us and
+// 35 (spans of 4, 9 and 11 colours, 17 own nodes a tile and up to 1,033 in LDS,
+// a tet projected 14.7 times), 64x16x16 90 and 44 (4 spans of 6, 74 own nodes
+// and up to 712, 3.9 times), 96x24x24 125 and 66 (4, 6, 7 and 7 colours, 3.0
+// times), 128x36x36 258 and 107, the same with 31 greedy colours 255 and 137;
+// 64 mixed boxes 206 and 93. The element data of a tile's
 // entries is stored in entry order: read from the schedule by position, 64x16x16
 // took 50.7 us (a 16-byte quarter of a line per tet and array).
 #include <hip/hip_runtime.h>

@@ -18,8 +18,10 @@ constexpr uint32_t kMaxPhase = 4 * kTileThreads;
 // Estimated times in microseconds (measured): a launch up to its first phase
 // and after its last, and a phase of cnt tets (up to 64 on quads; a wave on
 // each SIMD; two; further tets in turn). A sweep's sum and what it took:
-// 12x7x7 beam, 24 colours 35.4 and 32.3, 64x16x16 43.7 and 44.1, 96x24x24 54.5
-// and 65.6, greedy colours 74.8 and 87.1.
+// 12x7x7 beam, 24 colours 35.5 and 32.2, 24x12x12 41.1 and 34.8, 64x16x16 47.3
+// and 43.8, 96x24x24 58.4 and 65.5 (31 greedy colours 76.1 and 86.8), 128x36x36
+// 86.1 and 107 (99.6 and 137): a fifth too much to a quarter too little,
+// where the launches per colour that it is compared with take twice as long.
 double LaunchUs(size_t nodes) { return 4.6 + 0.5 * (double)nodes / 1024.0; }
 double PhaseUs(uint32_t cnt) {
     if (cnt == 0) return 0.1;
